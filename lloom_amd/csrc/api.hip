@@ -76,8 +76,10 @@ static int ensure_ws(lloom_hip_ctx* ctx, size_t bytes, hipStream_t s, void** out
         size_t want = bytes > 2 * ctx->ws_bytes ? bytes : 2 * ctx->ws_bytes;
         want = (want + 0xFFFFF) & ~(size_t)0xFFFFF;
         void* fresh = nullptr;
-        if (hipMalloc(&fresh, want) != hipSuccess)
+        if (hipMalloc(&fresh, want) != hipSuccess) {
+            (void)hipGetLastError();
             return fail(LLOOM_HIP_ENOMEM, "workspace allocation of %zu bytes failed", want);
+        }
         if (ctx->ws) ctx->retired.push_back(ctx->ws);
         ctx->ws = fresh;
         ctx->ws_bytes = want;
@@ -426,10 +428,17 @@ static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const 
     hipStream_t s = pick_stream(ctx, stream);
     std::lock_guard<std::mutex> lock(ctx->mu);
     void* ws = nullptr;
-    int rc = ensure_ws(ctx, moe_workspace_bytes(n_experts, batch * topk, n, k, mode), s, &ws);
+    // the grouped GEMM wants a copy of the activations; where the workspace
+    // cannot grow to hold it (a capture, or no memory), the kernels that need
+    // the routing ints alone serve the call
+    const int64_t rows = in_dim1 == 1 ? batch : batch * topk;
+    int rc = LLOOM_HIP_ENOMEM;
+    if (moe_gemm_fits(ggml_type, n_experts, batch * topk, rows, n, k))
+        rc = ensure_ws(ctx, moe_gemm_workspace_bytes(n_experts, batch * topk, rows, k), s, &ws);
+    if (rc) rc = ensure_ws(ctx, moe_workspace_bytes(n_experts, batch * topk, n, k, mode), s, &ws);
     if (rc) return rc;
     HIP_OK(launch_moe(ggml_type, w_dev, n_experts, n, k, x_dev, batch, in_dim1, ids_dev, topk, y_dev, (int*)ws,
-                      ctx->flags, mode, w2_dev, y2_dev, s));
+                      ctx->ws_bytes, ctx->flags, mode, w2_dev, y2_dev, s));
     if (strict) {
         int flag = 0;
         HIP_OK(hipMemcpyAsync(&flag, ws, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -113,8 +113,25 @@ size_t moe_workspace_ints(int64_t n_experts, int64_t planes);
 constexpr int MOE_ONE = 0, MOE_PAIR = 1, MOE_GLU = 2;
 size_t moe_workspace_bytes(int64_t n_experts, int64_t planes, int64_t n, int64_t k, int mode);
 bool moe_stages(int64_t k);
+// moe_gemm.hip: Q4_K / Q6_K experts with several planes an active expert as a
+// grouped GEMM.  Its workspace holds the converted activations (as many bytes
+// as x); launch_moe takes it where `ws_cap`, the workspace's size, has room
+// and else the kernels that need only the routing ints (moe_workspace_bytes).
+struct MoeGemmCall {
+    int type, mode;
+    const void *w, *w2;
+    int64_t E, n, k, batch, in_dim1, topk;
+    const float* x;
+    const uint32_t* ids;
+    float *y, *y2;
+    void* ws;
+    int* sticky;
+};
+bool moe_gemm_fits(int type, int64_t n_experts, int64_t planes, int64_t rows, int64_t n, int64_t k);
+size_t moe_gemm_workspace_bytes(int64_t n_experts, int64_t planes, int64_t rows, int64_t k);
+hipError_t launch_moe_gemm(const MoeGemmCall& c, hipStream_t s);
 hipError_t launch_moe(int type, const void* w, int64_t n_experts, int64_t n, int64_t k, const float* x,
                       int64_t batch, int64_t in_dim1, const uint32_t* ids, int64_t topk, float* y, int* ws,
-                      int* sticky, int mode, const void* w2, float* y2, hipStream_t s);
+                      size_t ws_cap, int* sticky, int mode, const void* w2, float* y2, hipStream_t s);
 
 }  // namespace lloom

@@ -1,0 +1,747 @@
+// moe_gemm.hip -- routed experts with several planes an expert (prefill):
+// QTensor::indexed_moe_forward* as a grouped GEMM on v_mfma_f32_16x16x32_f16.
+//
+// The contract is the CPU arm's (matmul_t_indexed, lloom-tensor/src/quantized
+// /mod.rs:766-810): f32 activations, exactly dequantized weights, f32 sums.
+// Two launches a call:
+//  1. k_moe_gemm_prep: one workgroup an expert collects the (b, t) planes
+//     routed to it and cuts them into tiles of up to 64; the others convert the
+//     activation rows, each once: x' = x * 2^s (one power of two a row, max
+//     |x'| in [2^13, 2^14): exact) as fp16 hi + lo (x' = hi + lo to about
+//     2^-22 relative), in the order the GEMM's operands want, and (Q4_K) the
+//     32-element sums of x' for the min term.
+//  2. k_moe_gemm: one workgroup per (tile of planes, block of weight rows).
+//     Weights go from HBM to registers and are unpacked there, once per 64
+//     planes, into exact fp16 integers; activations stream through LDS.
+//
+// The arithmetic per superblock of 256:
+//   Q4_K  acc = sum (sc q) x'     (sc q <= 945: exact in fp16)
+//         out += d acc - dmin sum_j m_j X_j   (X_j: the sub-blocks' sums)
+//   Q6_K  acc = sum (sc (q - 32)) x'; |sc (q - 32)| <= 4096 takes 12 bits,
+//         one more than fp16 has, so the weight is an fp16 pair hi + lo too
+//         (exact) and lo meets the activations' hi: a third MFMA (the fourth,
+//         lo lo, is below 2^-22 of the product)
+//         out += d acc
+// Every product is exact in f32 and only the sums round.
+#include "kernels.hpp"
+#include "kq_common.hpp"
+#include "kq_gemm.hpp"
+#include "kq_mfma.hpp"
+
+namespace lloom {
+
+#pragma clang fp contract(off)
+
+typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
+typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
+typedef float gf4 __attribute__((ext_vector_type(4)));
+
+constexpr int MG_WAVES = 4;   // waves of a GEMM workgroup
+constexpr int MG_NT = 2;      // 16-row weight tiles a wave holds
+constexpr int MG_COLS = MG_WAVES * MG_NT * 16;
+
+// ---------------------------------------------------------- the workspace --
+// int hdr[16] ([0] a bad id was seen, [1] tiles), then at 256-byte steps:
+// int4 tiles[] (expert, first place in sorted, planes), int sorted[planes],
+// float inv[rows] (2^-s), fp16 sums[rows][K/256][16] (hi, lo of the eight
+// sums / 32), and x' [rows][K/256][1 KB].
+static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Planes of a tile, at most: 64, and 32 up to 16 planes an expert, where the
+// smaller LDS and register budget keeps three workgroups a CU instead of two
+// ([128, 768, 2048] Q4_K, T tokens top-8, 32 / 64 a tile: T = 64 45 / 62 us,
+// 256 58 / 68, 512 93 / 79, 2000 183 / 161).
+static int mg_tile_rows(int64_t E, int64_t planes) {
+    return planes > 16 * (E < planes ? E : planes) ? 64 : 32;
+}
+
+struct MgLayout {
+    size_t tiles, sorted, inv, sums, xq, total;
+    int64_t max_tiles;
+    int tile_rows;
+};
+static MgLayout mg_layout(int64_t E, int64_t planes, int64_t rows, int64_t k) {
+    MgLayout l;
+    l.tile_rows = mg_tile_rows(E, planes);
+    l.max_tiles = planes / l.tile_rows + (E < planes ? E : planes);
+    l.tiles = 256;
+    l.sorted = l.tiles + up256((size_t)l.max_tiles * 16);
+    l.inv = l.sorted + up256((size_t)planes * 4);
+    l.sums = l.inv + up256((size_t)rows * 4);
+    l.xq = l.sums + up256((size_t)rows * (k / 256) * 32);
+    l.total = l.xq + up256((size_t)rows * k * 4);
+    return l;
+}
+
+size_t moe_gemm_workspace_bytes(int64_t E, int64_t planes, int64_t rows, int64_t k) {
+    return mg_layout(E, planes, rows, k).total;
+}
+
+// Where this route is taken.  It can be: rows of whole superblocks, 32-bit
+// byte offsets into x' and into one expert's weights.  It is the faster one:
+// its time hardly depends on the planes while each active expert has one tile
+// (10 us at k = 256, 25 at 2048, then the weight stream), and k_moe_lds's
+// grows with planes * n * k.  Measured against k_moe_lds, us, [E, n, k]:
+//   Q4_K, planes an expert: [128, 768, 2048] 3 45 / 50, 4 45 / 60; [64, 1280,
+//     2048] 3 43 / 44, 6 44 / 72; [256, 512, 2048] 2 66 / 43, 4 68 / 80
+//   and planes * n: [32, 768, 2048] 98 K 28 / 23, 147 K 28 / 30; [60, 512,
+//     1024] 66 K 16 / 15, 98 K 17 / 16, 131 K 17 / 19
+//   Q6_K [128, 768, 2048] 3 79 / 70, 4 77 / 85; [32, 768, 2048] 98 K 36 / 33,
+//     147 K 36 / 42; [32, 2048, 768] 131 K 26 / 19, 197 K 26 / 27, 262 K 26 / 30;
+//     [8, 768, 2048] 8 planes an expert, 49 K 35 / 30, 12 and 74 K 38 / 44
+// With 8 planes an expert Q4_K comes here at any size (10 / 14 us at [8, 256,
+// 256], 27 / 53 at [8, 768, 2048] against the kernel that served it before).
+bool moe_gemm_fits(int type, int64_t E, int64_t planes, int64_t rows, int64_t n, int64_t k) {
+    if ((type != T_Q4K && type != T_Q6K) || k % 256) return false;
+    if (rows * k * 4 >= ((int64_t)1 << 32) || n * (k / 256) * block_bytes(type) >= ((int64_t)1 << 31)) return false;
+    const int64_t experts = E < planes ? E : planes, size = planes * n;
+    if (type == T_Q4K) return planes >= 8 * experts || (2 * planes >= 7 * experts && size >= 131072);
+    return (planes >= 12 * experts && size >= 65536) || (planes >= 4 * experts && size >= 196608);
+}
+
+// ------------------------------------------------------------------- prep --
+
+// Workgroup e collects the planes of expert e.  It counts every expert's
+// planes, so it knows by itself where its planes and tiles go and the
+// workgroups need nothing of each other (one workgroup for all experts took
+// 17 us at 4096 planes, this 4).  The order inside an expert follows the LDS
+// atomics; every plane's dot is computed on its own, so no result depends on
+// it.
+__device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, int E, int* hdr, int4* tiles,
+                         int* sorted, int* sticky, float* y, float* y2, int n, int tile_rows) {
+    __shared__ int s_cnt[MOE_MAX_EXPERTS];
+    __shared__ int s_first, s_tile, s_tiles, s_at;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < E; i += 1024) s_cnt[i] = 0;
+    if (tid == 0) s_first = s_tile = s_tiles = s_at = 0;
+    __syncthreads();
+    int bad = 0;
+    for (int p0 = tid; p0 < planes; p0 += 8 * 1024) {
+        uint32_t id[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) id[i] = p0 + i * 1024 < planes ? ids[p0 + i * 1024] : 0u;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int p = p0 + i * 1024;
+            if (p >= planes) continue;
+            if (id[i] < (uint32_t)E) {
+                atomicAdd(&s_cnt[id[i]], 1);
+            } else if (e == 0) {
+                // an out-of-range id: zero outputs, and the flags
+                bad = 1;
+                for (int r = 0; r < n; r++) y[(int64_t)p * n + r] = 0.0f;
+                if (y2)
+                    for (int r = 0; r < n; r++) y2[(int64_t)p * n + r] = 0.0f;
+            }
+        }
+    }
+    bad = __syncthreads_or(bad);
+    int first = 0, tile = 0, all = 0;  // planes and tiles of smaller experts, tiles of all
+    for (int i = tid; i < E; i += 1024) {
+        const int c = s_cnt[i], t = (c + tile_rows - 1) / tile_rows;
+        first += i < e ? c : 0;
+        tile += i < e ? t : 0;
+        all += t;
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) {
+        first += __shfl_xor(first, o, 64);
+        tile += __shfl_xor(tile, o, 64);
+        all += __shfl_xor(all, o, 64);
+    }
+    if ((tid & 63) == 0 && all) {
+        atomicAdd(&s_first, first);
+        atomicAdd(&s_tile, tile);
+        atomicAdd(&s_tiles, all);
+    }
+    __syncthreads();
+    if (tid == 0 && e == 0) {
+        hdr[0] = bad;            // this call: read back by a strict call
+        if (bad) sticky[0] = 1;  // until the next lloom_hip_ctx_sync
+        hdr[1] = s_tiles;
+    }
+    const int c = s_cnt[e];
+    if (c == 0) return;  // uniform
+    first = s_first;
+    tile = s_tile;
+    // tiles of one size: the planes over as few tiles as hold them, each a
+    // multiple of 16
+    const int k = (c + tile_rows - 1) / tile_rows, rows = ((c + k - 1) / k + 15) & ~15;
+    for (int i = tid; i < k; i += 1024) tiles[tile + i] = make_int4(e, first + i * rows, min(rows, c - i * rows), 0);
+    for (int p0 = tid; p0 < planes; p0 += 8 * 1024) {
+        uint32_t id[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) id[i] = p0 + i * 1024 < planes ? ids[p0 + i * 1024] : ~0u;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (id[i] == (uint32_t)e) sorted[first + atomicAdd(&s_at, 1)] = p0 + i * 1024;
+    }
+}
+
+// Place of the 8-element group G (elements 8G .. 8G + 7) of a superblock in
+// the GEMM's operand order.  Lane group g of MFMA step s takes:
+//   Q4_K  qs bytes 32g + 8 (s / 2) .., the low (s even) or high nibbles:
+//         elements 64g + 32 (s & 1) + 8 (s / 2) ..
+//   Q6_K  ql bytes 32g + 8 (s / 2) .., likewise: elements
+//         128 (g / 2) + 32 (g & 1) + 64 (s & 1) + 8 (s / 2) ..
+// so a lane's weights of a superblock are 32 contiguous bytes (Q6_K: and 32
+// of qh) and it needs two scales (Q6_K: four).
+template <int TYPE>
+__device__ __forceinline__ void mg_place(int G, int& s, int& g) {
+    if constexpr (TYPE == T_Q4K) {
+        g = G >> 3;
+        s = 2 * (G & 3) + ((G >> 2) & 1);
+    } else {
+        g = 2 * (G >> 4) + ((G >> 2) & 1);
+        s = 2 * (G & 3) + ((G >> 3) & 1);
+    }
+}
+
+// x' of a superblock: [half s / 4][hi, lo][pair (s / 2) & 1][s & 1][g][8]
+// fp16, so a GEMM stage (four steps) takes whole 128-byte lines of a row.
+__device__ __forceinline__ int mg_xq_off(int s, int g) {
+    return (s >> 2) * 512 + ((s >> 1) & 1) * 128 + (s & 1) * 64 + g * 16;
+}
+
+// The first E workgroups route; the others convert 16 rows each, one a wave.
+template <int TYPE>
+__global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict__ X, int rows, int K,
+                                                        uint8_t* __restrict__ xq, _Float16* __restrict__ sums,
+                                                        float* __restrict__ inv, const uint32_t* __restrict__ ids,
+                                                        int planes, int E, int* hdr, int4* tiles, int* sorted,
+                                                        int* sticky, float* y, float* y2, int n, int tile_rows) {
+    if ((int)blockIdx.x < E) {
+        mg_route(ids, planes, blockIdx.x, E, hdr, tiles, sorted, sticky, y, y2, n, tile_rows);
+        return;
+    }
+    const int lane = threadIdx.x & 63, row = (blockIdx.x - E) * 16 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int k8 = K >> 3;
+    const float* x = X + (int64_t)row * K;
+    float mx = 0.0f;
+    for (int i = lane; i < k8; i += 64) {
+        const float4 a = *(const float4*)(x + 8 * i), b = *(const float4*)(x + 8 * i + 4);
+        mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
+                             fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w)))));
+    }
+    mx = wave_max(mx);
+    const bool fin = mx > 0.0f && mx <= 3.4028234e38f;
+    int ex = 0;
+    if (fin) (void)frexpf(mx, &ex);
+    // max |x'| in [2^13, 2^14); 2^s and 2^-s stay normal numbers
+    const int sh = fin ? max(-126, min(126, 14 - ex)) : 0;
+    const float sc = ldexpf(1.0f, sh);
+    if (lane == 0) inv[row] = ldexpf(1.0f, -sh);
+    uint8_t* q = xq + (size_t)row * K * 4;
+    _Float16* sm = sums + (size_t)row * (K >> 8) * 16;
+    for (int i = lane; i < k8; i += 64) {
+        const float4 a = *(const float4*)(x + 8 * i), b = *(const float4*)(x + 8 * i + 4);
+        const float v[8] = {a.x * sc, a.y * sc, a.z * sc, a.w * sc, b.x * sc, b.y * sc, b.z * sc, b.w * sc};
+        gh8 hi, lo;
+        float sum = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            // Q4_K's unpacking gives a dword's bytes in the order 0, 2, 1, 3
+            const int at = TYPE == T_Q4K && (u & 3) % 3 ? u ^ 3 : u;
+            const _Float16 h = (_Float16)v[u];
+            hi[at] = h;
+            lo[at] = (_Float16)(v[u] - (float)h);
+            sum += v[u];
+        }
+        const int sb = i >> 5, G = i & 31;
+        int s, g;
+        mg_place<TYPE>(G, s, g);
+        uint8_t* d = q + sb * 1024 + mg_xq_off(s, g);
+        *(gh8*)d = hi;
+        *(gh8*)(d + 256) = lo;
+        if constexpr (TYPE == T_Q4K) {
+            // the four groups of a 32-element sub-block are a quad of lanes
+            sum += dpp<DPP_XOR1>(sum);
+            sum += dpp<DPP_XOR2>(sum);
+            if ((G & 3) == 0) {
+                const float s32 = sum * 0.03125f;
+                const _Float16 h = (_Float16)s32;
+                sm[sb * 16 + (G >> 2)] = h;
+                sm[sb * 16 + 8 + (G >> 2)] = (_Float16)(s32 - (float)h);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------- GEMM --
+
+// A lane's weights of one superblock of its row.
+template <int TYPE>
+struct MgW;
+template <>
+struct MgW<T_Q4K> {
+    uint4 hdr, q[2];
+    static constexpr int LOADS = 3;
+};
+template <>
+struct MgW<T_Q6K> {
+    uint4 q[2], h[2];
+    uint4 sc;
+    uint32_t d;
+    static constexpr int LOADS = 9;  // at least: 36, 36, 20 and 2 bytes by at most 16
+};
+
+template <int TYPE>
+__device__ __forceinline__ void mg_load(const uint8_t* __restrict__ b, int g, MgW<TYPE>& w) {
+    if constexpr (TYPE == T_Q4K) {
+        w.hdr = *(const uint4*)b;
+        w.q[0] = *(const uint4*)(b + 16 + 32 * g);
+        w.q[1] = *(const uint4*)(b + 32 + 32 * g);
+    } else {
+        load32_a2(b + 32 * g, w.q[0], w.q[1]);
+        load32_a2(b + Q6K_QH + 32 * (g >> 1), w.h[0], w.h[1]);
+        w.sc = load16_a2(b + Q6K_SC);
+        w.d = *(const uint16_t*)(b + Q6K_D);
+    }
+}
+
+__device__ __forceinline__ gh2 as_h2(uint32_t v) { return __builtin_bit_cast(gh2, v); }
+__device__ __forceinline__ gh2 both(_Float16 v) { return gh2{v, v}; }
+__device__ __forceinline__ uint32_t dword_of(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+// two bytes (0..63) as fp16
+__device__ __forceinline__ gh2 bytes_h2(uint32_t w) {
+    return as_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) + both((_Float16)-1024.0f);
+}
+
+// What a lane needs of its superblock's header.
+template <int TYPE>
+struct MgS;
+template <>
+struct MgS<T_Q4K> {
+    gh2 s[2], o[2];  // low, high nibbles: scale and offset (twice each)
+};
+template <>
+struct MgS<T_Q6K> {
+    gh2 s[2][2];  // [low, high nibbles][bytes 0-15, 16-31]
+};
+
+template <int TYPE>
+__device__ __forceinline__ void mg_scales(const MgW<TYPE>& w, int g, MgS<TYPE>& c) {
+    if constexpr (TYPE == T_Q4K) {
+        // sub-blocks 2g and 2g + 1: scales 0-3 are bytes of hdr.y, 4-7 the
+        // low nibbles of hdr.w under hdr.y's top bits
+        const uint32_t lo = w.hdr.y & 0x3F3F3F3Fu, hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
+        const gh2 p = bytes_h2((g < 2 ? lo : hi) >> (16 * (g & 1)));
+        // (1024 + q) sc - 1024 sc, and for a high nibble left in place
+        // (1024 + 16 q) (sc / 16) - 64 sc: both are sc q, exact
+        c.s[0] = both(p[0]);
+        c.o[0] = both(p[0] * (_Float16)-1024.0f);
+        c.s[1] = both(p[1] * (_Float16)0.0625f);
+        c.o[1] = both(p[1] * (_Float16)-64.0f);
+    } else {
+        // the scale of element e is sc[e / 16]: 8 (g / 2) + 2 (g & 1) + 4 nibble + (byte / 16)
+        const uint32_t a = (g < 2 ? w.sc.x : w.sc.z) >> (16 * (g & 1)), b = (g < 2 ? w.sc.y : w.sc.w) >> (16 * (g & 1));
+        c.s[0][0] = both((_Float16)(int)(int8_t)(a & 0xff));
+        c.s[0][1] = both((_Float16)(int)(int8_t)((a >> 8) & 0xff));
+        c.s[1][0] = both((_Float16)(int)(int8_t)(b & 0xff));
+        c.s[1][1] = both((_Float16)(int)(int8_t)((b >> 8) & 0xff));
+    }
+}
+
+// (v & mask) | 0x64006400: two values of v under the exponent of 1024.  With
+// both constants in registers it is one instruction; left alone the compiler
+// takes two (and, or), each with a literal.
+__device__ __forceinline__ gh2 and_1024(uint32_t v, uint32_t mask, uint32_t k64) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(k64));
+    return as_h2(r);
+}
+
+// The B operand(s) of step s (compile-time): eight weights of the lane.
+template <int TYPE>
+__device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c, int s, int g, uint32_t k64, gh8& bh,
+                                          gh8& bl) {
+    const int nib = s & 1, at = (s >> 1) & 1, half = s >> 2;
+    uint32_t r[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t v = dword_of(w.q[half], 2 * at + i);
+        if constexpr (TYPE == T_Q4K) {
+            const uint32_t mask = nib ? 0x00F000F0u : 0x000F000Fu;
+            const gh2 e = and_1024(v, mask, k64), o = and_1024(v >> 8, mask, k64);
+            r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, c.s[nib], c.o[nib]));
+            r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(o, c.s[nib], c.o[nib]));
+        } else {
+            // two high bits of element q = (g & 1) + 2 nib: bits 2q of qh
+            const uint32_t h = dword_of(w.h[half], 2 * at + i) >> (2 * (g & 1));
+            const uint32_t q = nib ? ((v >> 4) & 0x0F0F0F0Fu) | (h & 0x30303030u)
+                                   : (v & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u);
+            const gh2 k = both((_Float16)-1056.0f);  // -(1024 + 32)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const gh2 t = as_h2(__builtin_amdgcn_perm(0x64646464u, q, j ? 0x04030402u : 0x04010400u)) + k;
+                const gh2 sc = c.s[nib][half];
+                const gh2 hi = t * sc;
+                r[2 * i + j] = __builtin_bit_cast(uint32_t, hi);
+                l[2 * i + j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, sc, -hi));
+            }
+        }
+    }
+    bh = __builtin_bit_cast(gh8, make_uint4(r[0], r[1], r[2], r[3]));
+    if constexpr (TYPE == T_Q6K) bl = __builtin_bit_cast(gh8, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// LDS of a workgroup: two stages of half a superblock, two of the sums
+constexpr int mg_stage(int rows) { return rows * 512; }
+constexpr int mg_lds(int rows) { return 2 * mg_stage(rows) + 2 * rows * 32; }
+
+template <int N>
+__device__ __forceinline__ void mg_wait_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// Keep a superblock's weights in registers at this point.
+__device__ __forceinline__ void mg_keep(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+__device__ __forceinline__ void mg_keep(MgW<T_Q4K>& w) {
+    mg_keep(w.hdr);
+    mg_keep(w.q[0]);
+    mg_keep(w.q[1]);
+}
+__device__ __forceinline__ void mg_keep(MgW<T_Q6K>& w) {
+    mg_keep(w.q[0]);
+    mg_keep(w.q[1]);
+    mg_keep(w.h[0]);
+    mg_keep(w.h[1]);
+    mg_keep(w.sc);
+    asm volatile("" : "+v"(w.d));
+}
+
+// The order of half a step's instructions: its LDS reads, then the unpacking
+// spread between the MFMAs.
+template <int TYPE, int MT>
+__device__ __forceinline__ void mg_sched(int n) {
+    constexpr int V = TYPE == T_Q6K ? 64 : 20;  // about the VALU instructions of a step's unpacking
+    __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+#pragma unroll
+    for (int i = 0; i < n * MT * MG_NT; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (V + 2 * MT * MG_NT - 1) / (2 * MT * MG_NT), 0);
+    }
+}
+
+struct MgArgs {
+    const uint8_t* w[2];
+    float* y[2];
+    const uint8_t* xq;
+    const uint8_t* sums;
+    int n, K, rowdiv;  // activation row of plane p: p / rowdiv
+};
+
+// A 16-byte LDS read serves a wave in four passes of 16 lanes, the first two
+// lanes {0-3, 12-15, 20-27} and the rest of 0-31 (two lane groups g of 16
+// rows c): with row c's piece p at place p ^ key(c) of its 128-byte line, the
+// 16 lanes of a pass read 16 different pieces of the 256 bytes of the banks.
+__device__ __forceinline__ int mg_key(int c) { return ((c >> 1) + 2) & 7; }
+
+// A tile of MT * 16 planes against the workgroup's weight rows.
+//
+// LDS holds two stages of half a superblock (four MFMA steps): the rows'
+// x' in octets of 8 rows, an octet's 128-byte line (hi or lo, step pair) as
+// one 1 KB DMA: row r's 16-byte piece u at place u ^ mg_key(r) of its line.
+// While a stage is computed, the next one's DMAs and the next superblock's
+// weight loads are in flight; a stage starts with one counted wait and one
+// barrier.
+template <int TYPE, int ROWS, int MT, bool GLU>
+__device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y, uint8_t* smem,
+                                        const int* s_plane, const float* s_inv) {
+    constexpr int NT = MG_NT, STAGE = mg_stage(ROWS);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c16 = lane & 15;
+    const int nsb = A.K >> 8;
+    const uint32_t rowbytes = (uint32_t)nsb * block_bytes(TYPE);
+
+    // this wave's weight rows: GLU takes 16 of the gate and the same of the up weight
+    uint32_t woff[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int r = GLU ? col0 + wave * 16 * (NT / 2) + 16 * (t % (NT / 2)) + c16 : col0 + wave * 16 * NT + 16 * t + c16;
+        woff[t] = (uint32_t)min(r, A.n - 1) * rowbytes;
+    }
+    auto load_w = [&](int sb, MgW<TYPE>(&w)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            mg_load<TYPE>((GLU && t >= NT / 2 ? W1 : W0) + (size_t)sb * block_bytes(TYPE) + woff[t], g, w[t]);
+    };
+
+    // x' DMAs: wave w moves (hi or lo, step pair) w of every octet
+    uint32_t xoff[2 * MT];
+#pragma unroll
+    for (int o = 0; o < 2 * MT; o++) {
+        const int r = s_plane[min(8 * o + (lane >> 3), np - 1)] / A.rowdiv;
+        xoff[o] = (uint32_t)r * (uint32_t)A.K * 4u + (uint32_t)(((lane & 7) ^ mg_key(8 * (o & 1) + (lane >> 3))) * 16);
+    }
+    uint32_t soff = 0;
+    if constexpr (TYPE == T_Q4K)
+        soff = (uint32_t)(s_plane[min(32 * (wave & 1) + (lane >> 1), np - 1)] / A.rowdiv) * (uint32_t)nsb * 32u + (lane & 1) * 16;
+    const uint32_t lds0 = lds_addr(smem);
+    auto issue = [&](int sb, int half) {
+        const uint8_t* base = A.xq + (size_t)sb * 1024 + half * 512 + wave * 128;
+        const uint32_t to = lds0 + half * STAGE + wave * 1024;
+#pragma unroll
+        for (int o = 0; o < 2 * MT; o++) dma16s(base, xoff[o], to + o * 4096);
+    };
+    auto issue_sums = [&](int sb) {
+        if constexpr (TYPE == T_Q4K)
+            if (wave < (MT + 1) / 2)
+                dma16s(A.sums + (size_t)sb * 32, soff, lds0 + 2 * STAGE + (sb & 1) * (ROWS * 32) + wave * 1024);
+    };
+    static_assert(MG_WAVES == 4, "a wave a (part, step pair)");
+
+    // the operand reads of a stage: row 16t + c16, piece 4 (s & 1) + g
+    const uint32_t a0 = (uint32_t)((c16 >> 3) * 4096 + (c16 & 7) * 128 + ((g ^ mg_key(c16)) * 16));
+    const uint8_t* ap[2] = {smem + a0, smem + (a0 ^ 64u)};
+
+    gf4 out[MT][NT], acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) out[t][j] = gf4{0.0f, 0.0f, 0.0f, 0.0f};
+    const gf4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // A step's MFMAs take the activations' lo, then their hi; its hi is read
+    // while lo's MFMAs run, the next step's lo while hi's run, and the next
+    // step's weights are unpacked between them.
+    // (Q6_K, whose weights take twice the registers, unpacks a step's own.)
+    constexpr bool AHEAD = TYPE == T_Q4K;
+    gh8 ah[MT], al[MT], bh[2][NT], bl[2][NT];
+    MgW<TYPE> w[NT], nxt[NT];
+    MgS<TYPE> sc[NT];
+    uint32_t k64 = 0x64006400u;
+    asm("" : "+v"(k64));
+    auto read_a = [&](int s, int lo, gh8(&a)[MT]) {
+        const uint8_t* p = ap[s & 1] + (s >> 2) * STAGE + lo * 2048 + ((s >> 1) & 1) * 1024;
+#pragma unroll
+        for (int t = 0; t < MT; t++) a[t] = *(const gh8*)(p + t * 8192);
+    };
+    auto unpack = [&](int s, int to) {
+#pragma unroll
+        for (int j = 0; j < NT; j++) mg_unpack<TYPE>(w[j], sc[j], s, g, k64, bh[to][j], bl[to][j]);
+    };
+    auto take_w = [&]() {
+        // the loaded weights become the current ones here, before the next
+        // loads and DMAs go out: the wait the compiler puts in front of their
+        // use then finds nothing younger in flight
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            w[j] = nxt[j];
+            mg_keep(w[j]);
+            mg_scales<TYPE>(w[j], g, sc[j]);
+        }
+    };
+    load_w(0, nxt);
+    issue(0, 0);
+    issue_sums(0);
+    mg_wait_barrier<0>();
+    take_w();
+    issue(0, 1);
+    load_w(min(1, nsb - 1), nxt);
+    read_a(0, 1, al);
+    if (AHEAD) unpack(0, 0);
+    for (int sb = 0; sb < nsb; sb++) {
+        float d[NT], dm32[NT];
+        gh8 bm[NT], am[MT];
+        const bool last = sb + 1 == nsb;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int cur = AHEAD ? s & 1 : 0;
+            read_a(s, 0, ah);
+            if (!AHEAD) unpack(s, 0);
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], bh[cur][j], s ? acc[t][j] : z, 0, 0, 0);
+            if (s < 7 && AHEAD) {
+                unpack(s + 1, cur ^ 1);
+                mg_sched<TYPE, MT>(1);
+            }
+            if (s == 3) {
+                // the half's last reads are done: the other half has landed
+                // (its DMAs are older than the weight loads), and this one's
+                // place is free
+                mg_wait_barrier<MgW<TYPE>::LOADS * NT>();
+                if (!last) {
+                    issue(sb + 1, 0);
+                    issue_sums(sb + 1);
+                }
+            }
+            if (s < 7) {
+                read_a(s + 1, 1, al);
+            } else {
+                // the epilogue's operands, before w moves on
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    if constexpr (TYPE == T_Q4K) {
+                        const uint4 hd = w[j].hdr;
+                        d[j] = f16_to_f32(hd.x & 0xffffu);
+                        dm32[j] = 32.0f * f16_to_f32(hd.x >> 16);
+                        const uint32_t ml = hd.z & 0x3F3F3F3Fu,
+                                       mh = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+                        const gh2 m0 = bytes_h2(ml), m1 = bytes_h2(ml >> 16), m2 = bytes_h2(mh), m3 = bytes_h2(mh >> 16);
+                        bm[j] = g < 2 ? gh8{m0[0], m0[1], m1[0], m1[1], m2[0], m2[1], m3[0], m3[1]} : gh8{};
+                    } else {
+                        d[j] = f16_to_f32(w[j].d);
+                    }
+                }
+                if constexpr (TYPE == T_Q4K) {
+                    const uint8_t* sp = smem + 2 * STAGE + (sb & 1) * (ROWS * 32) + c16 * 32 + (g & 1) * 16;
+#pragma unroll
+                    for (int t = 0; t < MT; t++) am[t] = *(const gh8*)(sp + t * 512);
+                }
+                if (!last) {  // uniform
+                    mg_wait_barrier<0>();
+                    take_w();
+                    issue(sb + 1, 1);
+                    load_w(min(sb + 2, nsb - 1), nxt);
+                    read_a(0, 1, al);
+                    if (AHEAD) unpack(0, 0);
+                }
+            }
+            if constexpr (TYPE == T_Q6K) {
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], bl[cur][j], acc[t][j], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], bh[cur][j], acc[t][j], 0, 0, 0);
+            if (s != 7 && AHEAD) mg_sched<TYPE, MT>(1);
+        }
+        // the superblock's scales (and the min term: K 0..7 the sums' hi,
+        // 8..15 their lo, the lanes of K 16..31 repeat them against zeros)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                if constexpr (TYPE == T_Q4K) {
+                    const gf4 mt = __builtin_amdgcn_mfma_f32_16x16x32_f16(am[t], bm[j], z, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        out[t][j][v] = __builtin_fmaf(d[j], acc[t][j][v], __builtin_fmaf(-dm32[j], mt[v], out[t][j][v]));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) out[t][j][v] = __builtin_fmaf(d[j], acc[t][j][v], out[t][j][v]);
+                }
+            }
+    }
+    // lane (g, c16): planes 16t + 4g + v of weight row c16 of each tile
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int q = 16 * t + 4 * g + v;
+            if (q >= np) continue;
+            float* yp = Y + (int64_t)s_plane[q] * A.n;
+            const float inv = s_inv[q];
+            if constexpr (GLU) {
+#pragma unroll
+                for (int j = 0; j < NT / 2; j++) {
+                    const int r = col0 + wave * 16 * (NT / 2) + 16 * j + c16;
+                    const float a = out[t][j][v] * inv, b = out[t][j + NT / 2][v] * inv;
+                    if (r < A.n) yp[r] = a / (1.0f + expf(-a)) * b;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const int r = col0 + wave * 16 * NT + 16 * j + c16;
+                    if (r < A.n) yp[r] = out[t][j][v] * inv;
+                }
+            }
+        }
+}
+
+// What bounds it: [128, 768, 2048] Q4_K, 2000 tokens top-8, the SwiGLU launch
+// (two weights, 201 TFLOP of hi and lo products) takes 290 us with its prep.
+// Left with only its loads (no MFMA, no unpacking) it took 273, with only
+// its arithmetic 246: the L2-to-LDS stream of x' (1.6 GB, each tile's planes
+// once a weight block) and the VALU and MFMA issue bound it about equally.
+// At 64 tokens it is the weight stream (113 MB a weight, 2.5 TB/s).  Eight
+// waves sharing one x' tile (half the stream) took 313: one workgroup a CU
+// leaves nothing to run at its barriers and its ends.
+// A workgroup takes item (tile of planes, weight block): items are dealt to
+// the XCDs in contiguous runs (workgroup b runs on XCD b % 8), so the blocks
+// of one tile, which read the same activations, and the tiles of one expert,
+// which read the same weights, meet in one XCD's L2.
+template <int TYPE, int ROWS, bool GLU>
+__global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 3 : 2) void k_moe_gemm(
+    MgArgs A, const int* __restrict__ hdr, const int4* __restrict__ tiles, const int* __restrict__ sorted,
+    const float* __restrict__ inv, int nblk, int pair) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ int s_plane[ROWS];
+    __shared__ float s_inv[ROWS];
+    const int per_tile = nblk << pair, total = hdr[1] * per_tile;
+    const int per = (total + 7) >> 3, at = (int)(blockIdx.x >> 3), item = (int)(blockIdx.x & 7) * per + at;
+    if (at >= per || item >= total) return;  // uniform
+    const int tile = item / per_tile, in = item - tile * per_tile;
+    const int second = pair ? in / nblk : 0, blk = in - second * nblk;
+    const int4 tl = tiles[tile];
+    const int e = tl.x, np = tl.z;
+    if ((int)threadIdx.x < ROWS) {
+        const int p = sorted[tl.y + min((int)threadIdx.x, np - 1)];
+        s_plane[threadIdx.x] = p;
+        s_inv[threadIdx.x] = inv[p / A.rowdiv];
+    }
+    __syncthreads();
+    const size_t ebytes = (size_t)e * A.n * (A.K >> 8) * block_bytes(TYPE);
+    const uint8_t* W0 = A.w[second] + ebytes;
+    const uint8_t* W1 = GLU ? A.w[1] + ebytes : W0;
+    float* Y = A.y[second];
+    const int col0 = blk * (GLU ? MG_COLS / 2 : MG_COLS);
+    const int mt = (np + 15) >> 4;  // uniform
+    if (mt == 1) {
+        mg_tile<TYPE, ROWS, 1, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
+    } else if (mt == 2) {
+        mg_tile<TYPE, ROWS, 2, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
+    } else if constexpr (ROWS == 64) {
+        if (mt == 3) mg_tile<TYPE, ROWS, 3, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
+        else mg_tile<TYPE, ROWS, 4, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
+    }
+}
+
+template <int TYPE>
+static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
+    const int64_t planes = c.batch * c.topk, rows = c.in_dim1 == 1 ? c.batch : planes;
+    const MgLayout l = mg_layout(c.E, planes, rows, c.k);
+    uint8_t* ws = (uint8_t*)c.ws;
+    int* hdr = (int*)ws;
+    int4* tiles = (int4*)(ws + l.tiles);
+    int* sorted = (int*)(ws + l.sorted);
+    float* inv = (float*)(ws + l.inv);
+    uint8_t* sums = ws + l.sums;
+    uint8_t* xq = ws + l.xq;
+    hipLaunchKernelGGL(k_moe_gemm_prep<TYPE>, dim3((unsigned)(c.E + (rows + 15) / 16)), dim3(1024), 0, s,
+                       c.x, (int)rows, (int)c.k, xq, (_Float16*)sums, inv, c.ids, (int)planes, (int)c.E, hdr, tiles,
+                       sorted, c.sticky, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, l.tile_rows);
+    if (hipError_t e = hipGetLastError()) return e;
+    const bool glu = c.mode == MOE_GLU;
+    const int pair = c.mode == MOE_PAIR ? 1 : 0;
+    const int cols = glu ? MG_COLS / 2 : MG_COLS;
+    const int nblk = (int)((c.n + cols - 1) / cols);
+    const int64_t items = (l.max_tiles * nblk) << pair;
+    const MgArgs a{{(const uint8_t*)c.w, (const uint8_t*)c.w2}, {c.y, c.y2}, xq, sums, (int)c.n, (int)c.k,
+                   c.in_dim1 == 1 ? (int)c.topk : 1};
+    const dim3 grid((unsigned)((items + 7) / 8 * 8));
+    auto gemm = [&](auto kern, int rows_) -> hipError_t {
+        if (hipError_t e = set_lds_limit((const void*)kern, mg_lds(rows_))) return e;
+        hipLaunchKernelGGL(kern, grid, dim3(64 * MG_WAVES), mg_lds(rows_), s, a, hdr, tiles, sorted, inv, nblk, pair);
+        return hipGetLastError();
+    };
+    if (l.tile_rows == 64) return glu ? gemm(k_moe_gemm<TYPE, 64, true>, 64) : gemm(k_moe_gemm<TYPE, 64, false>, 64);
+    return glu ? gemm(k_moe_gemm<TYPE, 32, true>, 32) : gemm(k_moe_gemm<TYPE, 32, false>, 32);
+}
+
+hipError_t launch_moe_gemm(const MoeGemmCall& c, hipStream_t s) {
+    return c.type == T_Q4K ? moe_gemm_type<T_Q4K>(c, s) : c.type == T_Q6K ? moe_gemm_type<T_Q6K>(c, s)
+                                                                         : hipErrorInvalidValue;
+}
+
+}  // namespace lloom

@@ -1,0 +1,150 @@
+"""The grouped GEMM of the routed experts (Q4_K and Q6_K with several planes
+an expert on average) against a float64 product of the dequantized
+weights (O.dequantize, the CPU oracle's to_float), through the public calls.
+
+Where it can go wrong: planes of one expert around the 16-row tile and the
+64-row cut (1, 15, 16, 17, 63, 64, 65, 129 and none), weight rows off the
+workgroup's 128 (64 for the SwiGLU), one superblock a row, activations one
+row a token and one a slot, tiles of 32 planes and of 64, an out-of-range id,
+and a capture whose workspace holds only the routing.
+
+The bound: a product enters as an exact weight against x' = hi + lo, off by
+at most 2^-22 of it (Q6_K drops lo * lo, 2^-22 more), and a row is summed in
+f32 in fewer than K / 8 steps, so |err| <= (2^-21 + K / 8 * 2^-24) * S with
+S = sum |x| (|d sc q| + |dmin m|) <= 3 max|w| sum |x|.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [1, 15, 16, 17, 63, 64, 65, 129, 0]
+FEW = [1, 4, 15, 16, 17, 33, 0, 8]  # up to 16 an expert on average: tiles of 32
+
+
+@pytest.fixture(scope="module")
+def L():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import lloom_amd
+
+    lloom_amd.lib()
+    return lloom_amd
+
+
+def _case(rng, dt, E, n, k, topk, per_slot, counts):
+    w = (rng.standard_normal((2, E, n, k)) * 0.05).astype(np.float32)
+    planes = sum(counts)
+    batch = -(-planes // topk)
+    flat = np.concatenate([np.full(c, e) for e, c in enumerate(counts)] + [np.full(batch * topk - planes, 0)])
+    ids = rng.permutation(flat).reshape(batch, topk).astype(np.int32)
+    x = rng.standard_normal((batch, topk if per_slot else 1, k)).astype(np.float32)
+    x[0, 0, :32] *= 1e4
+    x[-1] *= 1e-30
+    return w, x, ids
+
+
+def _want(dt, q, E, n, k, x, ids):
+    dense = O.dequantize(dt, q, E * n * k).reshape(E, n, k).astype(np.float64)
+    xs = np.broadcast_to(x, (ids.shape[0], ids.shape[1], k)).astype(np.float64)
+    want = np.zeros(ids.shape + (n,))
+    tol = np.zeros(ids.shape + (n,))
+    for e in range(E):
+        at = ids == e
+        want[at] = xs[at] @ dense[e].T
+        tol[at] = 3 * np.abs(xs[at]).sum(1, keepdims=True) * np.abs(dense[e]).max(1)[None]
+    return want, tol * (2.0 ** -21 + k / 8 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+@pytest.mark.parametrize("counts", [COUNTS, FEW], ids=["many", "few"])
+@pytest.mark.parametrize("n,k,topk,per_slot", [(200, 768, 4, False), (8, 256, 3, True), (1100, 512, 1, False),
+                                               (177, 2048, 2, True), (2065, 256, 2, False)])
+def test_moe_gemm_matches_f64(L, dt, n, k, topk, per_slot, counts):
+    rng = np.random.default_rng(n + k)
+    E = len(counts)
+    w, x, ids = _case(rng, dt, E, n, k, topk, per_slot, counts)
+    qg, qu = (L.QTensor.quantize(torch.from_numpy(v).cuda(), dt) for v in w)
+    xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    g, u = (q.indexed_moe_forward(xd, idd).cpu().numpy() for q in (qg, qu))
+    for got, q in ((g, qg), (u, qu)):
+        want, tol = _want(dt, q.data(), E, n, k, x, ids)
+        assert (np.abs(got - want) <= tol).all(), (np.abs(got - want) / tol).max()
+    # the pair is the two calls bit for bit, the SwiGLU their silu(g) * u
+    pg, pu = (v.cpu().numpy() for v in qg.indexed_moe_forward_pair(qu, xd, idd))
+    assert np.array_equal(pg.view(np.uint32), g.view(np.uint32)) and np.array_equal(pu.view(np.uint32), u.view(np.uint32))
+    glu = qg.indexed_moe_forward_glu_as(qu, xd, idd).cpu().numpy()
+    np.testing.assert_allclose(glu, g / (1 + np.exp(-g.astype(np.float64))) * u, rtol=2e-6, atol=1e-30)
+
+
+def test_moe_gemm_bad_id_and_nonfinite(L):
+    """A bad id zeroes its plane and is refused; a row with an infinity
+    spoils its own planes and no other."""
+    rng = np.random.default_rng(3)
+    E, n, k = 3, 70, 512
+    w = (rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)
+    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), O.Q4K)
+    ids = rng.integers(0, E, (40, 2)).astype(np.int32)
+    x = rng.standard_normal((40, 1, k)).astype(np.float32)
+    want, tol = _want(O.Q4K, q.data(), E, n, k, x, ids)
+    bad = ids.copy()
+    bad[7, 1] = E
+    xd = torch.from_numpy(x).cuda()
+    with pytest.raises(L.LloomHipError) as err:
+        q.indexed_moe_forward(xd, torch.from_numpy(bad).cuda())
+    assert err.value.name == "EEXPERT"
+    y = q.indexed_moe_forward(xd, torch.from_numpy(bad).cuda(), strict=False).cpu().numpy()
+    assert not y[7, 1].any()
+    y[7, 1] = want[7, 1]
+    assert (np.abs(y - want) <= tol).all()
+    from lloom_amd.lib import lib
+    from lloom_amd.quantized import _ctx
+
+    assert lib().lloom_hip_ctx_sync(_ctx(0)) == 4
+    x[5, 0, 100] = np.inf
+    y = q.indexed_moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()).cpu().numpy()
+    assert not np.isfinite(y[5]).any()
+    keep = np.arange(40) != 5
+    assert (np.abs(y - want) <= tol)[keep].all()
+
+
+def test_moe_gemm_captured(L):
+    """Replays equal the eager call, and a capture on a context whose
+    workspace cannot hold the activations is served all the same."""
+    import ctypes
+
+    from lloom_amd.lib import check, lib
+    from lloom_amd.quantized import _ptr
+
+    rng = np.random.default_rng(4)
+    E, n, k, batch, topk = 4, 96, 2048, 128, 4
+    w = (rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)
+    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), O.Q4K)
+    ids = torch.from_numpy(rng.integers(0, E, (batch, topk)).astype(np.int32)).cuda()
+    x = torch.from_numpy(rng.standard_normal((batch, topk, k)).astype(np.float32)).cuda()
+    eager = q.indexed_moe_forward(x, ids)
+    y = torch.empty_like(eager)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q.indexed_moe_forward_into(x, ids, y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert torch.equal(y, eager)
+    ctx = ctypes.c_void_p()
+    check(lib().lloom_hip_ctx_create(0, ctypes.byref(ctx)))
+    check(lib().lloom_hip_ctx_reserve(ctx, 1 << 20))
+    small = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(small):
+        check(lib().lloom_hip_moe_matmul(ctx, O.Q4K, _ptr(q.storage), E, n, k, _ptr(x), batch, topk, _ptr(ids), topk,
+                                         _ptr(y), 0, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    want, tol = _want(O.Q4K, q.data(), E, n, k, x.cpu().numpy(), ids.cpu().numpy())
+    for _ in range(2):
+        y.zero_()
+        small.replay()
+        assert (np.abs(y.cpu().numpy() - want) <= tol).all()
+    del small
+    lib().lloom_hip_ctx_destroy(ctx)
