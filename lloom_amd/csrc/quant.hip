@@ -97,51 +97,77 @@ __global__ __launch_bounds__(256) void k_quantize_q8_0(const float* __restrict__
 }
 
 // ------------------------------------------------------ Q4_K from_float --
-// utils.rs:227-290 make_qkx1_quants(nmax, ntry, x) -> (scale, -min), run
-// sequentially by one lane over its 32 values.
-__device__ void make_qkx1_quants_dev(int nmax, int ntry, const float* x, float* out_scale,
-                                     float* out_min) {
-    const int n = 32;
-    uint8_t l[32];
-    for (int i = 0; i < n; i++) l[i] = 0;
+// One lane fits one 32-element sub-block (the reference's sums are
+// sequential), 8 lanes a superblock, 8 superblocks a wave.  Bound by VALU
+// issue: about 13 instructions an element and fitting round, five rounds at
+// most.  So every loop is unrolled and the 32 values and 32 levels stay in
+// registers (with run-time indexes they lived in scratch memory: [8192, 2048]
+// 500 us), the wave's 8 KB of x come in as whole lines and reach their lanes
+// through LDS, and levels are floats (integers to 15: every product, sum of
+// squares and compare is exact).
+
+// n / d, correctly rounded, for r = 1 / d correctly rounded, and 2^-24 <= |d|:
+// n r corrected by its residual (exact in an fma) is within one ulp, and a
+// second correction of such a quotient rounds correctly (P. Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990, theorem on division).  Quotients past 64, infinities and
+// NaN come back uncorrected: the callers clamp them to 15 or 0.
+__device__ __forceinline__ float div_by(float n, float d, float r) {
+    const float q = n * r;
+    float c = __builtin_fmaf(__builtin_fmaf(-q, d, n), r, q);
+    c = __builtin_fmaf(__builtin_fmaf(-c, d, n), r, c);
+    return __builtin_fabsf(q) < 64.0f ? c : q;
+}
+
+// clampi(nearest_int(v), 0, 15) as a float: below zero the clamp decides, so
+// the half is added with no sign; a NaN gives 0, as the saturating cast does.
+__device__ __forceinline__ float level15(float v) {
+    return __builtin_truncf(__builtin_amdgcn_fmed3f(v + 0x1.fffffep-2f, 0.0f, 15.0f));
+}
+
+// utils.rs:227-290 make_qkx1_quants(15, 5, x) -> (scale, -min).
+__device__ __forceinline__ void make_qkx1_quants_dev(const float (&x)[32], float* out_scale, float* out_min) {
     // min_by(total_cmp) keeps the first minimum, max_by the last maximum.
     auto key = [](float f) -> int {
         int b = __builtin_bit_cast(int, f);
         return b ^ (int)(((unsigned)(b >> 31)) >> 1);
     };
-    float mn = x[0], mx = x[0];
+    // equal keys are equal bits, so the extreme keys name the values
     int kmn = key(x[0]), kmx = kmn;
-    for (int i = 1; i < n; i++) {
-        int kk = key(x[i]);
-        if (kk < kmn) { kmn = kk; mn = x[i]; }
-        if (kk >= kmx) { kmx = kk; mx = x[i]; }
+#pragma unroll
+    for (int i = 1; i < 32; i++) {
+        kmn = min(kmn, key(x[i]));
+        kmx = max(kmx, key(x[i]));
     }
+    const float mn = __builtin_bit_cast(float, key(__builtin_bit_cast(float, kmn)));
+    const float mx = __builtin_bit_cast(float, key(__builtin_bit_cast(float, kmx)));
     if (mx == mn) {
         *out_scale = 0.0f;
         *out_min = 0.0f;
         return;
     }
     float min = __builtin_fminf(mn, 0.0f);
-    float iscale = (float)nmax / (mx - min);
+    float iscale = 15.0f / (mx - min);
     float scale = 1.0f / iscale;
-    for (int it = 0; it < ntry; it++) {
-        float sumlx = 0.0f;
-        int suml2 = 0;
+    float l[32];
+#pragma unroll
+    for (int i = 0; i < 32; i++) l[i] = 0.0f;
+    for (int it = 0; it < 5; it++) {
+        float sumlx = 0.0f, suml2 = 0.0f;
         bool did_change = false;
-        for (int i = 0; i < n; i++) {
-            int li = clampi(nearest_int(iscale * (x[i] - min)), 0, nmax);
-            uint8_t cl = (uint8_t)li;
-            if (cl != l[i]) {
-                l[i] = cl;
-                did_change = true;
-            }
-            sumlx += (x[i] - min) * (float)li;
-            suml2 += li * li;
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            const float xm = x[i] - min, li = level15(iscale * xm);
+            did_change |= li != l[i];
+            l[i] = li;
+            sumlx += xm * li;
+            suml2 = __builtin_fmaf(li, li, suml2);
         }
-        scale = sumlx / (float)suml2;
+        scale = sumlx / suml2;
         float sum = -0.0f;
-        for (int i = 0; i < n; i++) sum += x[i] - scale * (float)l[i];
-        min = sum / (float)n;
+#pragma unroll
+        for (int i = 0; i < 32; i++) sum += x[i] - scale * l[i];
+        min = sum * 0.03125f;
         if (min > 0.0f) min = 0.0f;
         iscale = 1.0f / scale;
         if (!did_change) break;
@@ -160,82 +186,93 @@ __device__ __forceinline__ void scale_min_k4(int j, const uint8_t* q, int* d, in
     }
 }
 
+// max over the 8 lanes of a superblock
+__device__ __forceinline__ float max8(float v) {
+    v = __builtin_fmaxf(v, dpp<DPP_XOR1>(v));
+    v = __builtin_fmaxf(v, dpp<DPP_XOR2>(v));
+    return __builtin_fmaxf(v, dpp<DPP_HALF_MIRROR>(v));
+}
+
+struct __attribute__((packed, aligned(4))) Quad {
+    uint32_t v[4];
+};
+
+constexpr int Q4Q_WAVES = 4, Q4Q_PITCH = 36;  // floats from lane to lane in LDS
+
 // BlockQ4K::from_float (k_quants.rs:1622-1680).  8 lanes per superblock,
-// lane j fits sub-block j; a 64-thread group covers 8 superblocks.
-__global__ __launch_bounds__(64) void k_quantize_q4k(const float* __restrict__ x,
-                                                     uint8_t* __restrict__ out, int64_t nblocks) {
-    __shared__ uint8_t lbuf[8][256];
-    int t = threadIdx.x;
-    int g = t >> 3, j = t & 7;
-    int64_t blk = (int64_t)blockIdx.x * 8 + g;
-    bool ok = blk < nblocks;
-    const float* xb = x + (ok ? blk : 0) * 256;
+// lane j fits sub-block j; a wave covers 8 superblocks.
+__global__ __launch_bounds__(64 * Q4Q_WAVES) void k_quantize_q4k(const float* __restrict__ x,
+                                                                 uint8_t* __restrict__ out, int64_t nblocks) {
+    __shared__ __align__(16) float buf[Q4Q_WAVES][64 * Q4Q_PITCH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 7;
+    const int64_t blk0 = ((int64_t)blockIdx.x * Q4Q_WAVES + wave) * 8, blk = blk0 + (lane >> 3);
+    if (blk0 >= nblocks) return;  // the whole wave
+    // 8 KB as eight coalesced loads; float f of the wave's 2048 belongs to
+    // lane f / 32 (past the end the last superblock repeats)
+    float* lb = buf[wave];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int64_t src = min(blk0 + i, nblocks - 1) * 256 + 4 * lane;
+        *(float4*)(lb + (8 * i + (lane >> 3)) * Q4Q_PITCH + 4 * (lane & 7)) = *(const float4*)(x + src);
+    }
+    // a wave's LDS operations complete in order; this keeps the compiler from
+    // moving the reads above the writes
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     float xs[32];
-    for (int i = 0; i < 32; i++) xs[i] = ok ? xb[32 * j + i] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float4 v = *(const float4*)(lb + lane * Q4Q_PITCH + 4 * i);
+        xs[4 * i] = v.x;
+        xs[4 * i + 1] = v.y;
+        xs[4 * i + 2] = v.z;
+        xs[4 * i + 3] = v.w;
+    }
     float sc, mn;
-    make_qkx1_quants_dev(15, 5, xs, &sc, &mn);
-    // every lane of the group sees all 8 (scale, min)
-    float scales[8], mins[8];
+    make_qkx1_quants_dev(xs, &sc, &mn);
+    const float max_scale = max8(__builtin_fmaxf(sc, 0.0f)), max_min = max8(__builtin_fmaxf(mn, 0.0f));
+    const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
+    const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
+    const int a = nearest_int(inv_scale * sc), c = nearest_int(inv_min * mn);
+    const uint32_t ls = (uint32_t)(a < 63 ? a : 63) & 0xffu, lm = (uint32_t)(c < 63 ? c : 63) & 0xffu;
+    // the 12 scale bytes, as three dwords, from the eight lanes' pairs
+    uint32_t pk[3] = {0, 0, 0};
+#pragma unroll
     for (int i = 0; i < 8; i++) {
-        scales[i] = __shfl(sc, (t & ~7) + i, 64);
-        mins[i] = __shfl(mn, (t & ~7) + i, 64);
-    }
-    float max_scale = 0.0f, max_min = 0.0f;
-    for (int i = 0; i < 8; i++) {
-        max_scale = __builtin_fmaxf(scales[i], max_scale);
-        max_min = __builtin_fmaxf(mins[i], max_min);
-    }
-    float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
-    float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
-    uint8_t packed[12];
-    for (int i = 0; i < 12; i++) packed[i] = 0;
-    for (int i = 0; i < 8; i++) {
-        int a = nearest_int(inv_scale * scales[i]);
-        int c = nearest_int(inv_min * mins[i]);
-        uint8_t ls = (uint8_t)(a < 63 ? a : 63);
-        uint8_t lm = (uint8_t)(c < 63 ? c : 63);
+        const uint32_t v = (uint32_t)__shfl((int)(ls | lm << 8), (lane & ~7) + i, 64), s = v & 0xffu, m = v >> 8;
         if (i < 4) {
-            packed[i] = ls;
-            packed[i + 4] = lm;
+            pk[0] |= s << (8 * i);
+            pk[1] |= m << (8 * i);
         } else {
-            packed[i + 4] = (uint8_t)((ls & 0xF) | ((lm & 0xF) << 4));
-            packed[i - 4] |= (uint8_t)((ls >> 4) << 6);
-            packed[i] |= (uint8_t)((lm >> 4) << 6);
+            pk[2] |= ((s & 0xF) | ((m & 0xF) << 4)) << (8 * (i - 4));
+            pk[0] |= (((s >> 4) << 6) & 0xffu) << (8 * (i - 4));
+            pk[1] |= (((m >> 4) << 6) & 0xffu) << (8 * (i - 4));
         }
     }
-    uint16_t dh = f32_to_f16(max_scale / 63.0f);
-    uint16_t mh = f32_to_f16(max_min / 63.0f);
-    int s6, m6;
-    scale_min_k4(j, packed, &s6, &m6);
-    float d = f16_to_f32(dh) * (float)s6;
-    for (int i = 0; i < 32; i++) lbuf[g][32 * j + i] = 0;
+    const uint16_t dh = f32_to_f16(max_scale / 63.0f), mh = f32_to_f16(max_min / 63.0f);
+    const uint32_t b0 = byte_of(pk[0], j & 3), b1 = byte_of(pk[1], j & 3), b2 = byte_of(pk[2], j & 3);
+    const int s6 = (int)(j < 4 ? b0 & 63 : (b2 & 0xF) | ((b0 >> 6) << 4));
+    const int m6 = (int)(j < 4 ? b1 & 63 : (b2 >> 4) | ((b1 >> 6) << 4));
+    const float d = f16_to_f32(dh) * (float)s6, dm = f16_to_f32(mh) * (float)m6;
+    uint32_t q[8];  // this lane's 32 levels, a byte each
+#pragma unroll
+    for (int i = 0; i < 8; i++) q[i] = 0;
     if (d != 0.0f) {
-        float dm = f16_to_f32(mh) * (float)m6;
-        for (int i = 0; i < 32; i++) {
-            int lv = nearest_int((xs[i] + dm) / d);
-            lbuf[g][32 * j + i] = (uint8_t)clampi(lv, 0, 15);
-        }
+        const float r = 1.0f / d;
+#pragma unroll
+        for (int i = 0; i < 32; i++) q[i >> 2] |= (uint32_t)level15(div_by(xs[i] + dm, d, r)) << (8 * (i & 3));
     }
-    __syncthreads();
-    if (!ok) return;
+    // sub-blocks 2c and 2c + 1 share the 32 bytes qs[32c ..]: the even lane
+    // stores the first 16, the odd lane the rest
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t theirs = (uint32_t)dppi<DPP_XOR1>((int)((j & 1) ? q[i] : q[4 + i]));
+        w[i] = (j & 1) ? theirs | (q[4 + i] << 4) : q[i] | (theirs << 4);
+    }
+    if (blk >= nblocks) return;
     uint8_t* b = out + blk * Q4K_BYTES;
-    // lanes 2c and 2c+1 share the 32 bytes of qs[32c..32c+32)
-    int c = j >> 1, half = j & 1;
-    for (int i = 0; i < 16; i += 4) {
-        uint32_t w = 0;
-        for (int e = 0; e < 4; e++) {
-            int l = 16 * half + i + e;
-            uint32_t v = lbuf[g][64 * c + l] | (lbuf[g][64 * c + 32 + l] << 4);
-            w |= v << (8 * e);
-        }
-        *(uint32_t*)(b + 16 + 32 * c + 16 * half + i) = w;
-    }
-    if (j == 0) {
-        *(uint32_t*)b = (uint32_t)dh | ((uint32_t)mh << 16);
-        for (int i = 0; i < 12; i += 4)
-            *(uint32_t*)(b + 4 + i) = packed[i] | (packed[i + 1] << 8) | (packed[i + 2] << 16) |
-                                      ((uint32_t)packed[i + 3] << 24);
-    }
+    *(Quad*)(b + 16 + 16 * j) = Quad{{w[0], w[1], w[2], w[3]}};
+    if (j == 0) *(Quad*)b = Quad{{(uint32_t)dh | ((uint32_t)mh << 16), pk[0], pk[1], pk[2]}};
 }
 
 // ------------------------------------------------------ Q6_K from_float --
@@ -568,7 +605,8 @@ hipError_t launch_quantize_weights(int type, const float* x, void* out, int64_t 
         case T_Q8K: return launch_quantize_act(type, x, out, elems, s);
         case T_Q4K: {
             int64_t nb = elems / 256;
-            hipLaunchKernelGGL(k_quantize_q4k, dim3(grid_of(nb, 8)), dim3(64), 0, s, x, (uint8_t*)out, nb);
+            hipLaunchKernelGGL(k_quantize_q4k, dim3(grid_of(nb, 8 * Q4Q_WAVES)), dim3(64 * Q4Q_WAVES), 0, s, x, (uint8_t*)out,
+                               nb);
             return hipGetLastError();
         }
         case T_Q6K: {
