@@ -256,8 +256,12 @@ int lloom_hip_dequantize(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, i
 // The route a qmatmul call takes and the workspace it needs.  Activations
 // in F16 (matmul_t_f16, k_quants.rs:2802-2835: the f16 lhs converted to f32,
 // quantized to the VecDotType and dotted exactly as the f32 path; each f32
-// sum rounded to f16) are converted into the workspace first, and F16
-// outputs are formed in f32 in the workspace and rounded at the end.
+// sum rounded to f16) are widened where the kernels load them, and outputs
+// rounded where the GEMMs store them; the kernels that load f32 alone (one to
+// four rows) get x converted into the workspace, and the decode kernels' y is
+// formed there and rounded at the end.  The plan holds room for x and y
+// in f32 whichever they are, so what a call asks for, and what the
+// allocation-free call refuses, does not depend on the route.
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -303,21 +307,28 @@ int qmatmul_run(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, int64_t n,
     const float* x = (const float*)x_dev;
     float* y = (float*)y_dev;
     if (x_dtype == T_F16) {
-        float* x32 = (float*)((uint8_t*)ws + p.x32_off);
-        HIP_OK(launch_cast(T_F16, x_dev, T_F32, x32, m * k, s));
-        x = x32;
+        if (p.decode ? matvec_reads_f16(ggml_type, n, k, m) : gemm_reads_f16(ggml_type, n, k, m)) {
+            epi |= EPI_X16;
+        } else {
+            float* x32 = (float*)((uint8_t*)ws + p.x32_off);
+            HIP_OK(launch_cast(T_F16, x_dev, T_F32, x32, m * k, s));
+            x = x32;
+        }
     }
-    if (y_dtype == T_F16) {
+    const bool y16 = y_dtype == T_F16 && !p.decode && gemm_writes_f16(ggml_type, n, k, m, ctx->prefill_mma);
+    if (y16) {
+        epi |= EPI_Y16;
+    } else if (y_dtype == T_F16) {
         y = (float*)((uint8_t*)ws + p.y32_off);
         // the multiply-into store reads y: its f16 values, widened exactly
-        if (epi == EPI_MUL_INTO) HIP_OK(launch_cast(T_F16, y_dev, T_F32, y, m * n, s));
+        if (epi_store(epi) == EPI_MUL_INTO) HIP_OK(launch_cast(T_F16, y_dev, T_F32, y, m * n, s));
     }
     if (p.decode)
         HIP_OK(launch_matvec(ggml_type, w_dev, x, y, n, k, m, ws, epi, s));
     else
         HIP_OK(launch_gemm(ggml_type, w_dev, x, y, n, k, m, ws, p.total > p.x32_off ? p.x32_off : ws_cap,
                            ctx->prefill_mma, epi, s));
-    if (y_dtype == T_F16) HIP_OK(launch_cast(T_F32, y, T_F16, y_dev, m * n, s));
+    if (y_dtype == T_F16 && !y16) HIP_OK(launch_cast(T_F32, y, T_F16, y_dev, m * n, s));
     return LLOOM_HIP_OK;
 }
 

@@ -69,6 +69,7 @@ static size_t prep_bytes(int64_t m, int64_t k) {
     return q + s + (size_t)(k / 256) * m * sizeof(float) + 256;
 }
 
+template <bool X16>
 __global__ __launch_bounds__(256) void k_gemm_prep_q8k(const float* __restrict__ x, int8_t* __restrict__ xq,
                                                        int8_t* __restrict__ sp, float* __restrict__ dyt, int m,
                                                        int k) {
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(256) void k_gemm_prep_q8k(const float* __restrict__
     const int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (blk >= (int64_t)m * nsb) return;
     const int mi = (int)(blk / nsb), sb = (int)(blk - (int64_t)mi * nsb);
-    const float4 v = *(const float4*)(x + (int64_t)mi * k + sb * 256 + 4 * lane);
+    const float4 v = load_x4<X16>(x, (int64_t)mi * k + sb * 256 + 4 * lane);
     float d;
     int bs;
     const uint32_t q = q8k_block_wave(v, &d, &bs);
@@ -348,8 +349,8 @@ __global__ __launch_bounds__(G_THREADS) void k_gemm_q4k(const uint8_t* __restric
             for (int r = 0; r < 16; r++) {
                 const int row = m0 + wm * G_MT * 32 + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
                 if (row < m) {
-                    if (epi == EPI_STORE) Y[(int64_t)row * n + col] = out[a][b][r];
-                    else store_epi_slow(&Y[(int64_t)row * n + col], out[a][b][r], epi);
+                    if (epi == EPI_STORE) store_plain<false>(Y, (int64_t)row * n + col, out[a][b][r]);
+                    else store_epi_slow<false>(Y, (int64_t)row * n + col, out[a][b][r], epi);
                 }
             }
         }
@@ -455,6 +456,7 @@ static size_t x16_bytes(int64_t m, int64_t k) {
     return a + b + (size_t)(k / 256) * m * sizeof(float) + 256;
 }
 
+template <bool X16>
 __global__ __launch_bounds__(256) void k_gemm_prep_x16(const float* __restrict__ x, _Float16* __restrict__ x16,
                                                        _Float16* __restrict__ amin, float* __restrict__ dyt, int m,
                                                        int k) {
@@ -467,11 +469,11 @@ __global__ __launch_bounds__(256) void k_gemm_prep_x16(const float* __restrict__
     const bool real = blk0 < nblk;  // per 16-lane row
     const int64_t blk = real ? blk0 : 0;
     const int mi = (int)(blk / nsb), sb = (int)(blk - (int64_t)mi * nsb);
-    const float* xr = x + (int64_t)mi * k + sb * 256 + 16 * j;
+    const int64_t xr = (int64_t)mi * k + sb * 256 + 16 * j;
     float xs[16];
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        const float4 v = *(const float4*)(xr + 4 * c);
+        const float4 v = load_x4<X16>(x, xr + 4 * c);
         xs[4 * c] = v.x;
         xs[4 * c + 1] = v.y;
         xs[4 * c + 2] = v.z;
@@ -570,7 +572,7 @@ __device__ __forceinline__ v8h build_kk(const uint4& raw, const BScale& bs, int 
     return __builtin_bit_cast(v8h, make_uint4(p0.x, p0.y, p1.x, p1.y));
 }
 
-template <int MT, int WNW, int WV>
+template <int MT, int WNW, int WV, bool Y16>
 __global__ __launch_bounds__(64 * WV) void k_gemm_q4k_x16(const uint8_t* __restrict__ W,
                                                             const _Float16* __restrict__ x16,
                                                             const _Float16* __restrict__ amin,
@@ -832,8 +834,8 @@ __global__ __launch_bounds__(64 * WV) void k_gemm_q4k_x16(const uint8_t* __restr
             for (int r = 0; r < 16; r++) {
                 const int row = m0 + wm * (32 * MT) + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
                 if (row < m) {
-                    if (epi == EPI_STORE) Y[(int64_t)row * n + col] = out[a][b][r];
-                    else store_epi_slow(&Y[(int64_t)row * n + col], out[a][b][r], epi);
+                    if (epi == EPI_STORE) store_plain<Y16>(Y, (int64_t)row * n + col, out[a][b][r]);
+                    else store_epi_slow<Y16>(Y, (int64_t)row * n + col, out[a][b][r], epi);
                 }
             }
         }
@@ -850,7 +852,7 @@ __global__ __launch_bounds__(64 * WV) void k_gemm_q4k_x16(const uint8_t* __restr
 // step's MFMAs; each activation operand serves the NT weight tiles (the
 // activations re-read per column block are this kernel's main traffic).
 // The waves' partial sums meet in LDS in a fixed order.
-template <int KS, int NT>
+template <int KS, int NT, bool Y16>
 __global__ __launch_bounds__(64 * KS) void k_gemm_q4k_skinny(const uint8_t* __restrict__ W,
                                                                const _Float16* __restrict__ x16,
                                                                const _Float16* __restrict__ amin,
@@ -955,7 +957,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemm_q4k_skinny(const uint8_t* __re
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int row = m0 + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (row < m) store_epi(&Y[(int64_t)row * n + col], out[b][r], epi);
+                if (row < m) store_epi<Y16>(Y, (int64_t)row * n + col, out[b][r], epi);
             }
         }
     }
@@ -1023,10 +1025,11 @@ template <int MT, int WNW, int WV>
 static hipError_t launch_x16(const void* w, const X16Ptrs& p, float* y, int64_t n, int64_t k, int64_t m,
                              int epi, hipStream_t s) {
     using C = XCfg<MT, WNW, WV>;
-    if (hipError_t e = set_lds_limit((const void*)k_gemm_q4k_x16<MT, WNW, WV>, C::LDS)) return e;
+    const auto kern = (epi & EPI_Y16) ? k_gemm_q4k_x16<MT, WNW, WV, true> : k_gemm_q4k_x16<MT, WNW, WV, false>;
+    if (hipError_t e = set_lds_limit((const void*)kern, C::LDS)) return e;
     const unsigned grid = (unsigned)(((m + C::BM - 1) / C::BM) * ((n + C::BN - 1) / C::BN));
-    hipLaunchKernelGGL((k_gemm_q4k_x16<MT, WNW, WV>), dim3(grid), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w,
-                       p.x16, p.amin, p.dyt, y, (int)m, (int)n, (int)k, epi);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.x16, p.amin, p.dyt, y,
+                       (int)m, (int)n, (int)k, epi_store(epi));
     return hipGetLastError();
 }
 
@@ -1063,7 +1066,7 @@ hipError_t launch_gemm(int type, const void* w, const float* x, float* y, int64_
     if (type == T_Q4K && m <= skinny_max_rows() && fits_32bit(n, k, m) && mode != GEMM_INT8) {
         X16Ptrs p = x16_ptrs(qbuf, m, k);
         const int64_t nb = m * (k / 256);
-        hipLaunchKernelGGL(k_gemm_prep_x16, dim3((unsigned)((nb + 15) / 16)), dim3(256), 0, s, x, p.x16, p.amin,
+        hipLaunchKernelGGL((epi & EPI_X16) ? k_gemm_prep_x16<true> : k_gemm_prep_x16<false>, dim3((unsigned)((nb + 15) / 16)), dim3(256), 0, s, x, p.x16, p.amin,
                            p.dyt, (int)m, (int)k);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -1074,18 +1077,14 @@ hipError_t launch_gemm(int type, const void* w, const float* x, float* y, int64_
         const int nt = ctiles * layers >= 4 * 256 ? 4 : ctiles * layers >= 2 * 256 ? 2 : 1;
         const dim3 grid((unsigned)((ctiles + nt - 1) / nt), (unsigned)layers);
         const uint8_t* wb = (const uint8_t*)w;
-        if (nt == 4)
-            hipLaunchKernelGGL((k_gemm_q4k_skinny<4, 4>), grid, dim3(256), 0, s, wb, p.x16, p.amin, p.dyt, y, (int)m,
-                               (int)n, (int)k, epi);
-        else if (nt == 2)
-            hipLaunchKernelGGL((k_gemm_q4k_skinny<4, 2>), grid, dim3(256), 0, s, wb, p.x16, p.amin, p.dyt, y, (int)m,
-                               (int)n, (int)k, epi);
-        else if (k >= 8 * 256)
-            hipLaunchKernelGGL((k_gemm_q4k_skinny<8, 1>), grid, dim3(512), 0, s, wb, p.x16, p.amin, p.dyt, y, (int)m,
-                               (int)n, (int)k, epi);
-        else
-            hipLaunchKernelGGL((k_gemm_q4k_skinny<4, 1>), grid, dim3(256), 0, s, wb, p.x16, p.amin, p.dyt, y, (int)m,
-                               (int)n, (int)k, epi);
+        const bool y16 = epi & EPI_Y16;
+        const int ks = nt == 1 && k >= 8 * 256 ? 8 : 4;
+        const auto kern = nt == 4   ? (y16 ? k_gemm_q4k_skinny<4, 4, true> : k_gemm_q4k_skinny<4, 4, false>)
+                          : nt == 2 ? (y16 ? k_gemm_q4k_skinny<4, 2, true> : k_gemm_q4k_skinny<4, 2, false>)
+                          : ks == 8 ? (y16 ? k_gemm_q4k_skinny<8, 1, true> : k_gemm_q4k_skinny<8, 1, false>)
+                                    : (y16 ? k_gemm_q4k_skinny<4, 1, true> : k_gemm_q4k_skinny<4, 1, false>);
+        hipLaunchKernelGGL(kern, grid, dim3(64 * ks), 0, s, wb, p.x16, p.amin, p.dyt, y, (int)m, (int)n, (int)k,
+                           epi_store(epi));
         return hipGetLastError();
     }
     if (type == T_Q6K && m >= q6_min_rows() && q6_gemm_fits(n, k, m))
@@ -1096,7 +1095,7 @@ hipError_t launch_gemm(int type, const void* w, const float* x, float* y, int64_
     if (type == T_Q4K && fits_32bit(n, k, m) && mode != GEMM_INT8) {
         X16Ptrs p = x16_ptrs(qbuf, m, k);
         const int64_t nb = m * (k / 256);
-        hipLaunchKernelGGL(k_gemm_prep_x16, dim3((unsigned)((nb + 15) / 16)), dim3(256), 0, s, x, p.x16, p.amin,
+        hipLaunchKernelGGL((epi & EPI_X16) ? k_gemm_prep_x16<true> : k_gemm_prep_x16<false>, dim3((unsigned)((nb + 15) / 16)), dim3(256), 0, s, x, p.x16, p.amin,
                            p.dyt, (int)m, (int)k);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -1120,13 +1119,13 @@ hipError_t launch_gemm(int type, const void* w, const float* x, float* y, int64_
         if (hipError_t e = set_lds_limit((const void*)k_gemm_q4k, G_LDS)) return e;
         PrepPtrs p = prep_ptrs(qbuf, m, k);
         const int64_t nb = m * (k / 256);
-        hipLaunchKernelGGL(k_gemm_prep_q8k, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, s, x, p.xq, p.sp, p.dyt,
+        hipLaunchKernelGGL((epi & EPI_X16) ? k_gemm_prep_q8k<true> : k_gemm_prep_q8k<false>, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, s, x, p.xq, p.sp, p.dyt,
                            (int)m, (int)k);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const unsigned grid = (unsigned)(((m + G_BM - 1) / G_BM) * ((n + G_BN - 1) / G_BN));
         hipLaunchKernelGGL(k_gemm_q4k, dim3(grid), dim3(G_THREADS), G_LDS, s, (const uint8_t*)w, p.xq, p.sp, p.dyt,
-                           y, (int)m, (int)n, (int)k, epi);
+                           y, (int)m, (int)n, (int)k, epi_store(epi));
         return hipGetLastError();
     }
     if (type == T_Q8_0 && q8_gemm_fits(n, k, m)) return launch_q8_gemm(w, x, y, n, k, m, qbuf, ws_cap, epi, s);
@@ -1138,6 +1137,18 @@ hipError_t launch_gemm(int type, const void* w, const float* x, float* y, int64_
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// The decode tiles load f32 (and with the decode kernels store it).
+bool gemm_reads_f16(int type, int64_t n, int64_t k, int64_t m) {
+    return !(type == T_Q8_0 && !q8_gemm_fits(n, k, m)) && !(type == T_Q4K && !fits_32bit(n, k, m));
+}
+bool gemm_writes_f16(int type, int64_t n, int64_t k, int64_t m, int mode) {
+    mode = gemm_mode(mode, m);
+    if (!gemm_reads_f16(type, n, k, m) || use_dma_ma(type, k, m)) return false;
+    if (type == T_Q6K) return m >= q6_min_rows() && q6_gemm_fits(n, k, m);
+    if (type == T_Q4K && mode == GEMM_INT8) return !use_mq(type, m) && gemm_i8_fits(n, k, m);
+    return !(type == T_Q4K && m > skinny_max_rows() && use_mq(type, m));
 }
 
 }  // namespace lloom

@@ -180,7 +180,7 @@ bool gemm_i8_fits(int64_t n, int64_t k, int64_t m) {
 // from_float (k_quants.rs:2400-2438).
 // Weight prep (the blocks after): one thread per (column, superblock), a
 // wave's lanes 64 consecutive columns of one superblock.
-template <int NB, int BNR>
+template <int NB, int BNR, bool X16>
 __global__ __launch_bounds__(256) void k_gemm_prep_i8(const float* __restrict__ x, const uint8_t* __restrict__ W,
                                                       I8Ptrs p, int m, int n, int k, int act_blocks) {
     const int lane = threadIdx.x & 63;
@@ -238,13 +238,13 @@ __global__ __launch_bounds__(256) void k_gemm_prep_i8(const float* __restrict__ 
     if (wid >= (int64_t)(p.mp / 4) * ngr) return;
     const int mi = (int)(wid / ngr) * 4 + (lane >> 4), sb0 = NB * (int)(wid % ngr);
     const bool real = mi < m;
-    const float* xr = x + (int64_t)min(mi, m - 1) * k + 16 * j;
+    const int64_t xr = (int64_t)min(mi, m - 1) * k + 16 * j;
     float xs[NB][16];
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const float4 v = *(const float4*)(xr + (sb0 + b) * 256 + 4 * c);
+            const float4 v = load_x4<X16>(x, xr + (sb0 + b) * 256 + 4 * c);
             xs[b][4 * c] = v.x;
             xs[b][4 * c + 1] = v.y;
             xs[b][4 * c + 2] = v.z;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void k_gemm_prep_i8(const float* __restrict__ 
     }
 }
 
-template <int NCW>
+template <int NCW, bool Y16>
 __global__ __launch_bounds__(THREADS) void k_gemm_q4k_i8(const uint8_t* __restrict__ W, I8Ptrs p,
                                                          float* __restrict__ Y, int m, int n, int k, int epi) {
     // NCW 16-column halves a wave: a tile of 8 x 16 NCW weight columns
@@ -600,12 +600,17 @@ __global__ __launch_bounds__(THREADS) void k_gemm_q4k_i8(const uint8_t* __restri
 #pragma unroll
         for (int c = 0; c < NCW; c++) {
             const int col = n0 + WC * wave + 16 * c + 4 * g;
-            if (epi == EPI_STORE && col + 3 < n) {
-                *(float4*)(yr + col) = make_float4(out[R][c][0], out[R][c][1], out[R][c][2], out[R][c][3]);
+            if (epi == EPI_STORE && col + 3 < n && !(Y16 && (n & 3))) {
+                if constexpr (Y16)  // n a multiple of 4: the four halves are 8-byte aligned
+                    *(uint2*)((uint16_t*)Y + (int64_t)row * n + col) =
+                        make_uint2(f32_to_f16(out[R][c][0]) | (uint32_t)f32_to_f16(out[R][c][1]) << 16,
+                                   f32_to_f16(out[R][c][2]) | (uint32_t)f32_to_f16(out[R][c][3]) << 16);
+                else
+                    *(float4*)(yr + col) = make_float4(out[R][c][0], out[R][c][1], out[R][c][2], out[R][c][3]);
             } else {
 #pragma unroll
                 for (int v = 0; v < 4; v++)
-                    if (col + v < n) store_epi_slow(yr + col + v, out[R][c][v], epi);
+                    if (col + v < n) store_epi_slow<Y16>(Y, (int64_t)row * n + col + v, out[R][c][v], epi);
             }
         }
     }
@@ -622,24 +627,23 @@ template <int NCW>
 static hipError_t launch_i8(const void* w, const float* x, float* y, int64_t n, int64_t k, int64_t m, void* ws,
                             int epi, hipStream_t s) {
     constexpr int BNT = I8C<NCW>::BN, LDST = I8C<NCW>::LDS;
-    if (hipError_t e = set_lds_limit((const void*)k_gemm_q4k_i8<NCW>, LDST)) return e;
+    const auto kern = (epi & EPI_Y16) ? k_gemm_q4k_i8<NCW, true> : k_gemm_q4k_i8<NCW, false>;
+    if (hipError_t e = set_lds_limit((const void*)kern, LDST)) return e;
     const I8Ptrs p = i8_ptrs(ws, n, m, k);
     const int64_t nsb = k / 256;
     const int64_t wblocks = p.np * nsb / 256;
-    if (nsb % 2 == 0) {
-        const int64_t ablocks = (p.mp / 4 * (nsb / 2) + 3) / 4;
-        hipLaunchKernelGGL((k_gemm_prep_i8<2, BNT>), dim3((unsigned)(ablocks + wblocks)), dim3(256), 0, s, x,
-                           (const uint8_t*)w, p, (int)m, (int)n, (int)k, (int)ablocks);
-    } else {
-        const int64_t ablocks = (p.mp / 4 * nsb + 3) / 4;
-        hipLaunchKernelGGL((k_gemm_prep_i8<1, BNT>), dim3((unsigned)(ablocks + wblocks)), dim3(256), 0, s, x,
-                           (const uint8_t*)w, p, (int)m, (int)n, (int)k, (int)ablocks);
-    }
+    const int nb = nsb % 2 == 0 ? 2 : 1;
+    const int64_t ablocks = (p.mp / 4 * (nsb / nb) + 3) / 4;
+    const bool x16 = epi & EPI_X16;
+    const auto prep = nb == 2 ? (x16 ? k_gemm_prep_i8<2, BNT, true> : k_gemm_prep_i8<2, BNT, false>)
+                              : (x16 ? k_gemm_prep_i8<1, BNT, true> : k_gemm_prep_i8<1, BNT, false>);
+    hipLaunchKernelGGL(prep, dim3((unsigned)(ablocks + wblocks)), dim3(256), 0, s, x, (const uint8_t*)w, p, (int)m,
+                       (int)n, (int)k, (int)ablocks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const unsigned grid = (unsigned)((p.mp / BM) * ((n + BNT - 1) / BNT));
-    hipLaunchKernelGGL(k_gemm_q4k_i8<NCW>, dim3(grid), dim3(THREADS), LDST, s, (const uint8_t*)w, p, y, (int)m,
-                       (int)n, (int)k, epi);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(THREADS), LDST, s, (const uint8_t*)w, p, y, (int)m,
+                       (int)n, (int)k, epi_store(epi));
     return hipGetLastError();
 }
 

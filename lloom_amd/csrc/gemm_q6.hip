@@ -59,7 +59,7 @@ static size_t q6_prep_bytes(int64_t m, int64_t k, int64_t xq_rows = 0) {
 // GPU with such workgroups take one block a wave (k_gemm_prep_q6_wave).
 // (Block indices are 32-bit: m * k / 256 < 2^31.)
 constexpr int64_t Q6_XPREP_RB2 = 256 * 32;  // blocks from which a row takes two
-template <int RB, int W>
+template <int RB, int W, bool X16>
 __device__ __forceinline__ void q6_prep_x(const float* __restrict__ x, int8_t* __restrict__ xq,
                                           float* __restrict__ dyt, int m, int k, int mp, uint32_t bid) {
     const int lane = threadIdx.x & 63, j = lane & 15;
@@ -69,10 +69,10 @@ __device__ __forceinline__ void q6_prep_x(const float* __restrict__ x, int8_t* _
 #pragma unroll
     for (int r = 0; r < RB; r++) {
         const uint32_t blk = min(b0 + 4 * W * r, nblk - 1);  // past the end: a duplicate, not stored
-        const float4* src = (const float4*)(x + (size_t)blk * 256 + 16 * j);
+        const int64_t src = (int64_t)blk * 256 + 16 * j;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const float4 v = src[u];
+            const float4 v = load_x4<X16>(x, src + 4 * u);
             xs[r][4 * u] = v.x;
             xs[r][4 * u + 1] = v.y;
             xs[r][4 * u + 2] = v.z;
@@ -93,20 +93,21 @@ __device__ __forceinline__ void q6_prep_x(const float* __restrict__ x, int8_t* _
     }
 }
 
-template <int RB, int W>
+template <int RB, int W, bool X16>
 __global__ __launch_bounds__(64 * W) void k_gemm_prep_q6(const float* __restrict__ x, int8_t* __restrict__ xq,
                                                          float* __restrict__ dyt, int m, int k, int mp) {
-    q6_prep_x<RB, W>(x, xq, dyt, m, k, mp, blockIdx.x);
+    q6_prep_x<RB, W, X16>(x, xq, dyt, m, k, mp, blockIdx.x);
 }
 // The same blocks, one a wave (its 64 lanes four elements each), for calls
 // with few blocks: more waves, each with less to do.
+template <bool X16>
 __global__ __launch_bounds__(256) void k_gemm_prep_q6_wave(const float* __restrict__ x, int8_t* __restrict__ xq,
                                                            float* __restrict__ dyt, int m, int k, int mp) {
     const int lane = threadIdx.x & 63;
     const uint32_t nsb = (uint32_t)k >> 8, nblk = (uint32_t)m * nsb;
     const uint32_t blk = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (blk >= nblk) return;
-    const float4 v = *(const float4*)(x + (size_t)blk * 256 + 4 * lane);
+    const float4 v = load_x4<X16>(x, (int64_t)blk * 256 + 4 * lane);
     float d;
     int bs;
     const uint32_t q = q8k_block_wave(v, &d, &bs);
@@ -115,14 +116,14 @@ __global__ __launch_bounds__(256) void k_gemm_prep_q6_wave(const float* __restri
     if (lane == 0) dyt[(size_t)sb * mp + mi] = d;
 }
 // The launch for nb blocks.
-static hipError_t launch_prep_q6(const float* x, int8_t* xq, float* dyt, int64_t m, int64_t k, int64_t mp, hipStream_t s) {
+static hipError_t launch_prep_q6(const float* x, bool x16, int8_t* xq, float* dyt, int64_t m, int64_t k, int64_t mp,
+                                 hipStream_t s) {
     const int64_t nb = m * (k / 256);
-    if (nb >= Q6_XPREP_RB2)
-        hipLaunchKernelGGL((k_gemm_prep_q6<2, 4>), dim3((unsigned)((nb + 31) / 32)), dim3(256), 0, s, x, xq, dyt,
-                           (int)m, (int)k, (int)mp);
-    else  // few blocks: one a wave (more waves in flight)
-        hipLaunchKernelGGL(k_gemm_prep_q6_wave, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, s, x, xq, dyt, (int)m,
-                           (int)k, (int)mp);
+    const bool two = nb >= Q6_XPREP_RB2;  // few blocks: one a wave (more waves in flight)
+    const auto prep = two ? (x16 ? k_gemm_prep_q6<2, 4, true> : k_gemm_prep_q6<2, 4, false>)
+                          : (x16 ? k_gemm_prep_q6_wave<true> : k_gemm_prep_q6_wave<false>);
+    hipLaunchKernelGGL(prep, dim3((unsigned)(two ? (nb + 31) / 32 : (nb + 3) / 4)), dim3(256), 0, s, x, xq, dyt, (int)m,
+                       (int)k, (int)mp);
     return hipGetLastError();
 }
 
@@ -180,7 +181,7 @@ __device__ __forceinline__ uint32_t q6_i8(uint32_t q6) {
     return t | ((t & 0x20202020u) * 6u);
 }
 
-template <class C>
+template <class C, bool Y16>
 __global__ __launch_bounds__(C::THREADS) void k_gemm_q6k(const uint8_t* __restrict__ W, const int8_t* __restrict__ xq,
                                                          const float* __restrict__ dyt, float* __restrict__ Y, int m,
                                                          int n, int k, int mp, int epi, int sps,
@@ -365,8 +366,8 @@ __global__ __launch_bounds__(C::THREADS) void k_gemm_q6k(const uint8_t* __restri
                 const int row = m0 + wm * 32 * C::MT + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
                 if (row < m) {
                     if (psum) psum[((int64_t)blockIdx.y * m + row) * n + col] = out[a][b][r];
-                    else if (epi == EPI_STORE) Y[(int64_t)row * n + col] = out[a][b][r];
-                    else store_epi_slow(&Y[(int64_t)row * n + col], out[a][b][r], epi);
+                    else if (epi == EPI_STORE) store_plain<Y16>(Y, (int64_t)row * n + col, out[a][b][r]);
+                    else store_epi_slow<Y16>(Y, (int64_t)row * n + col, out[a][b][r], epi);
                 }
             }
         }
@@ -375,6 +376,7 @@ __global__ __launch_bounds__(C::THREADS) void k_gemm_q6k(const uint8_t* __restri
 // The split-K partial sums, added in split order, then the call's store
 // epilogue; four consecutive outputs a thread (16-byte loads and stores
 // where the four are in range and aligned, one at a time otherwise).
+template <bool Y16>
 __global__ __launch_bounds__(256) void k_q6_sum_splits(const float* __restrict__ psum, int splits, int64_t mn,
                                                        float* __restrict__ Y, int epi) {
     const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
@@ -389,19 +391,23 @@ __global__ __launch_bounds__(256) void k_q6_sum_splits(const float* __restrict__
             v.w += u.w;
         }
         if (epi == EPI_STORE) {
-            *(float4*)(Y + i) = v;
+            if constexpr (Y16)
+                *(uint2*)((uint16_t*)Y + i) = make_uint2(f32_to_f16(v.x) | (uint32_t)f32_to_f16(v.y) << 16,
+                                                         f32_to_f16(v.z) | (uint32_t)f32_to_f16(v.w) << 16);
+            else
+                *(float4*)(Y + i) = v;
         } else {
-            store_epi(&Y[i], v.x, epi);
-            store_epi(&Y[i + 1], v.y, epi);
-            store_epi(&Y[i + 2], v.z, epi);
-            store_epi(&Y[i + 3], v.w, epi);
+            store_epi<Y16>(Y, i, v.x, epi);
+            store_epi<Y16>(Y, i + 1, v.y, epi);
+            store_epi<Y16>(Y, i + 2, v.z, epi);
+            store_epi<Y16>(Y, i + 3, v.w, epi);
         }
         return;
     }
     for (int64_t t = i; t < min(i + 4, mn); t++) {
         float v = psum[t];
         for (int z = 1; z < splits; z++) v += psum[z * mn + t];
-        store_epi(&Y[t], v, epi);
+        store_epi<Y16>(Y, t, v, epi);
     }
 }
 
@@ -517,6 +523,7 @@ __device__ __forceinline__ void q6_planes(const uint8_t* __restrict__ W, int8_t*
 // spread evenly through the grid (workgroup b is activation workgroup
 // floor(b xwg / grid) when that count steps up at b, else a plane one), so
 // the memory-bound and the VALU-bound halves share the CUs.
+template <bool X16>
 __global__ __launch_bounds__(256) void k_q6p_prep(const float* __restrict__ x, int8_t* __restrict__ xq,
                                                   float* __restrict__ dyt, int m, int k, int mp, uint32_t xwg,
                                                   const uint8_t* __restrict__ W, int8_t* __restrict__ planes,
@@ -524,7 +531,7 @@ __global__ __launch_bounds__(256) void k_q6p_prep(const float* __restrict__ x, i
     __shared__ uint32_t raw[4][256];
     const uint64_t b = blockIdx.x, T = gridDim.x;
     const uint32_t xi = (uint32_t)(b * xwg / T);
-    if ((uint32_t)((b + 1) * xwg / T) > xi) q6_prep_x<2, 4>(x, xq, dyt, m, k, mp, xi);  // uniform
+    if ((uint32_t)((b + 1) * xwg / T) > xi) q6_prep_x<2, 4, X16>(x, xq, dyt, m, k, mp, xi);  // uniform
     else q6_planes(W, planes, dwt, n, k, np, (uint32_t)b - xi, raw);
 }
 
@@ -558,6 +565,7 @@ struct Q6P {
 __device__ __forceinline__ int q6p_akey(int row) { return ((row >> 1) ^ (row >> 3)) & 3; }
 __device__ __forceinline__ int q6p_bkey(int col) { return (col & 7) ^ ((col >> 3) & 1); }
 
+template <bool Y16>
 __global__ __launch_bounds__(Q6P::THREADS) void k_gemm_q6p(const int8_t* __restrict__ P, const float* __restrict__ dwt,
                                                           const int8_t* __restrict__ xq,
                                                           const float* __restrict__ dyt, float* __restrict__ Y, int m,
@@ -725,8 +733,8 @@ __global__ __launch_bounds__(Q6P::THREADS) void k_gemm_q6p(const int8_t* __restr
                 const int row = m0 + wm * 64 + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
                 if (row < m) {
                     if (psum) psum[((int64_t)blockIdx.y * m + row) * n + col] = out[a][b][r];
-                    else if (epi == EPI_STORE) Y[(int64_t)row * n + col] = out[a][b][r];
-                    else store_epi_slow(&Y[(int64_t)row * n + col], out[a][b][r], epi);
+                    else if (epi == EPI_STORE) store_plain<Y16>(Y, (int64_t)row * n + col, out[a][b][r]);
+                    else store_epi_slow<Y16>(Y, (int64_t)row * n + col, out[a][b][r], epi);
                 }
             }
         }
@@ -748,15 +756,19 @@ static int64_t q6_tiles(int64_t n, int64_t m) {
 template <class C>
 static hipError_t launch_q6_cfg(const void* w, const Q6Ptrs& p, float* y, int64_t n, int64_t k, int64_t m, int epi,
                                 hipStream_t s, float* psum, int sp) {
-    if (hipError_t e = set_lds_limit((const void*)k_gemm_q6k<C>, C::LDS)) return e;
+    const bool y16 = epi & EPI_Y16;
+    epi = epi_store(epi);
+    const auto kern = y16 ? k_gemm_q6k<C, true> : k_gemm_q6k<C, false>;
+    if (hipError_t e = set_lds_limit((const void*)kern, C::LDS)) return e;
     const int64_t tiles = q6_tiles<C>(n, m), nsb = k / 256;
     const int sps = (int)((nsb + sp - 1) / sp);
-    hipLaunchKernelGGL(k_gemm_q6k<C>, dim3((unsigned)tiles, sp), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq,
-                       p.dyt, y, (int)m, (int)n, (int)k, (int)p.mp, epi, sps, sp > 1 ? psum : nullptr);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, sp), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq, p.dyt,
+                       y, (int)m, (int)n, (int)k, (int)p.mp, epi, sps, sp > 1 ? psum : nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || sp == 1) return e;
     const int64_t mn = m * n;
-    hipLaunchKernelGGL(k_q6_sum_splits, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, psum, sp, mn, y, epi);
+    hipLaunchKernelGGL(y16 ? k_q6_sum_splits<true> : k_q6_sum_splits<false>, dim3((unsigned)((mn + 1023) / 1024)),
+                       dim3(256), 0, s, psum, sp, mn, y, epi);
     return hipGetLastError();
 }
 
@@ -811,18 +823,21 @@ static hipError_t launch_q6p(const void* w, const float* x, float* y, int64_t n,
     const int64_t nsb = k / 256, nb = m * nsb, wb = n * nsb;
     const uint32_t xwg = (uint32_t)((nb + 31) / 32);
     const uint32_t pwg = (uint32_t)((wb + Q6P_PLANE_WG - 1) / Q6P_PLANE_WG);
-    hipLaunchKernelGGL(k_q6p_prep, dim3(xwg + pwg), dim3(256), 0, s, x, p.xq, p.dyt, (int)m, (int)k, (int)p.mp, xwg,
+    hipLaunchKernelGGL((epi & EPI_X16) ? k_q6p_prep<true> : k_q6p_prep<false>, dim3(xwg + pwg), dim3(256), 0, s, x, p.xq, p.dyt, (int)m, (int)k, (int)p.mp, xwg,
                        (const uint8_t*)w, pp.planes, pp.dwt, (int)n, (int)pp.np);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if ((e = set_lds_limit((const void*)k_gemm_q6p, Q6P::LDS))) return e;
+    const bool y16 = epi & EPI_Y16;
+    const auto kern = y16 ? k_gemm_q6p<true> : k_gemm_q6p<false>;
+    if ((e = set_lds_limit((const void*)kern, Q6P::LDS))) return e;
     const int64_t tiles = ((m + Q6P::BM - 1) / Q6P::BM) * ((n + Q6P::BN - 1) / Q6P::BN);
     const int sps = (int)((nsb + sp - 1) / sp);
-    hipLaunchKernelGGL(k_gemm_q6p, dim3((unsigned)tiles, sp), dim3(Q6P::THREADS), Q6P::LDS, s, pp.planes, pp.dwt, p.xq,
-                       p.dyt, y, (int)m, (int)n, (int)k, (int)p.mp, (int)pp.np, epi, sps, sp > 1 ? psum : nullptr);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, sp), dim3(Q6P::THREADS), Q6P::LDS, s, pp.planes, pp.dwt, p.xq,
+                       p.dyt, y, (int)m, (int)n, (int)k, (int)p.mp, (int)pp.np, epi_store(epi), sps, sp > 1 ? psum : nullptr);
     if ((e = hipGetLastError()) != hipSuccess || sp == 1) return e;
     const int64_t mn = m * n;
-    hipLaunchKernelGGL(k_q6_sum_splits, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, psum, sp, mn, y, epi);
+    hipLaunchKernelGGL(y16 ? k_q6_sum_splits<true> : k_q6_sum_splits<false>, dim3((unsigned)((mn + 1023) / 1024)),
+                       dim3(256), 0, s, psum, sp, mn, y, epi_store(epi));
     return hipGetLastError();
 }
 
@@ -874,7 +889,7 @@ hipError_t launch_q6_gemm(const void* w, const float* x, float* y, int64_t n, in
     const int sp = q6_launch_splits(n, k, m);
     if (q6_prep_bytes(m, k) + (sp > 1 ? (size_t)sp * m * n * sizeof(float) : 0) > ws_cap) return hipErrorInvalidValue;
     const Q6Ptrs p = q6_ptrs(qbuf, m, k);
-    hipError_t e = launch_prep_q6(x, p.xq, p.dyt, m, k, p.mp, s);
+    hipError_t e = launch_prep_q6(x, epi & EPI_X16, p.xq, p.dyt, m, k, p.mp, s);
     if (e != hipSuccess) return e;
     float* psum = (float*)((uint8_t*)qbuf + q6_prep_bytes(m, k));
     const int tile = q6_tile_of(m);

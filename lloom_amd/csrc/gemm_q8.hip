@@ -53,6 +53,7 @@ static size_t q8_prep_bytes(int64_t m, int64_t k) {
 }
 
 // One wave a (row, 256 elements): eight blocks of eight lanes.
+template <bool X16>
 __global__ __launch_bounds__(256) void k_gemm_prep_q8_0(const float* __restrict__ x, int8_t* __restrict__ xq,
                                                         float* __restrict__ dxt, int m, int k, int mp) {
     const int lane = threadIdx.x & 63;
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256) void k_gemm_prep_q8_0(const float* __restrict_
     if (c >= (int64_t)m * nc) return;
     const int mi = (int)(c / nc), cc = (int)(c - (int64_t)mi * nc);
     const int64_t off = (int64_t)mi * k + 256 * cc + 4 * lane;
-    const float4 v = *(const float4*)(x + off);
+    const float4 v = load_x4<X16>(x, off);
     uint16_t d16;
     const uint32_t q = q8_0_block_8lanes(v, &d16);
     *(uint32_t*)(xq + off) = q;
@@ -127,7 +128,7 @@ __device__ __forceinline__ void vm_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <class C>
+template <class C, bool Y16>
 __global__ __launch_bounds__(C::THREADS) void k_gemm_q8_0(const uint8_t* __restrict__ W,
                                                             const int8_t* __restrict__ xq,
                                                             const float* __restrict__ dxt, float* __restrict__ Y,
@@ -285,8 +286,8 @@ __global__ __launch_bounds__(C::THREADS) void k_gemm_q8_0(const uint8_t* __restr
                 const int row = m0 + wm * 32 * C::MT + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
                 const float v = 0.5f * out[a][b][r];
                 if (row < m) {
-                    if (epi == EPI_STORE) Y[(int64_t)row * n + col] = v;
-                    else store_epi_slow(&Y[(int64_t)row * n + col], v, epi);
+                    if (epi == EPI_STORE) store_plain<Y16>(Y, (int64_t)row * n + col, v);
+                    else store_epi_slow<Y16>(Y, (int64_t)row * n + col, v, epi);
                 }
             }
         }
@@ -316,7 +317,7 @@ struct Q8KCfg {
     static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-template <class C>
+template <class C, bool Y16>
 __global__ __launch_bounds__(C::THREADS) void k_gemm_q8_0_splitk(const uint8_t* __restrict__ W,
                                                                    const int8_t* __restrict__ xq,
                                                                    const float* __restrict__ dxt,
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(C::THREADS) void k_gemm_q8_0_splitk(const uint8_t* 
 #pragma unroll
             for (int w = 0; w < C::KS; w++) v += red[(((w * C::MT + a) * C::NT + b) * 16 + r) * 64 + lane];
             const int row = m0 + a * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (row < m && col < n) store_epi(&Y[(int64_t)row * n + col], v, epi);
+            if (row < m && col < n) store_epi<Y16>(Y, (int64_t)row * n + col, v, epi);
         }
     }
 }
@@ -471,10 +472,11 @@ __global__ __launch_bounds__(C::THREADS) void k_gemm_q8_0_splitk(const uint8_t* 
 template <class C>
 static hipError_t launch_q8k_cfg(const void* w, const Q8Ptrs& p, float* y, int64_t n, int64_t k, int64_t m, int epi,
                                  hipStream_t s) {
-    if (hipError_t e = set_lds_limit((const void*)k_gemm_q8_0_splitk<C>, C::LDS)) return e;
+    const auto kern = (epi & EPI_Y16) ? k_gemm_q8_0_splitk<C, true> : k_gemm_q8_0_splitk<C, false>;
+    if (hipError_t e = set_lds_limit((const void*)kern, C::LDS)) return e;
     const dim3 grid((unsigned)((n + C::BN - 1) / C::BN), (unsigned)((m + C::BM - 1) / C::BM));
-    hipLaunchKernelGGL(k_gemm_q8_0_splitk<C>, grid, dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq, p.dxt, y,
-                       (int)m, (int)n, (int)k, (int)p.mp, epi);
+    hipLaunchKernelGGL(kern, grid, dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq, p.dxt, y,
+                       (int)m, (int)n, (int)k, (int)p.mp, epi_store(epi));
     return hipGetLastError();
 }
 
@@ -486,10 +488,11 @@ bool q8_gemm_fits(int64_t n, int64_t k, int64_t m) {
 template <class C>
 static hipError_t launch_q8_cfg(const void* w, const Q8Ptrs& p, float* y, int64_t n, int64_t k, int64_t m, int epi,
                                 hipStream_t s) {
-    if (hipError_t e = set_lds_limit((const void*)k_gemm_q8_0<C>, C::LDS)) return e;
+    const auto kern = (epi & EPI_Y16) ? k_gemm_q8_0<C, true> : k_gemm_q8_0<C, false>;
+    if (hipError_t e = set_lds_limit((const void*)kern, C::LDS)) return e;
     const unsigned grid = (unsigned)(((m + C::BM - 1) / C::BM) * ((n + C::BN - 1) / C::BN));
-    hipLaunchKernelGGL(k_gemm_q8_0<C>, dim3(grid), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq, p.dxt, y,
-                       (int)m, (int)n, (int)k, (int)p.mp, epi);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(C::THREADS), C::LDS, s, (const uint8_t*)w, p.xq, p.dxt, y,
+                       (int)m, (int)n, (int)k, (int)p.mp, epi_store(epi));
     return hipGetLastError();
 }
 
@@ -510,7 +513,7 @@ hipError_t launch_q8_gemm(const void* w, const float* x, float* y, int64_t n, in
     if (q8_prep_bytes(m, k) > ws_cap) return hipErrorInvalidValue;
     const Q8Ptrs p = q8_ptrs(qbuf, m, k);
     const int64_t nc = m * (k / 256);
-    hipLaunchKernelGGL(k_gemm_prep_q8_0, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, x, p.xq, p.dxt, (int)m,
+    hipLaunchKernelGGL((epi & EPI_X16) ? k_gemm_prep_q8_0<true> : k_gemm_prep_q8_0<false>, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, x, p.xq, p.dxt, (int)m,
                        (int)k, (int)p.mp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

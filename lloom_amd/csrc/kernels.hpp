@@ -26,12 +26,18 @@ hipError_t launch_embedding(int type, const void* w, int64_t rows, int64_t hidde
 size_t split_q8k_bytes(int64_t k, int64_t m);
 void split_q8k_ptrs(void* base, int64_t k, int64_t m, int8_t** qs, float** d, int8_t** bsp = nullptr);
 hipError_t launch_quantize_split_q8k(const float* x, int64_t m, int64_t k, int8_t* qs, float* d, hipStream_t s,
-                                     int8_t* bsp = nullptr, bool tiled = false);
+                                     int8_t* bsp = nullptr, bool tiled = false, bool x16 = false);
 
 // matvec.hip: m <= 16.  Rows up to MV_DOT_MAX_ROWS (Q4_K on a weight of at
 // most 2048^2 elements: up to 4) take the fused dot4 kernel; more rows take
 // the MFMA kernels on a workspace of matvec_workspace_bytes.
+// `epi` holds the store epilogue and EPI_X16 / EPI_Y16 (kq_common.hpp): an F16
+// x or y only where *_reads_f16 or gemm_writes_f16 says the call's kernels
+// take one.
 constexpr int MV_DOT_MAX_ROWS = 2;
+bool matvec_reads_f16(int type, int64_t n, int64_t k, int64_t m);
+bool gemm_reads_f16(int type, int64_t n, int64_t k, int64_t m);
+bool gemm_writes_f16(int type, int64_t n, int64_t k, int64_t m, int mode);
 size_t matvec_workspace_bytes(int type, int64_t n, int64_t k, int64_t m);
 hipError_t launch_matvec(int type, const void* w, const float* x, float* y, int64_t n, int64_t k, int64_t m,
                          void* ws, int epi, hipStream_t s);

@@ -198,23 +198,55 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += partner16(v);
     return v + partner32(v);
 }
-// Full-wave max (NaN-ignoring, as fmaxf), the result in every lane.
 // The quantized matmul's store epilogues (QMatMul::forward_silu /
 // forward_mul_into, mod.rs:2102-2156; the Metal store types of
 // kernels/metal_src/quantized_store.metal): the plain store, silu(v) =
 // v / (1 + exp(-v)), and y = y * v into the buffer's own value (the SwiGLU's
 // up projection multiplied into silu(gate)).
-constexpr int EPI_STORE = 0, EPI_SILU = 1, EPI_MUL_INTO = 2;
-__device__ __forceinline__ void store_epi(float* p, float v, int epi) {
-    if (epi == EPI_SILU) v = v / (1.0f + expf(-v));
-    else if (epi == EPI_MUL_INTO) v = *p * v;
-    *p = v;
+// On the host `epi` also says whether x and y are F16 (their float pointers
+// then point at halves): x is widened where it is loaded and y rounded (RNE)
+// where it is stored, by kernels built for it (X16, Y16), so an F16 prompt
+// has no conversion launches ([509, 2048] through gate, up and down: 7 of
+// them, 29 of 168 us).  A run-time flag in the kernels instead cost the F32
+// calls 1 to 2 %.
+constexpr int EPI_STORE = 0, EPI_SILU = 1, EPI_MUL_INTO = 2, EPI_Y16 = 4, EPI_X16 = 8;
+// What a kernel's store takes.
+constexpr int epi_store(int epi) { return epi & 3; }
+template <bool Y16 = false>
+__device__ __forceinline__ void store_epi(float* y, int64_t i, float v, int epi) {
+    if constexpr (Y16) {
+        uint16_t* p = (uint16_t*)y + i;
+        if (epi == EPI_SILU) v = v / (1.0f + expf(-v));
+        else if (epi == EPI_MUL_INTO) v = f16_to_f32(*p) * v;
+        *p = f32_to_f16(v);
+    } else {
+        float* p = y + i;
+        if (epi == EPI_SILU) v = v / (1.0f + expf(-v));
+        else if (epi == EPI_MUL_INTO) v = *p * v;
+        *p = v;
+    }
 }
 // The same, out of line: for kernels that store many values per lane, so
 // the SiLU's code is not unrolled into every store.
-__device__ __noinline__ void store_epi_slow(float* p, float v, int epi);
-__device__ __noinline__ inline void store_epi_slow(float* p, float v, int epi) { store_epi(p, v, epi); }
+template <bool Y16 = false>
+__device__ __noinline__ void store_epi_slow(float* y, int64_t i, float v, int epi) {
+    store_epi<Y16>(y, i, v, epi);
+}
+// A plain store of y's type.
+template <bool Y16>
+__device__ __forceinline__ void store_plain(float* y, int64_t i, float v) {
+    if constexpr (Y16) ((uint16_t*)y)[i] = f32_to_f16(v);
+    else y[i] = v;
+}
+// Four elements of x from element i (a multiple of 4).
+template <bool X16>
+__device__ __forceinline__ float4 load_x4(const float* __restrict__ x, int64_t i) {
+    if constexpr (!X16) return *(const float4*)(x + i);
+    const uint2 h = *(const uint2*)((const uint16_t*)x + i);
+    return make_float4(f16_to_f32(h.x & 0xffffu), f16_to_f32(h.x >> 16), f16_to_f32(h.y & 0xffffu), f16_to_f32(h.y >> 16));
+}
 
+// Full-wave max (NaN-ignoring, as fmaxf), the result in every lane.
 __device__ __forceinline__ float wave_max(float v) {
     v = __builtin_fmaxf(v, dpp<DPP_XOR1>(v));
     v = __builtin_fmaxf(v, dpp<DPP_XOR2>(v));

@@ -137,11 +137,12 @@ __device__ __forceinline__ uint32_t q8_0_block_8lanes(float4 x, uint16_t* d16) {
 // so a 16-row tile's operand pieces are 1 KB each), d into dt[sb][mp], and,
 // with bsp, the eight 32-element sums as int8 (sum & 63, sum >> 6) into
 // bsp[sb][mp][16].
+template <bool X16>
 __device__ __forceinline__ void q8k_split_block(const float* __restrict__ x, int8_t* __restrict__ qs,
                                                 float* __restrict__ dt, int8_t* __restrict__ bsp, int k, int mp,
                                                 int tiled, int mi, int sb, int lane) {
     const int nsb = k >> 8;
-    const float4 v = *(const float4*)(x + (int64_t)mi * k + sb * 256 + 4 * lane);
+    const float4 v = load_x4<X16>(x, (int64_t)mi * k + sb * 256 + 4 * lane);
     float d;
     int bs;
     const uint32_t q = q8k_block_wave(v, &d, &bs);

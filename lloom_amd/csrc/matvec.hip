@@ -345,7 +345,7 @@ __global__ __launch_bounds__(64 * WV) void k_matvec(const uint8_t* __restrict__ 
         const float tot = wave_sum_items<R * MB>(v);
         const int item = wave_sum_item_of_lane();
         const int r = item / MB, mi = item % MB;
-        if ((lane & 7) == 0 && item < R * MB && mi < m && row0 + r < n) store_epi(&Y[(int64_t)mi * n + row0 + r], tot, epi);
+        if ((lane & 7) == 0 && item < R * MB && mi < m && row0 + r < n) store_epi(Y, (int64_t)mi * n + row0 + r, tot, epi);
     } else {
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(64 * WV) void k_matvec(const uint8_t* __restrict__ 
             for (int mi = 0; mi < MB; mi++) {
                 if (mi < m) {
                     const float v = wave_sum(acc[r][mi]);
-                    if (lane == 0 && row < n) store_epi(&Y[(int64_t)mi * n + row], v, epi);
+                    if (lane == 0 && row < n) store_epi(Y, (int64_t)mi * n + row, v, epi);
                 }
             }
         }
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(64 * KS) void k_mv_mfma(const uint8_t* __restrict__
                     const int mi = 16 * (mt0 + u) + 4 * g + v;
                     if (mi < m) {
                         if (psum) psum[((int64_t)blockIdx.z * m + mi) * n + nrow] = out[t][u][v];
-                        else store_epi(&Y[(int64_t)mi * n + nrow], out[t][u][v], epi);
+                        else store_epi(Y, (int64_t)mi * n + nrow, out[t][u][v], epi);
                     }
                 }
         }
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(128 * KS) void k_mv_fused(const uint8_t* __restrict
     if (row < n) {
 #pragma unroll
         for (int u = 0; u < 4; u++)
-            if (4 * g + u < m) store_epi(&Y[(int64_t)(4 * g + u) * n + row], out[u], epi);
+            if (4 * g + u < m) store_epi(Y, (int64_t)(4 * g + u) * n + row, out[u], epi);
     }
 }
 
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(256) void k_sum_splits(const float* __restrict__ ps
     if (i >= mn) return;
     float v = psum[i];
     for (int z = 1; z < splits; z++) v += psum[z * mn + i];
-    store_epi(&Y[i], v, epi);
+    store_epi(Y, i, v, epi);
 }
 
 // ------------------- 3..128 rows, K <= 2048: weight DMAs, tiled activations --
@@ -895,7 +895,7 @@ __global__ __launch_bounds__(64 * NSB) void k_mv_dma_ma(const uint8_t* __restric
         if (row < n) {
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                if (16 * a + 4 * g + v < m) store_epi(&Y[(int64_t)(16 * a + 4 * g + v) * n + row], o[v], epi);
+                if (16 * a + 4 * g + v < m) store_epi(Y, (int64_t)(16 * a + 4 * g + v) * n + row, o[v], epi);
         }
     }
 }
@@ -954,14 +954,14 @@ hipError_t launch_mv_dma_ma(int type, const void* w, const float* x, float* y, i
     float* xd;
     int8_t* bsp;
     split_q8k_ptrs(ws, k, m, &xt, &xd, &bsp);
-    hipError_t e = launch_quantize_split_q8k(x, m, k, xt, xd, s, type == T_Q4K ? bsp : nullptr, true);
+    hipError_t e = launch_quantize_split_q8k(x, m, k, xt, xd, s, type == T_Q4K ? bsp : nullptr, true, epi & EPI_X16);
     if (e != hipSuccess) return e;
-    if (m <= 16) return launch_mv_dma_ma_m<1>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
-    if (m <= 32) return launch_mv_dma_ma_m<2>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
-    if (m <= 48) return launch_mv_dma_ma_m<3>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
-    if (m <= 64) return launch_mv_dma_ma_m<4>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
-    if (m <= 96) return launch_mv_dma_ma_m<6>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
-    return launch_mv_dma_ma_m<8>(type, w, y, n, k, m, xt, xd, bsp, epi, s);
+    if (m <= 16) return launch_mv_dma_ma_m<1>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
+    if (m <= 32) return launch_mv_dma_ma_m<2>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
+    if (m <= 48) return launch_mv_dma_ma_m<3>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
+    if (m <= 64) return launch_mv_dma_ma_m<4>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
+    if (m <= 96) return launch_mv_dma_ma_m<6>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
+    return launch_mv_dma_ma_m<8>(type, w, y, n, k, m, xt, xd, bsp, epi_store(epi), s);
 }
 
 template <int TYPE, int MA>
@@ -1007,10 +1007,10 @@ hipError_t launch_mq(int type, const void* w, const float* x, float* y, int64_t 
     int8_t* xq;
     float* xd;
     split_q8k_ptrs(ws, k, m, &xq, &xd);
-    hipError_t e = launch_quantize_split_q8k(x, m, k, xq, xd, s);
+    hipError_t e = launch_quantize_split_q8k(x, m, k, xq, xd, s, nullptr, false, epi & EPI_X16);
     if (e != hipSuccess) return e;
-    return type == T_Q4K ? launch_mv_mfma<T_Q4K, 4>(w, y, n, k, m, xq, xd, epi, s)
-                         : launch_mv_mfma<T_Q6K, 4>(w, y, n, k, m, xq, xd, epi, s);
+    return type == T_Q4K ? launch_mv_mfma<T_Q4K, 4>(w, y, n, k, m, xq, xd, epi_store(epi), s)
+                         : launch_mv_mfma<T_Q6K, 4>(w, y, n, k, m, xq, xd, epi_store(epi), s);
 }
 
 // Rows of Q4_K / Q6_K on the dot4 kernel: one or two, and Q4_K with 3-4
@@ -1019,6 +1019,12 @@ hipError_t launch_mq(int type, const void* w, const float* x, float* y, int64_t 
 // 6.49, and Q6_K [2048, 8192] 15.8 against 12.0).
 static bool mv_dot(int type, int64_t n, int64_t k, int64_t m) {
     return m <= MV_DOT_MAX_ROWS || (type == T_Q4K && m <= 4 && n * k <= 2048 * 2048);
+}
+
+// Past the dot4 and fused kernels (which quantize x themselves, from f32).
+bool matvec_reads_f16(int type, int64_t n, int64_t k, int64_t m) {
+    if (mv_stream_fits(type, n, k, m)) return true;
+    return type != T_Q8_0 && !mv_dot(type, n, k, m) && !(m <= FUSED_MAX_ROWS && (k == 2048 || k == 1024));
 }
 
 hipError_t launch_matvec(int type, const void* w, const float* x, float* y, int64_t n, int64_t k, int64_t m,
@@ -1039,11 +1045,11 @@ hipError_t launch_matvec(int type, const void* w, const float* x, float* y, int6
         int8_t* xq;
         float* xd;
         split_q8k_ptrs(ws, k, m, &xq, &xd);
-        hipError_t e = launch_quantize_split_q8k(x, m, k, xq, xd, s);
+        hipError_t e = launch_quantize_split_q8k(x, m, k, xq, xd, s, nullptr, false, epi & EPI_X16);
         if (e != hipSuccess) return e;
         float* ps = mv_psum(ws, k, m);
-        return type == T_Q4K ? launch_mv_mfma<T_Q4K, 1>(w, y, n, k, m, xq, xd, epi, s, ps)
-                             : launch_mv_mfma<T_Q6K, 1>(w, y, n, k, m, xq, xd, epi, s, ps);
+        return type == T_Q4K ? launch_mv_mfma<T_Q4K, 1>(w, y, n, k, m, xq, xd, epi_store(epi), s, ps)
+                             : launch_mv_mfma<T_Q6K, 1>(w, y, n, k, m, xq, xd, epi_store(epi), s, ps);
     }
     switch (type) {
         case T_Q4K: return launch_type<T_Q4K>(w, x, y, (int)n, (int)k, (int)m, epi, s);

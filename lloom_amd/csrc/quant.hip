@@ -46,13 +46,14 @@ __global__ __launch_bounds__(256) void k_quantize_q8k(const float* __restrict__ 
 // (the permuted offsets 64g .. 64g+63) split into four 16-byte pieces i,
 // piece i at [i][16g + r % 16]: the MFMA lane 16g + r % 16 then loads its
 // operand piece i of a row group's superblock from 1 KB of contiguous bytes.
+template <bool X16>
 __global__ __launch_bounds__(256) void k_quantize_split_q8k(const float* __restrict__ x, int8_t* __restrict__ qs,
                                                             float* __restrict__ dt, int8_t* __restrict__ bsp, int m,
                                                             int k, int mp, int tiled) {
     const int nsb = k >> 8;
     const int sb = blockIdx.y * 4 + (threadIdx.x >> 6), mi = blockIdx.x;
     if (sb >= nsb) return;
-    q8k_split_block(x, qs, dt, bsp, k, mp, tiled, mi, sb, threadIdx.x & 63);
+    q8k_split_block<X16>(x, qs, dt, bsp, k, mp, tiled, mi, sb, threadIdx.x & 63);
 }
 
 static int64_t pad16(int64_t m) { return (m + 15) & ~(int64_t)15; }
@@ -70,10 +71,10 @@ void split_q8k_ptrs(void* base, int64_t k, int64_t m, int8_t** qs, float** d, in
 }
 
 hipError_t launch_quantize_split_q8k(const float* x, int64_t m, int64_t k, int8_t* qs, float* d, hipStream_t s,
-                                     int8_t* bsp, bool tiled) {
+                                     int8_t* bsp, bool tiled, bool x16) {
     const int64_t nsb = k / 256;
-    hipLaunchKernelGGL(k_quantize_split_q8k, dim3((unsigned)m, (unsigned)((nsb + 3) / 4)), dim3(256), 0, s, x, qs, d,
-                       bsp, (int)m, (int)k, (int)pad16(m), tiled ? 1 : 0);
+    hipLaunchKernelGGL(x16 ? k_quantize_split_q8k<true> : k_quantize_split_q8k<false>,
+                       dim3((unsigned)m, (unsigned)((nsb + 3) / 4)), dim3(256), 0, s, x, qs, d, bsp, (int)m, (int)k, (int)pad16(m), tiled ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -235,7 +235,7 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_mv_stream(const uint8_t* __re
             if (row >= 16 * t) {
 #pragma unroll
                 for (int v = 0; v < 4; v++)
-                    if (4 * g + v < m) store_epi(&Y[(int64_t)(4 * g + v) * n + row], o[v], epi);
+                    if (4 * g + v < m) store_epi(Y, (int64_t)(4 * g + v) * n + row, o[v], epi);
             }
         }
     }
@@ -306,13 +306,13 @@ hipError_t launch_mv_stream(int type, const void* w, const float* x, float* y, i
     float* xd;
     int8_t* bsp;
     split_q8k_ptrs(ws, k, m, &xt, &xd, &bsp);
-    hipError_t e = launch_quantize_split_q8k(x, m, k, xt, xd, s, bsp, true);
+    hipError_t e = launch_quantize_split_q8k(x, m, k, xt, xd, s, bsp, true, epi & EPI_X16);
     if (e != hipSuccess) return e;
     switch (k / 2048) {
-        case 1: return launch_stream_s<1>(w, y, n, m, xt, xd, bsp, epi, s);
-        case 2: return launch_stream_s<2>(w, y, n, m, xt, xd, bsp, epi, s);
-        case 3: return launch_stream_s<3>(w, y, n, m, xt, xd, bsp, epi, s);
-        default: return launch_stream_s<4>(w, y, n, m, xt, xd, bsp, epi, s);
+        case 1: return launch_stream_s<1>(w, y, n, m, xt, xd, bsp, epi_store(epi), s);
+        case 2: return launch_stream_s<2>(w, y, n, m, xt, xd, bsp, epi_store(epi), s);
+        case 3: return launch_stream_s<3>(w, y, n, m, xt, xd, bsp, epi_store(epi), s);
+        default: return launch_stream_s<4>(w, y, n, m, xt, xd, bsp, epi_store(epi), s);
     }
 }
 
