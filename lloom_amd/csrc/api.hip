@@ -117,6 +117,12 @@ int lloom_hip_ctx_create(int device, lloom_hip_ctx** out) {
         delete c;
         return fail(LLOOM_HIP_ENOMEM, "ctx_create: flag allocation failed");
     }
+    if (hipHostMalloc((void**)&c->call_flag, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipFree(c->flags);
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return fail(LLOOM_HIP_ENOMEM, "ctx_create: host flag allocation failed");
+    }
     (void)hipMemset(c->flags, 0, 256);
     (void)hipDeviceSynchronize();
     *out = c;
@@ -130,6 +136,7 @@ int lloom_hip_ctx_destroy(lloom_hip_ctx* ctx) {
     if (ctx->ws) (void)hipFree(ctx->ws);
     for (void* p : ctx->retired) (void)hipFree(p);
     if (ctx->flags) (void)hipFree(ctx->flags);
+    if (ctx->call_flag) (void)hipHostFree(ctx->call_flag);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return LLOOM_HIP_OK;
@@ -412,6 +419,26 @@ int lloom_hip_cast(lloom_hip_ctx* ctx, const void* src_dev, int src_dtype, void*
 
 }  // extern "C"
 
+// The flags of a call that holds the context's lock.  A strict call's host
+// flag is cleared here: the one before it waited for its kernels.
+static IdFlags id_flags(lloom_hip_ctx* ctx, int strict) {
+    if (!strict) return {ctx->flags + 1, ctx->flags};
+    *(volatile int*)ctx->call_flag = 0;
+    return {ctx->call_flag, ctx->flags};
+}
+
+// Waits for a strict call's stream; *bad if its kernels saw an id out of
+// range, which the sticky flag then forgets (this call reports it).
+static int strict_bad(lloom_hip_ctx* ctx, hipStream_t s, bool* bad) {
+    HIP_OK(hipStreamSynchronize(s));
+    *bad = *(volatile int*)ctx->call_flag != 0;
+    if (*bad) {
+        int zero = 0;
+        HIP_OK(hipMemcpy(ctx->flags, &zero, sizeof(int), hipMemcpyHostToDevice));
+    }
+    return LLOOM_HIP_OK;
+}
+
 static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const void* w2_dev, int64_t n_experts,
                     int64_t n, int64_t k, const float* x_dev, int64_t batch, int64_t in_dim1,
                     const uint32_t* ids_dev, int64_t topk, float* y_dev, float* y2_dev, int mode, int strict,
@@ -449,16 +476,11 @@ static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const 
     if (rc) rc = ensure_ws(ctx, moe_workspace_bytes(n_experts, batch * topk, n, k, mode), s, &ws);
     if (rc) return rc;
     HIP_OK(launch_moe(ggml_type, w_dev, n_experts, n, k, x_dev, batch, in_dim1, ids_dev, topk, y_dev, (int*)ws,
-                      ctx->ws_bytes, ctx->flags, mode, w2_dev, y2_dev, s));
+                      ctx->ws_bytes, id_flags(ctx, strict), mode, w2_dev, y2_dev, s));
     if (strict) {
-        int flag = 0;
-        HIP_OK(hipMemcpyAsync(&flag, ws, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIP_OK(hipStreamSynchronize(s));
-        if (flag) {
-            int zero = 0;
-            HIP_OK(hipMemcpy(ctx->flags, &zero, sizeof(int), hipMemcpyHostToDevice));
-            return fail(LLOOM_HIP_EEXPERT, "expert id is out of range for %lld experts", (long long)n_experts);
-        }
+        bool bad = false;
+        if (int rc = strict_bad(ctx, s, &bad)) return rc;
+        if (bad) return fail(LLOOM_HIP_EEXPERT, "expert id is out of range for %lld experts", (long long)n_experts);
     }
     return LLOOM_HIP_OK;
 }
@@ -505,17 +527,11 @@ int lloom_hip_embedding(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, in
     HIP_OK(hipSetDevice(ctx->device));
     hipStream_t s = pick_stream(ctx, stream);
     std::lock_guard<std::mutex> lock(ctx->mu);
-    if (strict) HIP_OK(hipMemsetAsync(ctx->flags + 1, 0, sizeof(int), s));
-    HIP_OK(launch_embedding(ggml_type, w_dev, rows, hidden, ids_dev, n_ids, y_dev, out_dtype, ctx->flags, s));
+    HIP_OK(launch_embedding(ggml_type, w_dev, rows, hidden, ids_dev, n_ids, y_dev, out_dtype, id_flags(ctx, strict), s));
     if (strict) {
-        int flag = 0;
-        HIP_OK(hipMemcpyAsync(&flag, ctx->flags + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIP_OK(hipStreamSynchronize(s));
-        if (flag) {
-            int zero = 0;
-            HIP_OK(hipMemcpy(ctx->flags, &zero, sizeof(int), hipMemcpyHostToDevice));
-            return fail(LLOOM_HIP_EEXPERT, "embedding id is out of range for %lld rows", (long long)rows);
-        }
+        bool bad = false;
+        if (int rc = strict_bad(ctx, s, &bad)) return rc;
+        if (bad) return fail(LLOOM_HIP_EEXPERT, "embedding id is out of range for %lld rows", (long long)rows);
     }
     return LLOOM_HIP_OK;
 }

@@ -7,6 +7,13 @@
 
 namespace lloom {
 
+// Where a kernel reports an out-of-range id: `call` gets 0 or 1 (a strict
+// call's is host memory, read once its stream has drained), `sticky` 1, until
+// the next lloom_hip_ctx_sync.
+struct IdFlags {
+    int *call, *sticky;
+};
+
 // quant.hip
 hipError_t launch_quantize_act(int vec_dot_type, const float* x, void* out, int64_t elems, hipStream_t s);
 hipError_t launch_quantize_weights(int type, const float* x, void* out, int64_t elems, hipStream_t s);
@@ -15,9 +22,9 @@ hipError_t launch_dequantize(int type, const void* w, void* y, int out_dtype, in
 // src and dst 16-byte aligned.
 hipError_t launch_cast(int src_t, const void* src, int dst_t, void* dst, int64_t count, hipStream_t s);
 // Rows ids[0 .. n_ids) of an [rows, hidden] weight, dequantized; a bad id
-// gives a zero row and sets flag[0] and flag[1].
+// gives a zero row and sets both flags (flags.call only ever to 1).
 hipError_t launch_embedding(int type, const void* w, int64_t rows, int64_t hidden, const uint32_t* ids, int64_t n_ids,
-                            void* y, int out_dtype, int* flag, hipStream_t s);
+                            void* y, int out_dtype, IdFlags flags, hipStream_t s);
 
 // quant.hip: Q8_K activations in the split layout the MFMA kernels read:
 // qs int8 [m][k] then d f32 [k/256][mp] (m padded to mp, a multiple of 16),
@@ -131,13 +138,13 @@ struct MoeGemmCall {
     const uint32_t* ids;
     float *y, *y2;
     void* ws;
-    int* sticky;
+    IdFlags flags;
 };
 bool moe_gemm_fits(int type, int64_t n_experts, int64_t planes, int64_t rows, int64_t n, int64_t k);
 size_t moe_gemm_workspace_bytes(int64_t n_experts, int64_t planes, int64_t rows, int64_t k);
 hipError_t launch_moe_gemm(const MoeGemmCall& c, hipStream_t s);
 hipError_t launch_moe(int type, const void* w, int64_t n_experts, int64_t n, int64_t k, const float* x,
                       int64_t batch, int64_t in_dim1, const uint32_t* ids, int64_t topk, float* y, int* ws,
-                      size_t ws_cap, int* sticky, int mode, const void* w2, float* y2, hipStream_t s);
+                      size_t ws_cap, IdFlags flags, int mode, const void* w2, float* y2, hipStream_t s);
 
 }  // namespace lloom

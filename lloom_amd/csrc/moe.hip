@@ -28,7 +28,7 @@ namespace lloom {
 
 #pragma clang fp contract(off)
 
-// Workspace (ints): [0] error flag, [1] active experts,
+// Workspace (ints): [1] active experts,
 // [2 .. 2+E) count, [2+E .. 2+2E) start, [2+2E .. 2+3E) active list,
 // [2+3E .. 2+3E+P) planes sorted by expert, [.. +E) fill cursor.
 size_t moe_workspace_ints(int64_t n_experts, int64_t planes) { return 2 + 4 * (size_t)n_experts + (size_t)planes; }
@@ -38,7 +38,7 @@ size_t moe_workspace_ints(int64_t n_experts, int64_t planes) { return 2 + 4 * (s
 // follows the LDS atomics, but every plane's dot is computed on its own, so
 // no result depends on it.
 __global__ __launch_bounds__(1024) void k_moe_route(const uint32_t* __restrict__ ids, int planes, int E, int* ws,
-                                                    int* sticky, float* __restrict__ y, float* __restrict__ y2, int n) {
+                                                    IdFlags flags, float* __restrict__ y, float* __restrict__ y2, int n) {
     extern __shared__ int s_mem[];  // [E] counts, then [E] cursors
     __shared__ int s_part[1024];
     __shared__ int s_bad, s_active;
@@ -108,8 +108,8 @@ __global__ __launch_bounds__(1024) void k_moe_route(const uint32_t* __restrict__
         if (e < (uint32_t)E) sorted[atomicAdd(&s_cur[e], 1)] = p;
     }
     if (tid == 0) {
-        ws[0] = s_bad;             // this call: read back by a strict call
-        if (s_bad) sticky[0] = 1;  // until the next lloom_hip_ctx_sync
+        flags.call[0] = s_bad;             // this call: read back by a strict call
+        if (s_bad) flags.sticky[0] = 1;  // until the next lloom_hip_ctx_sync
         ws[1] = s_active;
     }
 }
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void k_moe_lds(const uint8_t* __restrict__ W, 
                                                  float* __restrict__ Y, int* ws, int E, int n, int K, int in_dim1,
                                                  int topk, int pgmax, const uint8_t* __restrict__ W2,
                                                  float* __restrict__ Y2, const uint32_t* __restrict__ ids,
-                                                 int planes, int* sticky, int route) {
+                                                 int planes, IdFlags flags, int route) {
     using Tr = MvTraits<TYPE>;
     constexpr int NR = MoeRuns<TYPE>::N;
     constexpr int RR = GLU ? 2 * R : R;  // weight rows a lane holds
@@ -430,8 +430,8 @@ __global__ __launch_bounds__(256) void k_moe_lds(const uint8_t* __restrict__ W, 
             }
             bad = __syncthreads_or(bad);
             if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.z == 0) {
-                ws[0] = bad;  // this call: read back by a strict call
-                if (bad) sticky[0] = 1;
+                flags.call[0] = bad;  // this call: read back by a strict call
+                if (bad) flags.sticky[0] = 1;
             }
             return;
         }
@@ -674,7 +674,7 @@ struct MoedCfg {
 template <int NSB, bool GLU>
 __global__ __launch_bounds__(64 * NSB) void k_moe_dma(const uint8_t* __restrict__ W, const float* __restrict__ X,
                                                       float* __restrict__ Y, const uint32_t* __restrict__ ids,
-                                                      int planes, int* ws, int* sticky, int E, int n, int in_dim1,
+                                                      int planes, int* ws, IdFlags flags, int E, int n, int in_dim1,
                                                       int topk, const uint8_t* __restrict__ W2,
                                                       float* __restrict__ Y2, int tpw) {
     using C = MoedCfg<NSB>;
@@ -705,8 +705,8 @@ __global__ __launch_bounds__(64 * NSB) void k_moe_dma(const uint8_t* __restrict_
         }
         bad = __syncthreads_or(bad);
         if (tid == 0 && blockIdx.x == 0 && blockIdx.z == 0) {
-            ws[0] = bad;  // this call: read back by a strict call
-            if (bad) sticky[0] = 1;
+            flags.call[0] = bad;  // this call: read back by a strict call
+            if (bad) flags.sticky[0] = 1;
         }
         return;
     }
@@ -960,7 +960,7 @@ __global__ __launch_bounds__(64 * NSB) void k_moe_dma(const uint8_t* __restrict_
 
 template <int NSB>
 static hipError_t moe_dma_nsb(const void* w, const float* x, float* y, const uint32_t* ids, int planes, int* ws,
-                              int* sticky, int E, int n, int in_dim1, int topk, const void* w2, float* y2, int mode,
+                              IdFlags flags, int E, int n, int in_dim1, int topk, const void* w2, float* y2, int mode,
                               hipStream_t s) {
     using C = MoedCfg<NSB>;
     const bool glu = mode == MOE_GLU;
@@ -978,10 +978,10 @@ static hipError_t moe_dma_nsb(const void* w, const float* x, float* y, const uin
     if (hipError_t e = set_lds_limit(kern, C::LDS)) return e;
     if (glu)
         hipLaunchKernelGGL((k_moe_dma<NSB, true>), grid, dim3(64 * NSB), C::LDS, s, (const uint8_t*)w, x, y, ids,
-                           planes, ws, sticky, E, n, in_dim1, topk, (const uint8_t*)w2, y2, tpw);
+                           planes, ws, flags, E, n, in_dim1, topk, (const uint8_t*)w2, y2, tpw);
     else
         hipLaunchKernelGGL((k_moe_dma<NSB, false>), grid, dim3(64 * NSB), C::LDS, s, (const uint8_t*)w, x, y, ids,
-                           planes, ws, sticky, E, n, in_dim1, topk, (const uint8_t*)w2, y2, tpw);
+                           planes, ws, flags, E, n, in_dim1, topk, (const uint8_t*)w2, y2, tpw);
     return hipGetLastError();
 }
 
@@ -1014,10 +1014,10 @@ static bool moe_dma_fits(int type, int64_t n, int64_t k, int64_t E, int planes) 
 }
 
 static hipError_t launch_moe_dma(const void* w, const float* x, float* y, const uint32_t* ids, int planes, int* ws,
-                                 int* sticky, int E, int n, int k, int in_dim1, int topk, const void* w2, float* y2,
+                                 IdFlags flags, int E, int n, int k, int in_dim1, int topk, const void* w2, float* y2,
                                  int mode, hipStream_t s) {
     if (k != 2048) return hipErrorInvalidValue;
-    return moe_dma_nsb<8>(w, x, y, ids, planes, ws, sticky, E, n, in_dim1, topk, w2, y2, mode, s);
+    return moe_dma_nsb<8>(w, x, y, ids, planes, ws, flags, E, n, in_dim1, topk, w2, y2, mode, s);
 }
 
 // The weights of one call: w alone (MOE_ONE), w and w2 into y and y2
@@ -1028,7 +1028,7 @@ struct MoeOut {
     float* y2;
     const uint32_t* ids;  // the routing inputs, for a call routed in-kernel
     int planes;
-    int* sticky;
+    IdFlags flags;
     bool route;  // k_moe_route sorted the planes
 };
 
@@ -1044,7 +1044,7 @@ static hipError_t moe_lds_cfg(const void* w, const float* x, float* y, int* ws, 
     if (hipError_t e = set_lds_limit((const void*)k_moe_lds<TYPE, LPR, R, TPL, GLU>, MOE_LDS)) return e;
     dim3 grid((n + ROWS - 1) / ROWS, o.route ? max_slots : E + 1, o.mode == MOE_PAIR ? 2 : 1);
     hipLaunchKernelGGL((k_moe_lds<TYPE, LPR, R, TPL, GLU>), grid, dim3(256), shm, s, (const uint8_t*)w, x, y, ws, E,
-                       n, K, in_dim1, topk, pgmax, (const uint8_t*)o.w2, o.y2, o.ids, o.planes, o.sticky,
+                       n, K, in_dim1, topk, pgmax, (const uint8_t*)o.w2, o.y2, o.ids, o.planes, o.flags,
                        o.route ? 1 : 0);
     return hipGetLastError();
 }
@@ -1106,20 +1106,20 @@ bool moe_stages(int64_t k) {
 
 hipError_t launch_moe(int type, const void* w, int64_t E, int64_t n, int64_t k, const float* x, int64_t batch,
                       int64_t in_dim1, const uint32_t* ids, int64_t topk, float* y, int* ws,
-                      size_t ws_cap, int* sticky, int mode, const void* w2, float* y2, hipStream_t s) {
+                      size_t ws_cap, IdFlags flags, int mode, const void* w2, float* y2, hipStream_t s) {
     int planes = (int)(batch * topk);
     // several planes an expert (prefill): the grouped GEMM, where its
     // workspace fits
     const int64_t rows = in_dim1 == 1 ? batch : planes;
     if (moe_gemm_fits(type, E, planes, rows, n, k) && moe_gemm_workspace_bytes(E, planes, rows, k) <= ws_cap)
-        return launch_moe_gemm({type, mode, w, w2, E, n, k, batch, in_dim1, topk, x, ids, y, y2, ws, sticky}, s);
+        return launch_moe_gemm({type, mode, w, w2, E, n, k, batch, in_dim1, topk, x, ids, y, y2, ws, flags}, s);
     // the staged kernel routes up to MOE_FUSE_MAX planes itself (no routing
     // launch); otherwise k_moe_route sorts them first.  Planes of bad ids are
     // zeroed in every output either way.
     const bool route = !moe_stages(k) || planes > MOE_FUSE_MAX;
     hipError_t err = hipSuccess;
     if (route) {
-        hipLaunchKernelGGL(k_moe_route, dim3(1), dim3(1024), 2 * E * sizeof(int), s, ids, planes, (int)E, ws, sticky,
+        hipLaunchKernelGGL(k_moe_route, dim3(1), dim3(1024), 2 * E * sizeof(int), s, ids, planes, (int)E, ws, flags,
                            y, mode == MOE_PAIR ? y2 : nullptr, (int)n);
         if ((err = hipGetLastError()) != hipSuccess) return err;
     }
@@ -1133,9 +1133,9 @@ hipError_t launch_moe(int type, const void* w, int64_t E, int64_t n, int64_t k, 
     // decode-like routing of Q4_K rows of 2048 elements: k_moe_dma, routed
     // in-kernel
     if (moe_dma_fits(type, n, k, E, planes))
-        return launch_moe_dma(w, x, y, ids, planes, ws, sticky, (int)E, (int)n, (int)k, (int)in_dim1, (int)topk, w2,
+        return launch_moe_dma(w, x, y, ids, planes, ws, flags, (int)E, (int)n, (int)k, (int)in_dim1, (int)topk, w2,
                               y2, mode, s);
-    const MoeOut o{mode, w2, y2, ids, planes, sticky, route};
+    const MoeOut o{mode, w2, y2, ids, planes, flags, route};
     const int Ei = (int)E, ni = (int)n, ki = (int)k, d1 = (int)in_dim1, tk = (int)topk;
     if (moe_stages(k)) {
         if (mode == MOE_GLU) {

@@ -41,7 +41,7 @@ constexpr int MG_NT = 2;      // 16-row weight tiles a wave holds
 constexpr int MG_COLS = MG_WAVES * MG_NT * 16;
 
 // ---------------------------------------------------------- the workspace --
-// int hdr[16] ([0] a bad id was seen, [1] tiles), then at 256-byte steps:
+// int hdr[16] ([1] tiles), then at 256-byte steps:
 // int4 tiles[] (expert, first place in sorted, planes), int sorted[planes],
 // float inv[rows] (2^-s), fp16 sums[rows][K/256][16] (hi, lo of the eight
 // sums / 32), and x' [rows][K/256][1 KB].
@@ -108,7 +108,7 @@ bool moe_gemm_fits(int type, int64_t E, int64_t planes, int64_t rows, int64_t n,
 // atomics; every plane's dot is computed on its own, so no result depends on
 // it.
 __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, int E, int* hdr, int4* tiles,
-                         int* sorted, int* sticky, float* y, float* y2, int n, int tile_rows) {
+                         int* sorted, IdFlags flags, float* y, float* y2, int n, int tile_rows) {
     __shared__ int s_cnt[MOE_MAX_EXPERTS];
     __shared__ int s_first, s_tile, s_tiles, s_at;
     const int tid = threadIdx.x;
@@ -156,8 +156,8 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
     }
     __syncthreads();
     if (tid == 0 && e == 0) {
-        hdr[0] = bad;            // this call: read back by a strict call
-        if (bad) sticky[0] = 1;  // until the next lloom_hip_ctx_sync
+        flags.call[0] = bad;            // this call: read back by a strict call
+        if (bad) flags.sticky[0] = 1;  // until the next lloom_hip_ctx_sync
         hdr[1] = s_tiles;
     }
     const int c = s_cnt[e];
@@ -209,9 +209,9 @@ __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict_
                                                         uint8_t* __restrict__ xq, _Float16* __restrict__ sums,
                                                         float* __restrict__ inv, const uint32_t* __restrict__ ids,
                                                         int planes, int E, int* hdr, int4* tiles, int* sorted,
-                                                        int* sticky, float* y, float* y2, int n, int tile_rows) {
+                                                        IdFlags flags, float* y, float* y2, int n, int tile_rows) {
     if ((int)blockIdx.x < E) {
-        mg_route(ids, planes, blockIdx.x, E, hdr, tiles, sorted, sticky, y, y2, n, tile_rows);
+        mg_route(ids, planes, blockIdx.x, E, hdr, tiles, sorted, flags, y, y2, n, tile_rows);
         return;
     }
     const int lane = threadIdx.x & 63, row = (blockIdx.x - E) * 16 + (threadIdx.x >> 6);
@@ -720,7 +720,7 @@ static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     uint8_t* xq = ws + l.xq;
     hipLaunchKernelGGL(k_moe_gemm_prep<TYPE>, dim3((unsigned)(c.E + (rows + 15) / 16)), dim3(1024), 0, s,
                        c.x, (int)rows, (int)c.k, xq, (_Float16*)sums, inv, c.ids, (int)planes, (int)c.E, hdr, tiles,
-                       sorted, c.sticky, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, l.tile_rows);
+                       sorted, c.flags, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, l.tile_rows);
     if (hipError_t e = hipGetLastError()) return e;
     const bool glu = c.mode == MOE_GLU;
     const int pair = c.mode == MOE_PAIR ? 1 : 0;

@@ -467,11 +467,11 @@ __device__ __forceinline__ void store_out<uint16_t>(uint16_t* y, int64_t i, floa
 // CPU arm's QuantizedType::embedding, :812-838): output block ob belongs to
 // output row ob / rb and reads block ob % rb of weight row ids[row].  With
 // ids null the map is the identity (dequantize).  An id >= rows stores a
-// zero row and raises flag[0] (sticky) and flag[1] (this call).
+// zero row and raises both flags.
 struct RowMap {
     const uint32_t* ids;
     int64_t rb, rows;
-    int* flag;
+    IdFlags flags;
 };
 
 // The source block of output block ob, or -1 for a bad id.
@@ -481,8 +481,8 @@ __device__ __forceinline__ int64_t src_block(int64_t ob, const RowMap& rm) {
     const uint32_t id = rm.ids[r];
     if ((int64_t)id >= rm.rows) {
         if (ob % rm.rb == 0) {
-            atomicOr(&rm.flag[0], 1);
-            atomicOr(&rm.flag[1], 1);
+            *rm.flags.sticky = 1;
+            *rm.flags.call = 1;
         }
         return -1;
     }
@@ -649,8 +649,8 @@ hipError_t launch_dequantize(int type, const void* w, void* y, int out_dtype, in
 }
 
 hipError_t launch_embedding(int type, const void* w, int64_t rows, int64_t hidden, const uint32_t* ids, int64_t n_ids,
-                            void* y, int out_dtype, int* flag, hipStream_t s) {
-    const RowMap rm{ids, hidden / block_elems(type), rows, flag};
+                            void* y, int out_dtype, IdFlags flags, hipStream_t s) {
+    const RowMap rm{ids, hidden / block_elems(type), rows, flags};
     const int64_t elems = n_ids * hidden;
     if (out_dtype == T_F16) return dequant_t<uint16_t>(type, w, (uint16_t*)y, elems, rm, s);
     return dequant_t<float>(type, w, (float*)y, elems, rm, s);
