@@ -1,5 +1,5 @@
 // moe_gemm.hip -- routed experts with several planes an expert (prefill):
-// QTensor::indexed_moe_forward* as a grouped GEMM on v_mfma_f32_16x16x32_f16.
+// QTensor::indexed_moe_forward* as a grouped GEMM on v_mfma_f32_32x32x16_f16.
 //
 // The contract is the CPU arm's (matmul_t_indexed, lloom-tensor/src/quantized
 // /mod.rs:766-810): f32 activations, exactly dequantized weights, f32 sums.
@@ -34,11 +34,10 @@ namespace lloom {
 
 typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
-typedef float gf4 __attribute__((ext_vector_type(4)));
+typedef float gf16 __attribute__((ext_vector_type(16)));
 
 constexpr int MG_WAVES = 4;   // waves of a GEMM workgroup
-constexpr int MG_NT = 2;      // 16-row weight tiles a wave holds
-constexpr int MG_COLS = MG_WAVES * MG_NT * 16;
+constexpr int MG_COLS = MG_WAVES * 32;  // weight rows of a workgroup (SwiGLU: half of each weight)
 
 // ---------------------------------------------------------- the workspace --
 // int hdr[16] ([1] tiles), then at 256-byte steps:
@@ -48,22 +47,22 @@ constexpr int MG_COLS = MG_WAVES * MG_NT * 16;
 static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Planes of a tile, at most: 64, and 32 up to 16 planes an expert, where the
-// smaller LDS and register budget keeps three workgroups a CU instead of two
-// ([128, 768, 2048] Q4_K, T tokens top-8, 32 / 64 a tile: T = 64 45 / 62 us,
-// 256 58 / 68, 512 93 / 79, 2000 183 / 161).
-static int mg_tile_rows(int64_t E, int64_t planes) {
+// smaller LDS and register budget keeps four (Q6_K three) workgroups a CU
+// instead of two ([128, 768, 2048], T tokens top-8, 32 / 64 a tile: Q4_K T = 64
+// 46 / 53 us, 256 51 / 58, 512 74 / 68; Q6_K 64 81 / 92, 256 86 / 93, 512 126 /
+// 107; the Q4_K SwiGLU launch, whose 32 spill, 64 87 / 82, 256 98 / 88).
+static int mg_tile_rows(int type, int64_t E, int64_t planes, int mode) {
+    if (type == T_Q4K && mode == MOE_GLU) return 64;
     return planes > 16 * (E < planes ? E : planes) ? 64 : 32;
 }
 
 struct MgLayout {
     size_t tiles, sorted, inv, sums, xq, total;
     int64_t max_tiles;
-    int tile_rows;
 };
 static MgLayout mg_layout(int64_t E, int64_t planes, int64_t rows, int64_t k) {
     MgLayout l;
-    l.tile_rows = mg_tile_rows(E, planes);
-    l.max_tiles = planes / l.tile_rows + (E < planes ? E : planes);
+    l.max_tiles = planes / 32 + (E < planes ? E : planes);
     l.tiles = 256;
     l.sorted = l.tiles + up256((size_t)l.max_tiles * 16);
     l.inv = l.sorted + up256((size_t)planes * 4);
@@ -164,9 +163,8 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
     if (c == 0) return;  // uniform
     first = s_first;
     tile = s_tile;
-    // tiles of one size: the planes over as few tiles as hold them, each a
-    // multiple of 16
-    const int k = (c + tile_rows - 1) / tile_rows, rows = ((c + k - 1) / k + 15) & ~15;
+    // the planes over as few tiles as hold them, each a multiple of 32
+    const int k = (c + tile_rows - 1) / tile_rows, rows = ((c + k - 1) / k + 31) & ~31;
     for (int i = tid; i < k; i += 1024) tiles[tile + i] = make_int4(e, first + i * rows, min(rows, c - i * rows), 0);
     for (int p0 = tid; p0 < planes; p0 += 8 * 1024) {
         uint32_t id[8];
@@ -179,28 +177,25 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
 }
 
 // Place of the 8-element group G (elements 8G .. 8G + 7) of a superblock in
-// the GEMM's operand order.  Lane group g of MFMA step s takes:
-//   Q4_K  qs bytes 32g + 8 (s / 2) .., the low (s even) or high nibbles:
-//         elements 64g + 32 (s & 1) + 8 (s / 2) ..
-//   Q6_K  ql bytes 32g + 8 (s / 2) .., likewise: elements
-//         128 (g / 2) + 32 (g & 1) + 64 (s & 1) + 8 (s / 2) ..
-// so a lane's weights of a superblock are 32 contiguous bytes (Q6_K: and 32
-// of qh) and it needs two scales (Q6_K: four).
+// the GEMM's operand order: lane half h of MFMA step t (16 of them) takes
+//   Q4_K  qs bytes 64h + 8 (t / 2) .., the low (t even) or high nibbles
+//   Q6_K  ql bytes 64h + 8 (t / 2) .., likewise
+// so a lane's weights of a superblock are 64 contiguous bytes (Q6_K: and 32
+// of qh), and eight steps hold half of them.
 template <int TYPE>
-__device__ __forceinline__ void mg_place(int G, int& s, int& g) {
-    if constexpr (TYPE == T_Q4K) {
-        g = G >> 3;
-        s = 2 * (G & 3) + ((G >> 2) & 1);
-    } else {
-        g = 2 * (G >> 4) + ((G >> 2) & 1);
-        s = 2 * (G & 3) + ((G >> 3) & 1);
-    }
+__device__ __forceinline__ void mg_place(int G, int& t, int& h) {
+    h = G >> 4;
+    const int q = (G >> 2) & 3;  // the 32-element run in the half
+    // Q4_K: runs 2i, 2i + 1 are the nibbles of qs bytes 32i ..; Q6_K: runs q,
+    // q + 2 those of ql bytes 32q ..
+    const int chunk = TYPE == T_Q4K ? q >> 1 : q & 1, nib = TYPE == T_Q4K ? q & 1 : q >> 1;
+    t = 2 * (4 * chunk + (G & 3)) + nib;
 }
 
-// x' of a superblock: [half s / 4][hi, lo][pair (s / 2) & 1][s & 1][g][8]
-// fp16, so a GEMM stage (four steps) takes whole 128-byte lines of a row.
-__device__ __forceinline__ int mg_xq_off(int s, int g) {
-    return (s >> 2) * 512 + ((s >> 1) & 1) * 128 + (s & 1) * 64 + g * 16;
+// x' of a superblock: [half t / 8][hi, lo][(t / 4) & 1][t & 3][h][8] fp16, so a
+// GEMM stage (eight steps) takes whole 128-byte lines of a row.
+__device__ __forceinline__ int mg_xq_off(int t, int h) {
+    return (t >> 3) * 512 + ((t >> 2) & 1) * 128 + ((t & 3) * 2 + h) * 16;
 }
 
 // The first E workgroups route; the others convert 16 rows each, one a wave.
@@ -270,32 +265,33 @@ __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict_
 
 // ------------------------------------------------------------------- GEMM --
 
-// A lane's weights of one superblock of its row.
+// A lane's weights of one superblock of its row: half h of the quants.
 template <int TYPE>
 struct MgW;
 template <>
 struct MgW<T_Q4K> {
-    uint4 hdr, q[2];
-    static constexpr int LOADS = 3;
+    uint4 hdr, q[4];
+    static constexpr int LOADS = 5;
 };
 template <>
 struct MgW<T_Q6K> {
-    uint4 q[2], h[2];
-    uint4 sc;
+    uint4 q[4], h[2];
+    uint2 sc;
     uint32_t d;
-    static constexpr int LOADS = 9;  // at least: 36, 36, 20 and 2 bytes by at most 16
+    static constexpr int LOADS = 10;  // at least: 68, 36, 12 and 2 bytes by at most 16
 };
 
 template <int TYPE>
-__device__ __forceinline__ void mg_load(const uint8_t* __restrict__ b, int g, MgW<TYPE>& w) {
+__device__ __forceinline__ void mg_load(const uint8_t* __restrict__ b, int h, MgW<TYPE>& w) {
     if constexpr (TYPE == T_Q4K) {
         w.hdr = *(const uint4*)b;
-        w.q[0] = *(const uint4*)(b + 16 + 32 * g);
-        w.q[1] = *(const uint4*)(b + 32 + 32 * g);
+#pragma unroll
+        for (int i = 0; i < 4; i++) w.q[i] = *(const uint4*)(b + 16 + 64 * h + 16 * i);
     } else {
-        load32_a2(b + 32 * g, w.q[0], w.q[1]);
-        load32_a2(b + Q6K_QH + 32 * (g >> 1), w.h[0], w.h[1]);
-        w.sc = load16_a2(b + Q6K_SC);
+        load32_a2(b + 64 * h, w.q[0], w.q[1]);
+        load32_a2(b + 64 * h + 32, w.q[2], w.q[3]);
+        load32_a2(b + Q6K_QH + 32 * h, w.h[0], w.h[1]);
+        w.sc = load8_a2(b + Q6K_SC + 8 * h);
         w.d = *(const uint16_t*)(b + Q6K_D);
     }
 }
@@ -308,38 +304,42 @@ __device__ __forceinline__ gh2 bytes_h2(uint32_t w) {
     return as_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) + both((_Float16)-1024.0f);
 }
 
-// What a lane needs of its superblock's header.
+// The scales of a lane's half superblock.
 template <int TYPE>
 struct MgS;
 template <>
 struct MgS<T_Q4K> {
-    gh2 s[2], o[2];  // low, high nibbles: scale and offset (twice each)
+    gh2 s[2], o[2];  // [32-byte chunk]{low, high nibbles}: scale and offset
 };
 template <>
 struct MgS<T_Q6K> {
-    gh2 s[2][2];  // [low, high nibbles][bytes 0-15, 16-31]
+    gh2 s[2][2];  // [32-byte chunk][low, high nibbles]{bytes 0-15, 16-31}
 };
 
 template <int TYPE>
-__device__ __forceinline__ void mg_scales(const MgW<TYPE>& w, int g, MgS<TYPE>& c) {
+__device__ __forceinline__ void mg_scales(const MgW<TYPE>& w, int h, MgS<TYPE>& c) {
     if constexpr (TYPE == T_Q4K) {
-        // sub-blocks 2g and 2g + 1: scales 0-3 are bytes of hdr.y, 4-7 the
-        // low nibbles of hdr.w under hdr.y's top bits
-        const uint32_t lo = w.hdr.y & 0x3F3F3F3Fu, hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
-        const gh2 p = bytes_h2((g < 2 ? lo : hi) >> (16 * (g & 1)));
+        // sub-blocks 4h .. 4h + 3: scales 0-3 are bytes of hdr.y, 4-7 the low
+        // nibbles of hdr.w under hdr.y's top bits.
         // (1024 + q) sc - 1024 sc, and for a high nibble left in place
         // (1024 + 16 q) (sc / 16) - 64 sc: both are sc q, exact
-        c.s[0] = both(p[0]);
-        c.o[0] = both(p[0] * (_Float16)-1024.0f);
-        c.s[1] = both(p[1] * (_Float16)0.0625f);
-        c.o[1] = both(p[1] * (_Float16)-64.0f);
+        const uint32_t lo = w.hdr.y & 0x3F3F3F3Fu, hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
+        const uint32_t v = h ? hi : lo;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const gh2 p = bytes_h2(v >> (16 * i));
+            c.s[i] = p * gh2{(_Float16)1.0f, (_Float16)0.0625f};
+            c.o[i] = p * gh2{(_Float16)-1024.0f, (_Float16)-64.0f};
+        }
     } else {
-        // the scale of element e is sc[e / 16]: 8 (g / 2) + 2 (g & 1) + 4 nibble + (byte / 16)
-        const uint32_t a = (g < 2 ? w.sc.x : w.sc.z) >> (16 * (g & 1)), b = (g < 2 ? w.sc.y : w.sc.w) >> (16 * (g & 1));
-        c.s[0][0] = both((_Float16)(int)(int8_t)(a & 0xff));
-        c.s[0][1] = both((_Float16)(int)(int8_t)((a >> 8) & 0xff));
-        c.s[1][0] = both((_Float16)(int)(int8_t)(b & 0xff));
-        c.s[1][1] = both((_Float16)(int)(int8_t)((b >> 8) & 0xff));
+        // element 128h + 32q + l has scale sc[8h + 2q + l / 16]
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t v = i ? w.sc.y : w.sc.x;  // runs 2i, 2i + 1: high nibbles of chunks 0, 1 for i = 1
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                c.s[j][i] = gh2{(_Float16)(int)(int8_t)byte_of(v, 2 * j), (_Float16)(int)(int8_t)byte_of(v, 2 * j + 1)};
+        }
     }
 }
 
@@ -352,33 +352,34 @@ __device__ __forceinline__ gh2 and_1024(uint32_t v, uint32_t mask, uint32_t k64)
     return as_h2(r);
 }
 
-// The B operand(s) of step s (compile-time): eight weights of the lane.
+// The B operand(s) of step t (compile-time): eight weights of the lane.
 template <int TYPE>
-__device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c, int s, int g, uint32_t k64, gh8& bh,
-                                          gh8& bl) {
-    const int nib = s & 1, at = (s >> 1) & 1, half = s >> 2;
+__device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c, int t, uint32_t k64, gh8& bh, gh8& bl) {
+    const int nib = t & 1, g = t >> 1, chunk = g >> 2;  // byte group g of 8: bytes 8g .. 8g + 7 of the lane's 64
     uint32_t r[4], l[4];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const uint32_t v = dword_of(w.q[half], 2 * at + i);
+        const uint32_t v = dword_of(w.q[g >> 1], 2 * (g & 1) + i);
         if constexpr (TYPE == T_Q4K) {
             const uint32_t mask = nib ? 0x00F000F0u : 0x000F000Fu;
+            const gh2 sc = both(c.s[chunk][nib]), of = both(c.o[chunk][nib]);
             const gh2 e = and_1024(v, mask, k64), o = and_1024(v >> 8, mask, k64);
-            r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, c.s[nib], c.o[nib]));
-            r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(o, c.s[nib], c.o[nib]));
+            r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, sc, of));
+            r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(o, sc, of));
         } else {
-            // two high bits of element q = (g & 1) + 2 nib: bits 2q of qh
-            const uint32_t h = dword_of(w.h[half], 2 * at + i) >> (2 * (g & 1));
-            const uint32_t q = nib ? ((v >> 4) & 0x0F0F0F0Fu) | (h & 0x30303030u)
-                                   : (v & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u);
+            // the two high bits of run q = chunk + 2 nib are bits 2q of qh byte 8 (g % 4) ..
+            const uint32_t hb = dword_of(w.h[(g & 3) >> 1], 2 * (g & 1) + i);
+            const int sh = 2 * chunk + 4 * nib;  // to bits 4, 5
+            const uint32_t hi2 = (sh <= 4 ? hb << (4 - sh) : hb >> (sh - 4)) & 0x30303030u;
+            const uint32_t q = ((nib ? v >> 4 : v) & 0x0F0F0F0Fu) | hi2;
             const gh2 k = both((_Float16)-1056.0f);  // -(1024 + 32)
+            const gh2 sc = both(c.s[chunk][nib][(g & 3) >> 1]);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const gh2 t = as_h2(__builtin_amdgcn_perm(0x64646464u, q, j ? 0x04030402u : 0x04010400u)) + k;
-                const gh2 sc = c.s[nib][half];
-                const gh2 hi = t * sc;
+                const gh2 x = as_h2(__builtin_amdgcn_perm(0x64646464u, q, j ? 0x04030402u : 0x04010400u)) + k;
+                const gh2 hi = x * sc;
                 r[2 * i + j] = __builtin_bit_cast(uint32_t, hi);
-                l[2 * i + j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, sc, -hi));
+                l[2 * i + j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(x, sc, -hi));
             }
         }
     }
@@ -399,28 +400,28 @@ __device__ __forceinline__ void mg_wait_barrier() {
 __device__ __forceinline__ void mg_keep(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 __device__ __forceinline__ void mg_keep(MgW<T_Q4K>& w) {
     mg_keep(w.hdr);
-    mg_keep(w.q[0]);
-    mg_keep(w.q[1]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) mg_keep(w.q[i]);
 }
 __device__ __forceinline__ void mg_keep(MgW<T_Q6K>& w) {
-    mg_keep(w.q[0]);
-    mg_keep(w.q[1]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) mg_keep(w.q[i]);
     mg_keep(w.h[0]);
     mg_keep(w.h[1]);
-    mg_keep(w.sc);
-    asm volatile("" : "+v"(w.d));
+    asm volatile("" : "+v"(w.sc.x), "+v"(w.sc.y), "+v"(w.d));
 }
 
-// The order of half a step's instructions: its LDS reads, then the unpacking
-// spread between the MFMAs.
+// The order of half a step's instructions: its LDS reads, then half of the
+// next step's unpacking spread between its n MFMAs.
 template <int TYPE, int MT>
 __device__ __forceinline__ void mg_sched(int n) {
-    constexpr int V = TYPE == T_Q6K ? 64 : 20;  // about the VALU instructions of a step's unpacking
+    constexpr int V = TYPE == T_Q6K ? 32 : 12;  // about the VALU instructions of a step's unpacking
+    constexpr int M = (TYPE == T_Q6K ? 3 : 2) * MT;
     __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
 #pragma unroll
-    for (int i = 0; i < n * MT * MG_NT; i++) {
+    for (int i = 0; i < n; i++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, (V + 2 * MT * MG_NT - 1) / (2 * MT * MG_NT), 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (V + M - 1) / M, 0);
     }
 }
 
@@ -433,105 +434,89 @@ struct MgArgs {
 };
 
 // A 16-byte LDS read serves a wave in four passes of 16 lanes, the first two
-// lanes {0-3, 12-15, 20-27} and the rest of 0-31 (two lane groups g of 16
-// rows c): with row c's piece p at place p ^ key(c) of its 128-byte line, the
-// 16 lanes of a pass read 16 different pieces of the 256 bytes of the banks.
-__device__ __forceinline__ int mg_key(int c) { return ((c >> 1) + 2) & 7; }
+// lanes {0-3, 12-15, 20-27} and the rest of 0-31: with row r's piece p at
+// place p ^ key(r) of its 128-byte line, the 16 rows of a pass read 16
+// different pieces of the 256 bytes of the banks.
+__device__ __forceinline__ int mg_key(int r) { return (r >> 1) & 7; }
 
-// A tile of MT * 16 planes against the workgroup's weight rows.
+// A tile of np <= 32 MT planes against the workgroup's weight rows.  MFMA
+// operands (32x32x16): lane l holds plane (weight row) l % 32, elements 8 (l /
+// 32) .. of the step; the result's lane l holds weight row l % 32, planes 8 (i
+// / 4) + 4 (l / 32) + i % 4.
 //
-// LDS holds two stages of half a superblock (four MFMA steps): the rows'
-// x' in octets of 8 rows, an octet's 128-byte line (hi or lo, step pair) as
-// one 1 KB DMA: row r's 16-byte piece u at place u ^ mg_key(r) of its line.
+// LDS holds two stages of half a superblock (eight MFMA steps): the rows' x'
+// in octets of 8 rows, an octet's 128-byte line (hi or lo, four steps) as one
+// 1 KB DMA: row r's 16-byte piece u at place u ^ mg_key(r) of its line.
 // While a stage is computed, the next one's DMAs and the next superblock's
 // weight loads are in flight; a stage starts with one counted wait and one
-// barrier.
+// barrier.  Rows past np hold whatever LDS held: their sums are not stored.
 template <int TYPE, int ROWS, int MT, bool GLU>
-__device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y, uint8_t* smem,
-                                        const int* s_plane, const float* s_inv) {
-    constexpr int NT = MG_NT, STAGE = mg_stage(ROWS);
+__device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y,
+                                        uint8_t* smem, const int* s_plane, const int* s_row, const float* s_inv) {
+    constexpr int STAGE = mg_stage(ROWS);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, c16 = lane & 15;
+    const int h = lane >> 5, c32 = lane & 31;
     const int nsb = A.K >> 8;
-    const uint32_t rowbytes = (uint32_t)nsb * block_bytes(TYPE);
 
-    // this wave's weight rows: GLU takes 16 of the gate and the same of the up weight
-    uint32_t woff[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int r = GLU ? col0 + wave * 16 * (NT / 2) + 16 * (t % (NT / 2)) + c16 : col0 + wave * 16 * NT + 16 * t + c16;
-        woff[t] = (uint32_t)min(r, A.n - 1) * rowbytes;
-    }
-    auto load_w = [&](int sb, MgW<TYPE>(&w)[NT]) {
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-            mg_load<TYPE>((GLU && t >= NT / 2 ? W1 : W0) + (size_t)sb * block_bytes(TYPE) + woff[t], g, w[t]);
-    };
+    // this lane's weight row: SwiGLU takes 16 of the gate (lanes c32 < 16) and
+    // the same 16 of the up weight
+    const int wrow = GLU ? col0 + wave * 16 + (c32 & 15) : col0 + wave * 32 + c32;
+    const uint8_t* wp = (GLU && c32 >= 16 ? W1 : W0) + (size_t)min(wrow, A.n - 1) * ((uint32_t)nsb * block_bytes(TYPE));
+    auto load_w = [&](int sb, MgW<TYPE>& w) { mg_load<TYPE>(wp + (size_t)sb * block_bytes(TYPE), h, w); };
 
-    // x' DMAs: wave w moves (hi or lo, step pair) w of every octet
-    uint32_t xoff[2 * MT];
+    // x' DMAs: wave w moves line w (hi or lo, step quad) of every octet
+    const int octets = (np + 7) >> 3;
+    uint32_t xoff[4 * MT];
 #pragma unroll
-    for (int o = 0; o < 2 * MT; o++) {
-        const int r = s_plane[min(8 * o + (lane >> 3), np - 1)] / A.rowdiv;
-        xoff[o] = (uint32_t)r * (uint32_t)A.K * 4u + (uint32_t)(((lane & 7) ^ mg_key(8 * (o & 1) + (lane >> 3))) * 16);
+    for (int o = 0; o < 4 * MT; o++) {
+        const int r = 8 * o + (lane >> 3);
+        xoff[o] = (uint32_t)s_row[min(r, np - 1)] * (uint32_t)A.K * 4u + (uint32_t)(((lane & 7) ^ mg_key(r & 31)) * 16);
     }
-    uint32_t soff = 0;
-    if constexpr (TYPE == T_Q4K)
-        soff = (uint32_t)(s_plane[min(32 * (wave & 1) + (lane >> 1), np - 1)] / A.rowdiv) * (uint32_t)nsb * 32u + (lane & 1) * 16;
+    const uint32_t soff = (uint32_t)s_row[min(32 * (wave & 1) + (lane >> 1), np - 1)] * (uint32_t)nsb * 32u + (lane & 1) * 16;
     const uint32_t lds0 = lds_addr(smem);
     auto issue = [&](int sb, int half) {
         const uint8_t* base = A.xq + (size_t)sb * 1024 + half * 512 + wave * 128;
         const uint32_t to = lds0 + half * STAGE + wave * 1024;
 #pragma unroll
-        for (int o = 0; o < 2 * MT; o++) dma16s(base, xoff[o], to + o * 4096);
+        for (int o = 0; o < 4 * MT; o++)
+            if (o < octets) dma16s(base, xoff[o], to + o * 4096);  // uniform
     };
     auto issue_sums = [&](int sb) {
         if constexpr (TYPE == T_Q4K)
-            if (wave < (MT + 1) / 2)
+            if (wave < MT)
                 dma16s(A.sums + (size_t)sb * 32, soff, lds0 + 2 * STAGE + (sb & 1) * (ROWS * 32) + wave * 1024);
     };
-    static_assert(MG_WAVES == 4, "a wave a (part, step pair)");
+    static_assert(MG_WAVES == 4, "a wave a line");
 
-    // the operand reads of a stage: row 16t + c16, piece 4 (s & 1) + g
-    const uint32_t a0 = (uint32_t)((c16 >> 3) * 4096 + (c16 & 7) * 128 + ((g ^ mg_key(c16)) * 16));
-    const uint8_t* ap[2] = {smem + a0, smem + (a0 ^ 64u)};
+    // the operand reads of a stage: row 32 T + c32, piece 2 (t % 4) + h
+    const uint32_t a0 = (uint32_t)((c32 >> 3) * 4096 + (c32 & 7) * 128 + ((h ^ mg_key(c32)) * 16));
+    const uint8_t* ap[4] = {smem + a0, smem + (a0 ^ 32u), smem + (a0 ^ 64u), smem + (a0 ^ 96u)};
 
-    gf4 out[MT][NT], acc[MT][NT];
+    gf16 out[MT], acc[MT];
+    const gf16 z = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < MT; t++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) out[t][j] = gf4{0.0f, 0.0f, 0.0f, 0.0f};
-    const gf4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int T = 0; T < MT; T++) out[T] = z;
 
     // A step's MFMAs take the activations' lo, then their hi; its hi is read
     // while lo's MFMAs run, the next step's lo while hi's run, and the next
     // step's weights are unpacked between them.
-    // (Q6_K, whose weights take twice the registers, unpacks a step's own.)
-    constexpr bool AHEAD = TYPE == T_Q4K;
-    gh8 ah[MT], al[MT], bh[2][NT], bl[2][NT];
-    MgW<TYPE> w[NT], nxt[NT];
-    MgS<TYPE> sc[NT];
+    gh8 ah[MT], al[MT], bh[2], bl[2];
+    MgW<TYPE> w, nxt;
+    MgS<TYPE> sc;
     uint32_t k64 = 0x64006400u;
     asm("" : "+v"(k64));
-    auto read_a = [&](int s, int lo, gh8(&a)[MT]) {
-        const uint8_t* p = ap[s & 1] + (s >> 2) * STAGE + lo * 2048 + ((s >> 1) & 1) * 1024;
+    auto read_a = [&](int t, int lo, gh8(&a)[MT]) {
+        const uint8_t* p = ap[t & 3] + (t >> 3) * STAGE + lo * 2048 + ((t >> 2) & 1) * 1024;
 #pragma unroll
-        for (int t = 0; t < MT; t++) a[t] = *(const gh8*)(p + t * 8192);
-    };
-    auto unpack = [&](int s, int to) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) mg_unpack<TYPE>(w[j], sc[j], s, g, k64, bh[to][j], bl[to][j]);
+        for (int T = 0; T < MT; T++) a[T] = *(const gh8*)(p + T * 16384);
     };
     auto take_w = [&]() {
         // the loaded weights become the current ones here, before the next
         // loads and DMAs go out: the wait the compiler puts in front of their
         // use then finds nothing younger in flight
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            w[j] = nxt[j];
-            mg_keep(w[j]);
-            mg_scales<TYPE>(w[j], g, sc[j]);
-        }
+        w = nxt;
+        mg_keep(w);
+        mg_scales<TYPE>(w, h, sc);
     };
     load_w(0, nxt);
     issue(0, 0);
@@ -541,57 +526,49 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
     issue(0, 1);
     load_w(min(1, nsb - 1), nxt);
     read_a(0, 1, al);
-    if (AHEAD) unpack(0, 0);
+    mg_unpack<TYPE>(w, sc, 0, k64, bh[0], bl[0]);
     for (int sb = 0; sb < nsb; sb++) {
-        float d[NT], dm32[NT];
-        gh8 bm[NT], am[MT];
+        float d, dm32 = 0.0f;
+        gh8 bm, am[MT];
         const bool last = sb + 1 == nsb;
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
-            const int cur = AHEAD ? s & 1 : 0;
-            read_a(s, 0, ah);
-            if (!AHEAD) unpack(s, 0);
+        for (int t = 0; t < 16; t++) {
+            const int cur = t & 1;
+            read_a(t, 0, ah);
 #pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], bh[cur][j], s ? acc[t][j] : z, 0, 0, 0);
-            if (s < 7 && AHEAD) {
-                unpack(s + 1, cur ^ 1);
-                mg_sched<TYPE, MT>(1);
+            for (int T = 0; T < MT; T++)
+                acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[T], bh[cur], t ? acc[T] : z, 0, 0, 0);
+            if (t < 15) {
+                mg_unpack<TYPE>(w, sc, t + 1, k64, bh[cur ^ 1], bl[cur ^ 1]);
+                mg_sched<TYPE, MT>(MT);
             }
-            if (s == 3) {
+            if (t == 7) {
                 // the half's last reads are done: the other half has landed
                 // (its DMAs are older than the weight loads), and this one's
                 // place is free
-                mg_wait_barrier<MgW<TYPE>::LOADS * NT>();
+                mg_wait_barrier<MgW<TYPE>::LOADS>();
                 if (!last) {
                     issue(sb + 1, 0);
                     issue_sums(sb + 1);
                 }
             }
-            if (s < 7) {
-                read_a(s + 1, 1, al);
+            if (t < 15) {
+                read_a(t + 1, 1, al);
             } else {
                 // the epilogue's operands, before w moves on
-#pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    if constexpr (TYPE == T_Q4K) {
-                        const uint4 hd = w[j].hdr;
-                        d[j] = f16_to_f32(hd.x & 0xffffu);
-                        dm32[j] = 32.0f * f16_to_f32(hd.x >> 16);
-                        const uint32_t ml = hd.z & 0x3F3F3F3Fu,
-                                       mh = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
-                        const gh2 m0 = bytes_h2(ml), m1 = bytes_h2(ml >> 16), m2 = bytes_h2(mh), m3 = bytes_h2(mh >> 16);
-                        bm[j] = g < 2 ? gh8{m0[0], m0[1], m1[0], m1[1], m2[0], m2[1], m3[0], m3[1]} : gh8{};
-                    } else {
-                        d[j] = f16_to_f32(w[j].d);
-                    }
-                }
                 if constexpr (TYPE == T_Q4K) {
-                    const uint8_t* sp = smem + 2 * STAGE + (sb & 1) * (ROWS * 32) + c16 * 32 + (g & 1) * 16;
+                    const uint4 hd = w.hdr;
+                    d = f16_to_f32(hd.x & 0xffffu);
+                    dm32 = 32.0f * f16_to_f32(hd.x >> 16);
+                    const uint32_t ml = hd.z & 0x3F3F3F3Fu,
+                                   mh = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+                    const gh2 m0 = bytes_h2(ml), m1 = bytes_h2(ml >> 16), m2 = bytes_h2(mh), m3 = bytes_h2(mh >> 16);
+                    bm = gh8{m0[0], m0[1], m1[0], m1[1], m2[0], m2[1], m3[0], m3[1]};
+                    const uint8_t* sp = smem + 2 * STAGE + (sb & 1) * (ROWS * 32) + c32 * 32 + h * 16;
 #pragma unroll
-                    for (int t = 0; t < MT; t++) am[t] = *(const gh8*)(sp + t * 512);
+                    for (int T = 0; T < MT; T++) am[T] = *(const gh8*)(sp + T * 1024);
+                } else {
+                    d = f16_to_f32(w.d);
                 }
                 if (!last) {  // uniform
                     mg_wait_barrier<0>();
@@ -599,84 +576,81 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
                     issue(sb + 1, 1);
                     load_w(min(sb + 2, nsb - 1), nxt);
                     read_a(0, 1, al);
-                    if (AHEAD) unpack(0, 0);
+                    mg_unpack<TYPE>(w, sc, 0, k64, bh[0], bl[0]);
                 }
             }
             if constexpr (TYPE == T_Q6K) {
 #pragma unroll
-                for (int t = 0; t < MT; t++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++)
-                        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], bl[cur][j], acc[t][j], 0, 0, 0);
+                for (int T = 0; T < MT; T++)
+                    acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bl[cur], acc[T], 0, 0, 0);
             }
 #pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], bh[cur][j], acc[t][j], 0, 0, 0);
-            if (s != 7 && AHEAD) mg_sched<TYPE, MT>(1);
+            for (int T = 0; T < MT; T++)
+                acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bh[cur], acc[T], 0, 0, 0);
+            if (t != 15) mg_sched<TYPE, MT>((TYPE == T_Q6K ? 2 : 1) * MT);
         }
         // the superblock's scales (and the min term: K 0..7 the sums' hi,
-        // 8..15 their lo, the lanes of K 16..31 repeat them against zeros)
+        // 8..15 their lo, both against the mins)
 #pragma unroll
-        for (int j = 0; j < NT; j++)
+        for (int T = 0; T < MT; T++) {
+            if constexpr (TYPE == T_Q4K) {
+                const gf16 mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[T], bm, z, 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < MT; t++) {
-                if constexpr (TYPE == T_Q4K) {
-                    const gf4 mt = __builtin_amdgcn_mfma_f32_16x16x32_f16(am[t], bm[j], z, 0, 0, 0);
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        out[t][j][v] = __builtin_fmaf(d[j], acc[t][j][v], __builtin_fmaf(-dm32[j], mt[v], out[t][j][v]));
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; v++) out[t][j][v] = __builtin_fmaf(d[j], acc[t][j][v], out[t][j][v]);
-                }
-            }
-    }
-    // lane (g, c16): planes 16t + 4g + v of weight row c16 of each tile
-#pragma unroll
-    for (int t = 0; t < MT; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int q = 16 * t + 4 * g + v;
-            if (q >= np) continue;
-            float* yp = Y + (int64_t)s_plane[q] * A.n;
-            const float inv = s_inv[q];
-            if constexpr (GLU) {
-#pragma unroll
-                for (int j = 0; j < NT / 2; j++) {
-                    const int r = col0 + wave * 16 * (NT / 2) + 16 * j + c16;
-                    const float a = out[t][j][v] * inv, b = out[t][j + NT / 2][v] * inv;
-                    if (r < A.n) yp[r] = a / (1.0f + expf(-a)) * b;
-                }
+                for (int i = 0; i < 16; i++)
+                    out[T][i] = __builtin_fmaf(d, acc[T][i], __builtin_fmaf(-dm32, mt[i], out[T][i]));
             } else {
 #pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    const int r = col0 + wave * 16 * NT + 16 * j + c16;
-                    if (r < A.n) yp[r] = out[t][j][v] * inv;
-                }
+                for (int i = 0; i < 16; i++) out[T][i] = __builtin_fmaf(d, acc[T][i], out[T][i]);
             }
         }
+    }
+#pragma unroll
+    for (int T = 0; T < MT; T++) {
+        if constexpr (GLU) {
+            // lanes c32 < 16 hold the gate's sums, the others the up weight's
+            // of the same rows: exchanged between the two 16-lane rows, the
+            // first row has both of plane i, the second of plane i + 1
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+                const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, (float)out[T][i]),
+                                                                __builtin_bit_cast(unsigned, (float)out[T][i + 1]), false, false);
+                const unsigned r0 = r[0], r1 = r[1];
+                const int q = 32 * T + 8 * (i >> 2) + 4 * h + (i & 3) + (c32 >> 4);
+                if (q < np && wrow < A.n) {
+                    const float a = __builtin_bit_cast(float, r0) * s_inv[q], b = __builtin_bit_cast(float, r1) * s_inv[q];
+                    Y[(int64_t)s_plane[q] * A.n + wrow] = a / (1.0f + expf(-a)) * b;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int q = 32 * T + 8 * (i >> 2) + 4 * h + (i & 3);
+                if (q < np && wrow < A.n) Y[(int64_t)s_plane[q] * A.n + wrow] = out[T][i] * s_inv[q];
+            }
+        }
+    }
 }
 
 // What bounds it: [128, 768, 2048] Q4_K, 2000 tokens top-8, the SwiGLU launch
-// (two weights, 201 TFLOP of hi and lo products) takes 290 us with its prep.
-// Left with only its loads (no MFMA, no unpacking) it took 273, with only
-// its arithmetic 246: the L2-to-LDS stream of x' (1.6 GB, each tile's planes
-// once a weight block) and the VALU and MFMA issue bound it about equally.
+// (two weights, 201 GFLOP of hi and lo products) takes 273 us with its prep
+// (0.74 PFLOP/s; 301 on 16x16x32 MFMAs, whose twice as many issue slots left
+// less room for the unpacking).  On that earlier form, only the loads (no MFMA,
+// no unpacking) took 273, only the arithmetic 246: a superblock's two L2 round
+// trips and its arithmetic hide each other only in part at two workgroups a CU.
 // At 64 tokens it is the weight stream (113 MB a weight, 2.5 TB/s).  Eight
-// waves sharing one x' tile (half the stream) took 313: one workgroup a CU
-// leaves nothing to run at its barriers and its ends.
+// waves sharing one x' tile (half the L2 stream) took 313: one workgroup a CU
+// leaves nothing to run at its barriers and its ends.  With the rows of x'
+// interleaved by half superblock instead of whole it measured the same.
 // A workgroup takes item (tile of planes, weight block): items are dealt to
 // the XCDs in contiguous runs (workgroup b runs on XCD b % 8), so the blocks
 // of one tile, which read the same activations, and the tiles of one expert,
 // which read the same weights, meet in one XCD's L2.
 template <int TYPE, int ROWS, bool GLU>
-__global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 3 : 2) void k_moe_gemm(
+__global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 4 : 3) void k_moe_gemm(
     MgArgs A, const int* __restrict__ hdr, const int4* __restrict__ tiles, const int* __restrict__ sorted,
     const float* __restrict__ inv, int nblk, int pair) {
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int s_plane[ROWS];
+    __shared__ int s_plane[ROWS], s_row[ROWS];
     __shared__ float s_inv[ROWS];
     const int per_tile = nblk << pair, total = hdr[1] * per_tile;
     const int per = (total + 7) >> 3, at = (int)(blockIdx.x >> 3), item = (int)(blockIdx.x & 7) * per + at;
@@ -688,6 +662,7 @@ __global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 3 :
     if ((int)threadIdx.x < ROWS) {
         const int p = sorted[tl.y + min((int)threadIdx.x, np - 1)];
         s_plane[threadIdx.x] = p;
+        s_row[threadIdx.x] = p / A.rowdiv;
         s_inv[threadIdx.x] = inv[p / A.rowdiv];
     }
     __syncthreads();
@@ -696,21 +671,20 @@ __global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 3 :
     const uint8_t* W1 = GLU ? A.w[1] + ebytes : W0;
     float* Y = A.y[second];
     const int col0 = blk * (GLU ? MG_COLS / 2 : MG_COLS);
-    const int mt = (np + 15) >> 4;  // uniform
-    if (mt == 1) {
-        mg_tile<TYPE, ROWS, 1, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
-    } else if (mt == 2) {
-        mg_tile<TYPE, ROWS, 2, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
-    } else if constexpr (ROWS == 64) {
-        if (mt == 3) mg_tile<TYPE, ROWS, 3, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
-        else mg_tile<TYPE, ROWS, 4, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_inv);
+    if constexpr (ROWS == 64) {
+        if (np > 32) {  // uniform
+            mg_tile<TYPE, ROWS, 2, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
+            return;
+        }
     }
+    mg_tile<TYPE, ROWS, 1, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
 }
 
 template <int TYPE>
 static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     const int64_t planes = c.batch * c.topk, rows = c.in_dim1 == 1 ? c.batch : planes;
     const MgLayout l = mg_layout(c.E, planes, rows, c.k);
+    const int tile_rows = mg_tile_rows(TYPE, c.E, planes, c.mode);
     uint8_t* ws = (uint8_t*)c.ws;
     int* hdr = (int*)ws;
     int4* tiles = (int4*)(ws + l.tiles);
@@ -720,13 +694,13 @@ static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     uint8_t* xq = ws + l.xq;
     hipLaunchKernelGGL(k_moe_gemm_prep<TYPE>, dim3((unsigned)(c.E + (rows + 15) / 16)), dim3(1024), 0, s,
                        c.x, (int)rows, (int)c.k, xq, (_Float16*)sums, inv, c.ids, (int)planes, (int)c.E, hdr, tiles,
-                       sorted, c.flags, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, l.tile_rows);
+                       sorted, c.flags, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, tile_rows);
     if (hipError_t e = hipGetLastError()) return e;
     const bool glu = c.mode == MOE_GLU;
     const int pair = c.mode == MOE_PAIR ? 1 : 0;
     const int cols = glu ? MG_COLS / 2 : MG_COLS;
     const int nblk = (int)((c.n + cols - 1) / cols);
-    const int64_t items = (l.max_tiles * nblk) << pair;
+    const int64_t items = ((planes / tile_rows + (c.E < planes ? c.E : planes)) * nblk) << pair;
     const MgArgs a{{(const uint8_t*)c.w, (const uint8_t*)c.w2}, {c.y, c.y2}, xq, sums, (int)c.n, (int)c.k,
                    c.in_dim1 == 1 ? (int)c.topk : 1};
     const dim3 grid((unsigned)((items + 7) / 8 * 8));
@@ -735,7 +709,7 @@ static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
         hipLaunchKernelGGL(kern, grid, dim3(64 * MG_WAVES), mg_lds(rows_), s, a, hdr, tiles, sorted, inv, nblk, pair);
         return hipGetLastError();
     };
-    if (l.tile_rows == 64) return glu ? gemm(k_moe_gemm<TYPE, 64, true>, 64) : gemm(k_moe_gemm<TYPE, 64, false>, 64);
+    if (tile_rows == 64) return glu ? gemm(k_moe_gemm<TYPE, 64, true>, 64) : gemm(k_moe_gemm<TYPE, 64, false>, 64);
     return glu ? gemm(k_moe_gemm<TYPE, 32, true>, 32) : gemm(k_moe_gemm<TYPE, 32, false>, 32);
 }
 

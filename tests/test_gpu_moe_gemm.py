@@ -3,7 +3,7 @@ an expert on average) against a float64 product of the dequantized
 weights (O.dequantize, the CPU oracle's to_float), through the public calls.
 
 Where it can go wrong: planes of one expert around the 16-row tile and the
-64-row cut (1, 15, 16, 17, 63, 64, 65, 129 and none), weight rows off the
+64-row cut (1, 31, 32, 33, 63, 64, 65, 129 and none), weight rows off the
 workgroup's 128 (64 for the SwiGLU), one superblock a row, activations one
 row a token and one a slot, tiles of 32 planes and of 64, an out-of-range id,
 and a capture whose workspace holds only the routing.
@@ -21,8 +21,8 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-COUNTS = [1, 15, 16, 17, 63, 64, 65, 129, 0]
-FEW = [1, 4, 15, 16, 17, 33, 0, 8]  # up to 16 an expert on average: tiles of 32
+COUNTS = [1, 31, 32, 33, 63, 64, 65, 129, 0]
+FEW = [1, 4, 31, 32, 33, 9, 0, 8]  # up to 16 an expert on average: tiles of 32
 
 
 @pytest.fixture(scope="module")
