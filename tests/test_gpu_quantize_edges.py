@@ -1,4 +1,5 @@
-"""The Q4_K weight quantizer against the CPU oracle, bit for bit, where its
+"""The dequantizers into outputs aligned to their element alone, and the Q4_K
+weight quantizer against the CPU oracle, bit for bit, where its
 work split can go wrong: superblock counts around a wave (8) and a workgroup
 (32), and values around its clamps and divisions (levels at exact halves,
 constant and zero sub-blocks, scales from subnormal to the top of f32,
@@ -43,3 +44,23 @@ def test_quantize_q4k_bits(name):
     got = L.QTensor.quantize(torch.from_numpy(x).cuda(), O.Q4K).data()
     with np.errstate(all="ignore"):
         assert np.array_equal(got, O.quantize(O.Q4K, x.ravel()))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("dt", [O.Q8_0, O.Q4K, O.Q6K, O.Q8K])
+def test_dequantize_unaligned_output(dt, f16):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import lloom_amd as L
+    from lloom_amd.lib import check, lib
+    from lloom_amd.quantized import _ctx, _stream
+
+    x = torch.from_numpy(_input("count9", np.random.default_rng(2))).cuda()
+    q = L.QTensor.quantize(x, dt)
+    want = q.dequantize_f16() if f16 else q.dequantize()
+    for off in (1, 2, 3):
+        y = torch.full((x.numel() + 8,), 7.0, dtype=want.dtype, device="cuda")
+        check(lib().lloom_hip_dequantize(_ctx(0), int(dt), q.storage.data_ptr(), x.numel(), y[off:].data_ptr(),
+                                         1 if f16 else 0, _stream(y)))
+        assert torch.equal(y[off:off + x.numel()], want.reshape(-1))
+        assert (y[:off] == 7).all() and (y[off + x.numel():] == 7).all()
