@@ -139,7 +139,8 @@ int lloom_hip_dequantize(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, i
  * CPU result.  x_dtype / y_dtype: F32 or F16 each.  F16 activations are
  * the CPU arm's matmul_t_f16 (mod.rs:722,761; k_quants.rs:2802-2835): x
  * widened to f32 exactly, then the f32 path; an F16 y is each f32 sum
- * rounded to nearest-even.  The conversions run in the workspace. */
+ * rounded to nearest-even.  Where a kernel does not convert by itself, the
+ * workspace holds the f32 copy. */
 int lloom_hip_qmatmul(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, int64_t n, int64_t k,
                       const void* x_dev, int x_dtype, int64_t m, void* y_dev, int y_dtype,
                       void* stream);
@@ -204,7 +205,10 @@ int lloom_hip_qmatmul_noalloc(lloom_hip_ctx* ctx, int ggml_type, const void* w_d
  * quantization, as on the CPU arm) against the exactly dequantized weights,
  * factored per 16-element run: scale * sum(q * x) - min * sum(x), the CPU
  * arm's dot of a dequantized row in another rounding order.  n_experts is at
- * most 4096 (LLOOM_HIP_ESHAPE beyond).  An id >= n_experts yields a zero plane
+ * most 4096 (LLOOM_HIP_ESHAPE beyond).  Calls with several planes an expert
+ * keep a converted copy of x in the workspace; where it cannot grow (a capture)
+ * another kernel serves the call, in another rounding order.  An id >=
+ * n_experts yields a zero plane
  * and LLOOM_HIP_EEXPERT from this call (it synchronizes the stream to read
  * the device flag) unless strict is 0, in which case the next
  * lloom_hip_ctx_sync reports it. */
