@@ -7,22 +7,35 @@
 //  1. k_moe_gemm_prep: one workgroup an expert collects the (b, t) planes
 //     routed to it and cuts them into tiles of up to 64; the others convert the
 //     activation rows, each once: x' = x * 2^s (one power of two a row, max
-//     |x'| in [2^13, 2^14): exact) as fp16 hi + lo (x' = hi + lo to about
-//     2^-22 relative), in the order the GEMM's operands want, and (Q4_K) the
-//     32-element sums of x' for the min term.
+//     |x'| in [2^13, 2^14): exact) as fp16 hi + lo / 2^13, in the order the
+//     GEMM's operands want, and (Q4_K) the 32-element sums of x' likewise.
 //  2. k_moe_gemm: one workgroup per (tile of planes, block of weight rows).
 //     Weights go from HBM to registers and are unpacked there, once per 64
 //     planes, into exact fp16 integers; activations stream through LDS.
 //
-// The arithmetic per superblock of 256:
+// The arithmetic per superblock of 256, the products of hi and of lo in sums of
+// their own (acc = acc_hi + acc_lo / 2^13):
 //   Q4_K  acc = sum (sc q) x'     (sc q <= 945: exact in fp16)
 //         out += d acc - dmin sum_j m_j X_j   (X_j: the sub-blocks' sums)
+//         Tiles of 32 planes take q - 8 for q and 8 d sc_j - dmin m_j for
+//         -dmin m_j (as an fp16 pair): their sums are of the result's own size
+//         and round less than those of the unsigned q, which nearly cancel.
 //   Q6_K  acc = sum (sc (q - 32)) x'; |sc (q - 32)| <= 4096 takes 12 bits,
 //         one more than fp16 has, so the weight is an fp16 pair hi + lo too
-//         (exact) and lo meets the activations' hi: a third MFMA (the fourth,
-//         lo lo, is below 2^-22 of the product)
+//         (exact) and lo meets the activations' hi: a third MFMA
 //         out += d acc
-// Every product is exact in f32 and only the sums round.
+// Every product is exact in f32 and only the sums round.  What an element of x
+// loses to its two halves is at most 2^-23 of it, or 2^-50 of its row's largest
+// element where that is more; Q6_K's fourth product, lo lo, is at most 2^-22 of
+// the whole one (and zero for the weights below 2048).  Error against 64 bits
+// (2-norm, standard normal x into k = 1280 .. 2048 and products of two normals
+// into k = 512 and 768; k_moe_lds and k_moe_mfma before / this):
+//   Q4_K  tiles of 32: SwiGLU 3.4e-7 (from 8 planes an expert 5.5e-7) / 2.0e-7,
+//         one weight 2.3e-7 (3.9e-7) / 1.3e-7; tiles of 64: 5.6e-7 / 4.8e-7 and
+//         3.9e-7 / 3.3e-7
+//   Q6_K  one weight 2.4e-7 / 1.4e-7
+// With hi and lo in one sum and lo unscaled it was 5.7e-7, 4.0e-7 and 1.7e-7,
+// and an element lost up to 2^-39 of its row's largest.
 #include "kernels.hpp"
 #include "kq_common.hpp"
 #include "kq_gemm.hpp"
@@ -36,24 +49,29 @@ typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
 typedef float gf16 __attribute__((ext_vector_type(16)));
 
+// x' = hi + lo / MG_LO.  |x'| < 2^14 leaves |x' - hi| <= 4, so lo stays below
+// 2^15, and it is a normal number wherever hi is one.
+constexpr float MG_LO = 8192.0f;
+constexpr float MG_SUM = 32.0f;  // the sums of 32 x' are stored / 32: below 2^14 too
 constexpr int MG_WAVES = 4;   // waves of a GEMM workgroup
 constexpr int MG_COLS = MG_WAVES * 32;  // weight rows of a workgroup (SwiGLU: half of each weight)
 
 // ---------------------------------------------------------- the workspace --
 // int hdr[16] ([1] tiles), then at 256-byte steps:
 // int4 tiles[] (expert, first place in sorted, planes), int sorted[planes],
-// float inv[rows] (2^-s), fp16 sums[rows][K/256][16] (hi, lo of the eight
-// sums / 32), and x' [rows][K/256][1 KB].
+// float inv[rows] (2^-s), fp16 sums[rows][K/256][2][hi, lo][4] (sub-block 4h +
+// i at [h][..][i], / 32), and x' [rows][K/256][1 KB].
 static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Planes of a tile, at most: 64, and 32 up to 16 planes an expert, where the
-// smaller LDS and register budget keeps four (Q6_K three) workgroups a CU
-// instead of two ([128, 768, 2048], T tokens top-8, 32 / 64 a tile: Q4_K T = 64
-// 46 / 53 us, 256 51 / 58, 512 74 / 68; Q6_K 64 81 / 92, 256 86 / 93, 512 126 /
-// 107; the Q4_K SwiGLU launch, whose 32 spill, 64 87 / 82, 256 98 / 88).
-static int mg_tile_rows(int type, int64_t E, int64_t planes, int mode) {
-    if (type == T_Q4K && mode == MOE_GLU) return 64;
-    return planes > 16 * (E < planes ? E : planes) ? 64 : 32;
+// smaller LDS and register budget keeps three workgroups a CU instead of two
+// (Q6_K SwiGLU: two).  [128, 768, 2048], T tokens top-8, us with tiles of 32 /
+// 64: Q4_K T = 64 45.8 / 47.2, 256 45.5 / 51.0, 512 65.4 / 63.3; its SwiGLU
+// launch 256 77 / 77, 512 114 / 102; Q6_K 64 66 / 71, 256 69 / 74, 512 104 /
+// 90.  Q4_K rows past 32768 elements, which f32 dots served before, stay with
+// the tiles of 32 and their smaller error.
+static int mg_tile_rows(int type, int64_t E, int64_t planes, int64_t k) {
+    return planes > 16 * (E < planes ? E : planes) && !(type == T_Q4K && k > 32768) ? 64 : 32;
 }
 
 struct MgLayout {
@@ -79,17 +97,20 @@ size_t moe_gemm_workspace_bytes(int64_t E, int64_t planes, int64_t rows, int64_t
 // Where this route is taken.  It can be: rows of whole superblocks, 32-bit
 // byte offsets into x' and into one expert's weights.  It is the faster one:
 // its time hardly depends on the planes while each active expert has one tile
-// (10 us at k = 256, 25 at 2048, then the weight stream), and k_moe_lds's
-// grows with planes * n * k.  Measured against k_moe_lds, us, [E, n, k]:
-//   Q4_K, planes an expert: [128, 768, 2048] 3 45 / 50, 4 45 / 60; [64, 1280,
-//     2048] 3 43 / 44, 6 44 / 72; [256, 512, 2048] 2 66 / 43, 4 68 / 80
-//   and planes * n: [32, 768, 2048] 98 K 28 / 23, 147 K 28 / 30; [60, 512,
-//     1024] 66 K 16 / 15, 98 K 17 / 16, 131 K 17 / 19
-//   Q6_K [128, 768, 2048] 3 79 / 70, 4 77 / 85; [32, 768, 2048] 98 K 36 / 33,
-//     147 K 36 / 42; [32, 2048, 768] 131 K 26 / 19, 197 K 26 / 27, 262 K 26 / 30;
-//     [8, 768, 2048] 8 planes an expert, 49 K 35 / 30, 12 and 74 K 38 / 44
-// With 8 planes an expert Q4_K comes here at any size (10 / 14 us at [8, 256,
-// 256], 27 / 53 at [8, 768, 2048] against the kernel that served it before).
+// (11 us at k = 256, 25 at 2048, then the weight stream), and k_moe_lds's
+// grows with planes * n * k.  Measured against k_moe_lds with random routing
+// and the weights in HBM, us for one weight, SwiGLU in brackets, [E, n, k]:
+//   Q4_K, planes an expert: [128, 768, 2048] 3.5 45 (77) / 53 (97); [64, 1280,
+//     2048] 3.5 43 (64) / 47 (83); and planes * n: [32, 2048, 768] 229 K 20 (28)
+//     / 18 (30), 262 K 20 (28) / 21 (35); [32, 768, 2048] 98 K 23 (31) / 21 (35),
+//     123 K 23 (32) / 29 (43)
+//   Q6_K [128, 768, 2048] 3 82 (146) / 74 (194), 4 81 (147) / 84 (233); [32,
+//     2048, 768] 4 28 (44) / 31 (71); [32, 768, 2048] 147 K 42 (57) / 42 (84);
+//     [8, 768, 2048] 8 planes an expert 34 (34) / 31 (41), 12 34 (34) / 41 (55)
+// Over E 8 .. 256, n 512 .. 2048, k 256 .. 4096 the rule is at most 1.11 (Q4_K)
+// and 1.19 (Q6_K, [8, 768, 4096] with 12 planes an expert) of the better one.
+// With 8 planes an expert Q4_K comes here at any size (11 / 14 us at [8, 256,
+// 256], 21 / 53 at [8, 768, 2048] against k_moe_mfma).
 bool moe_gemm_fits(int type, int64_t E, int64_t planes, int64_t rows, int64_t n, int64_t k) {
     if ((type != T_Q4K && type != T_Q6K) || k % 256) return false;
     if (rows * k * 4 >= ((int64_t)1 << 32) || n * (k / 256) * block_bytes(type) >= ((int64_t)1 << 31)) return false;
@@ -223,7 +244,8 @@ __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict_
     const bool fin = mx > 0.0f && mx <= 3.4028234e38f;
     int ex = 0;
     if (fin) (void)frexpf(mx, &ex);
-    // max |x'| in [2^13, 2^14); 2^s and 2^-s stay normal numbers
+    // max |x'| in [2^13, 2^14); 2^s and 2^-s stay normal numbers (a row of
+    // subnormals comes out smaller, its last bit 2^-23: still exact)
     const int sh = fin ? max(-126, min(126, 14 - ex)) : 0;
     const float sc = ldexpf(1.0f, sh);
     if (lane == 0) inv[row] = ldexpf(1.0f, -sh);
@@ -240,7 +262,7 @@ __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict_
             const int at = TYPE == T_Q4K && (u & 3) % 3 ? u ^ 3 : u;
             const _Float16 h = (_Float16)v[u];
             hi[at] = h;
-            lo[at] = (_Float16)(v[u] - (float)h);
+            lo[at] = (_Float16)((v[u] - (float)h) * MG_LO);
             sum += v[u];
         }
         const int sb = i >> 5, G = i & 31;
@@ -254,10 +276,11 @@ __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict_
             sum += dpp<DPP_XOR1>(sum);
             sum += dpp<DPP_XOR2>(sum);
             if ((G & 3) == 0) {
-                const float s32 = sum * 0.03125f;
+                const float s32 = sum * (1.0f / MG_SUM);
                 const _Float16 h = (_Float16)s32;
-                sm[sb * 16 + (G >> 2)] = h;
-                sm[sb * 16 + 8 + (G >> 2)] = (_Float16)(s32 - (float)h);
+                _Float16* sj = sm + sb * 16 + (G >> 4) * 8 + ((G >> 2) & 3);
+                sj[0] = h;
+                sj[4] = (_Float16)((s32 - (float)h) * MG_LO);
             }
         }
     }
@@ -304,6 +327,17 @@ __device__ __forceinline__ gh2 bytes_h2(uint32_t w) {
     return as_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) + both((_Float16)-1024.0f);
 }
 
+// Scales (mins) of sub-blocks 4h .. 4h + 3, a byte each: 0-3 are the low six
+// bits of hdr.y (hdr.z), 4-7 the low (high) nibbles of hdr.w under its top bits.
+__device__ __forceinline__ uint32_t q4k_scales4(const uint4& hdr, int h) {
+    const uint32_t lo = hdr.y & 0x3F3F3F3Fu, hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+    return h ? hi : lo;
+}
+__device__ __forceinline__ uint32_t q4k_mins4(const uint4& hdr, int h) {
+    const uint32_t lo = hdr.z & 0x3F3F3F3Fu, hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+    return h ? hi : lo;
+}
+
 // The scales of a lane's half superblock.
 template <int TYPE>
 struct MgS;
@@ -316,20 +350,18 @@ struct MgS<T_Q6K> {
     gh2 s[2][2];  // [32-byte chunk][low, high nibbles]{bytes 0-15, 16-31}
 };
 
-template <int TYPE>
+template <int TYPE, bool MID>
 __device__ __forceinline__ void mg_scales(const MgW<TYPE>& w, int h, MgS<TYPE>& c) {
     if constexpr (TYPE == T_Q4K) {
-        // sub-blocks 4h .. 4h + 3: scales 0-3 are bytes of hdr.y, 4-7 the low
-        // nibbles of hdr.w under hdr.y's top bits.
-        // (1024 + q) sc - 1024 sc, and for a high nibble left in place
-        // (1024 + 16 q) (sc / 16) - 64 sc: both are sc q, exact
-        const uint32_t lo = w.hdr.y & 0x3F3F3F3Fu, hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
-        const uint32_t v = h ? hi : lo;
+        // MID: (64 + q) sc - 72 sc = (q - 8) sc.  Else (1024 + q) sc - 1024 sc,
+        // and for a high nibble left in place (1024 + 16 q) (sc / 16) - 64 sc:
+        // both q sc.  All of it exact.
+        const uint32_t v = q4k_scales4(w.hdr, h);
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const gh2 p = bytes_h2(v >> (16 * i));
-            c.s[i] = p * gh2{(_Float16)1.0f, (_Float16)0.0625f};
-            c.o[i] = p * gh2{(_Float16)-1024.0f, (_Float16)-64.0f};
+            c.s[i] = MID ? p : p * gh2{(_Float16)1.0f, (_Float16)0.0625f};
+            c.o[i] = MID ? p * both((_Float16)-72.0f) : p * gh2{(_Float16)-1024.0f, (_Float16)-64.0f};
         }
     } else {
         // element 128h + 32q + l has scale sc[8h + 2q + l / 16]
@@ -343,27 +375,28 @@ __device__ __forceinline__ void mg_scales(const MgW<TYPE>& w, int h, MgS<TYPE>& 
     }
 }
 
-// (v & mask) | 0x64006400: two values of v under the exponent of 1024.  With
-// both constants in registers it is one instruction; left alone the compiler
-// takes two (and, or), each with a literal.
-__device__ __forceinline__ gh2 and_1024(uint32_t v, uint32_t mask, uint32_t k64) {
+// (v & mask) | base: two nibbles of v under the exponent of 1024 or, four bits
+// higher, of 64.  With both constants in registers it is one instruction; left
+// alone the compiler takes two (and, or), each with a literal.
+constexpr uint32_t MG_1024 = 0x64006400u, MG_64 = 0x54005400u;
+__device__ __forceinline__ gh2 and_or(uint32_t v, uint32_t mask, uint32_t base) {
     uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(k64));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(base));
     return as_h2(r);
 }
 
 // The B operand(s) of step t (compile-time): eight weights of the lane.
-template <int TYPE>
-__device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c, int t, uint32_t k64, gh8& bh, gh8& bl) {
+template <int TYPE, bool MID>
+__device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c, int t, uint32_t base, gh8& bh, gh8& bl) {
     const int nib = t & 1, g = t >> 1, chunk = g >> 2;  // byte group g of 8: bytes 8g .. 8g + 7 of the lane's 64
     uint32_t r[4], l[4];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const uint32_t v = dword_of(w.q[g >> 1], 2 * (g & 1) + i);
         if constexpr (TYPE == T_Q4K) {
-            const uint32_t mask = nib ? 0x00F000F0u : 0x000F000Fu;
             const gh2 sc = both(c.s[chunk][nib]), of = both(c.o[chunk][nib]);
-            const gh2 e = and_1024(v, mask, k64), o = and_1024(v >> 8, mask, k64);
+            const uint32_t mask = MID || nib ? 0x00F000F0u : 0x000F000Fu;
+            const gh2 e = and_or(MID && !nib ? v << 4 : v, mask, base), o = and_or(MID && !nib ? v >> 4 : v >> 8, mask, base);
             r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, sc, of));
             r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(o, sc, of));
         } else {
@@ -385,6 +418,41 @@ __device__ __forceinline__ void mg_unpack(const MgW<TYPE>& w, const MgS<TYPE>& c
     }
     bh = __builtin_bit_cast(gh8, make_uint4(r[0], r[1], r[2], r[3]));
     if constexpr (TYPE == T_Q6K) bl = __builtin_bit_cast(gh8, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// The B operands that meet the sums of x' (MFMA k 8h + i: the hi of sub-block
+// 4h + i for i < 4, then the lo), and their scale: d, cs and ch (with MID, cl
+// too) such that the superblock adds d acc + cs (sums . (ch + cl)).
+template <bool MID>
+__device__ __forceinline__ void mg_mins(const uint4& hdr, int h, float& d, float& cs, gh8& ch, gh8& cl) {
+    d = f16_to_f32(hdr.x & 0xffffu);
+    const float dmin = f16_to_f32(hdr.x >> 16);
+    const gh2 il = both((_Float16)(1.0f / MG_LO));
+    const uint32_t mv = q4k_mins4(hdr, h);
+    if constexpr (!MID) {
+        cs = -MG_SUM * dmin;
+        const gh2 m0 = bytes_h2(mv), m1 = bytes_h2(mv >> 16), l0 = m0 * il, l1 = m1 * il;
+        ch = gh8{m0[0], m0[1], m1[0], m1[1], l0[0], l0[1], l1[0], l1[1]};
+    } else {
+        // c = 8 d sc - dmin m, rounded once, times a power of two that brings
+        // the larger of 8 d and dmin into [2^7, 2^8): |c| < 2^15
+        const float d8 = 8.0f * d;
+        const int ex = 8 - __builtin_amdgcn_frexp_expf(fmaxf(fabsf(d8), fabsf(dmin)));
+        const float ds = ldexpf(d8, ex), ms = ldexpf(dmin, ex);
+        cs = ldexpf(MG_SUM, -ex);
+        const uint32_t sv = q4k_scales4(hdr, h);
+        gh2 hi[2], lo[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float a = __builtin_fmaf(ds, (float)byte_of(sv, 2 * i), -(ms * (float)byte_of(mv, 2 * i)));
+            const float b = __builtin_fmaf(ds, (float)byte_of(sv, 2 * i + 1), -(ms * (float)byte_of(mv, 2 * i + 1)));
+            hi[i] = gh2{(_Float16)a, (_Float16)b};
+            lo[i] = gh2{(_Float16)(a - (float)hi[i][0]), (_Float16)(b - (float)hi[i][1])};
+        }
+        const gh2 h0 = hi[0] * il, h1 = hi[1] * il, l0 = lo[0] * il, l1 = lo[1] * il;
+        ch = gh8{hi[0][0], hi[0][1], hi[1][0], hi[1][1], h0[0], h0[1], h1[0], h1[1]};
+        cl = gh8{lo[0][0], lo[0][1], lo[1][0], lo[1][1], l0[0], l0[1], l1[0], l1[1]};
+    }
 }
 
 // LDS of a workgroup: two stages of half a superblock, two of the sums
@@ -450,7 +518,7 @@ __device__ __forceinline__ int mg_key(int r) { return (r >> 1) & 7; }
 // While a stage is computed, the next one's DMAs and the next superblock's
 // weight loads are in flight; a stage starts with one counted wait and one
 // barrier.  Rows past np hold whatever LDS held: their sums are not stored.
-template <int TYPE, int ROWS, int MT, bool GLU>
+template <int TYPE, int ROWS, int MT, bool GLU, bool MID>
 __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y,
                                         uint8_t* smem, const int* s_plane, const int* s_row, const float* s_inv) {
     constexpr int STAGE = mg_stage(ROWS);
@@ -492,7 +560,7 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
     const uint32_t a0 = (uint32_t)((c32 >> 3) * 4096 + (c32 & 7) * 128 + ((h ^ mg_key(c32)) * 16));
     const uint8_t* ap[4] = {smem + a0, smem + (a0 ^ 32u), smem + (a0 ^ 64u), smem + (a0 ^ 96u)};
 
-    gf16 out[MT], acc[MT];
+    gf16 out[MT], acc[MT], acl[MT];
     const gf16 z = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int T = 0; T < MT; T++) out[T] = z;
@@ -503,8 +571,8 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
     gh8 ah[MT], al[MT], bh[2], bl[2];
     MgW<TYPE> w, nxt;
     MgS<TYPE> sc;
-    uint32_t k64 = 0x64006400u;
-    asm("" : "+v"(k64));
+    uint32_t base = MID ? MG_64 : MG_1024;
+    asm("" : "+v"(base));
     auto read_a = [&](int t, int lo, gh8(&a)[MT]) {
         const uint8_t* p = ap[t & 3] + (t >> 3) * STAGE + lo * 2048 + ((t >> 2) & 1) * 1024;
 #pragma unroll
@@ -516,7 +584,7 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
         // use then finds nothing younger in flight
         w = nxt;
         mg_keep(w);
-        mg_scales<TYPE>(w, h, sc);
+        mg_scales<TYPE, MID>(w, h, sc);
     };
     load_w(0, nxt);
     issue(0, 0);
@@ -526,10 +594,10 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
     issue(0, 1);
     load_w(min(1, nsb - 1), nxt);
     read_a(0, 1, al);
-    mg_unpack<TYPE>(w, sc, 0, k64, bh[0], bl[0]);
+    mg_unpack<TYPE, MID>(w, sc, 0, base, bh[0], bl[0]);
     for (int sb = 0; sb < nsb; sb++) {
-        float d, dm32 = 0.0f;
-        gh8 bm, am[MT];
+        float d, cs;
+        gh8 am[MT], ch, cl;
         const bool last = sb + 1 == nsb;
 #pragma unroll
         for (int t = 0; t < 16; t++) {
@@ -537,9 +605,9 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
             read_a(t, 0, ah);
 #pragma unroll
             for (int T = 0; T < MT; T++)
-                acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[T], bh[cur], t ? acc[T] : z, 0, 0, 0);
+                acl[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[T], bh[cur], t ? acl[T] : z, 0, 0, 0);
             if (t < 15) {
-                mg_unpack<TYPE>(w, sc, t + 1, k64, bh[cur ^ 1], bl[cur ^ 1]);
+                mg_unpack<TYPE, MID>(w, sc, t + 1, base, bh[cur ^ 1], bl[cur ^ 1]);
                 mg_sched<TYPE, MT>(MT);
             }
             if (t == 7) {
@@ -557,13 +625,7 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
             } else {
                 // the epilogue's operands, before w moves on
                 if constexpr (TYPE == T_Q4K) {
-                    const uint4 hd = w.hdr;
-                    d = f16_to_f32(hd.x & 0xffffu);
-                    dm32 = 32.0f * f16_to_f32(hd.x >> 16);
-                    const uint32_t ml = hd.z & 0x3F3F3F3Fu,
-                                   mh = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
-                    const gh2 m0 = bytes_h2(ml), m1 = bytes_h2(ml >> 16), m2 = bytes_h2(mh), m3 = bytes_h2(mh >> 16);
-                    bm = gh8{m0[0], m0[1], m1[0], m1[1], m2[0], m2[1], m3[0], m3[1]};
+                    mg_mins<MID>(w.hdr, h, d, cs, ch, cl);
                     const uint8_t* sp = smem + 2 * STAGE + (sb & 1) * (ROWS * 32) + c32 * 32 + h * 16;
 #pragma unroll
                     for (int T = 0; T < MT; T++) am[T] = *(const gh8*)(sp + T * 1024);
@@ -576,32 +638,32 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
                     issue(sb + 1, 1);
                     load_w(min(sb + 2, nsb - 1), nxt);
                     read_a(0, 1, al);
-                    mg_unpack<TYPE>(w, sc, 0, k64, bh[0], bl[0]);
+                    mg_unpack<TYPE, MID>(w, sc, 0, base, bh[0], bl[0]);
                 }
             }
             if constexpr (TYPE == T_Q6K) {
 #pragma unroll
                 for (int T = 0; T < MT; T++)
-                    acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bl[cur], acc[T], 0, 0, 0);
+                    acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bl[cur], t ? acc[T] : z, 0, 0, 0);
             }
 #pragma unroll
             for (int T = 0; T < MT; T++)
-                acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bh[cur], acc[T], 0, 0, 0);
+                acc[T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[T], bh[cur], TYPE == T_Q6K || t ? acc[T] : z, 0, 0, 0);
             if (t != 15) mg_sched<TYPE, MT>((TYPE == T_Q6K ? 2 : 1) * MT);
         }
-        // the superblock's scales (and the min term: K 0..7 the sums' hi,
-        // 8..15 their lo, both against the mins)
+        // the superblock's scale, and (Q4_K) what the sums of x' contribute
 #pragma unroll
         for (int T = 0; T < MT; T++) {
             if constexpr (TYPE == T_Q4K) {
-                const gf16 mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[T], bm, z, 0, 0, 0);
+                gf16 mt = z;
+                if constexpr (MID) mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[T], cl, mt, 0, 0, 0);
+                mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[T], ch, mt, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 16; i++)
-                    out[T][i] = __builtin_fmaf(d, acc[T][i], __builtin_fmaf(-dm32, mt[i], out[T][i]));
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; i++) out[T][i] = __builtin_fmaf(d, acc[T][i], out[T][i]);
+                for (int i = 0; i < 16; i++) out[T][i] = __builtin_fmaf(cs, mt[i], out[T][i]);
             }
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                out[T][i] = __builtin_fmaf(d, __builtin_fmaf(acl[T][i], 1.0f / MG_LO, acc[T][i]), out[T][i]);
         }
     }
 #pragma unroll
@@ -632,8 +694,8 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
 }
 
 // What bounds it: [128, 768, 2048] Q4_K, 2000 tokens top-8, the SwiGLU launch
-// (two weights, 201 GFLOP of hi and lo products) takes 273 us with its prep
-// (0.74 PFLOP/s; 301 on 16x16x32 MFMAs, whose twice as many issue slots left
+// (two weights, 201 GFLOP of hi and lo products) takes 267 us with its prep
+// (0.75 PFLOP/s; 261 with hi and lo in one sum; 301 on 16x16x32 MFMAs, whose twice as many issue slots left
 // less room for the unpacking).  On that earlier form, only the loads (no MFMA,
 // no unpacking) took 273, only the arithmetic 246: a superblock's two L2 round
 // trips and its arithmetic hide each other only in part at two workgroups a CU.
@@ -646,9 +708,10 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
 // of one tile, which read the same activations, and the tiles of one expert,
 // which read the same weights, meet in one XCD's L2.
 template <int TYPE, int ROWS, bool GLU>
-__global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 4 : 3) void k_moe_gemm(
+__global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 || (GLU && TYPE == T_Q6K) ? 2 : 3) void k_moe_gemm(
     MgArgs A, const int* __restrict__ hdr, const int4* __restrict__ tiles, const int* __restrict__ sorted,
     const float* __restrict__ inv, int nblk, int pair) {
+    constexpr bool MID = TYPE == T_Q4K && ROWS == 32;
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ int s_plane[ROWS], s_row[ROWS];
     __shared__ float s_inv[ROWS];
@@ -673,18 +736,18 @@ __global__ __launch_bounds__(64 * MG_WAVES, ROWS == 64 ? 2 : TYPE == T_Q4K ? 4 :
     const int col0 = blk * (GLU ? MG_COLS / 2 : MG_COLS);
     if constexpr (ROWS == 64) {
         if (np > 32) {  // uniform
-            mg_tile<TYPE, ROWS, 2, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
+            mg_tile<TYPE, ROWS, 2, GLU, MID>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
             return;
         }
     }
-    mg_tile<TYPE, ROWS, 1, GLU>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
+    mg_tile<TYPE, ROWS, 1, GLU, MID>(A, np, col0, W0, W1, Y, smem, s_plane, s_row, s_inv);
 }
 
 template <int TYPE>
 static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     const int64_t planes = c.batch * c.topk, rows = c.in_dim1 == 1 ? c.batch : planes;
     const MgLayout l = mg_layout(c.E, planes, rows, c.k);
-    const int tile_rows = mg_tile_rows(TYPE, c.E, planes, c.mode);
+    const int tile_rows = mg_tile_rows(TYPE, c.E, planes, c.k);
     uint8_t* ws = (uint8_t*)c.ws;
     int* hdr = (int*)ws;
     int4* tiles = (int4*)(ws + l.tiles);

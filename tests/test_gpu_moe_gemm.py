@@ -8,10 +8,13 @@ workgroup's 128 (64 for the SwiGLU), one superblock a row, activations one
 row a token and one a slot, tiles of 32 planes and of 64, an out-of-range id,
 and a capture whose workspace holds only the routing.
 
-The bound: a product enters as an exact weight against x' = hi + lo, off by
-at most 2^-22 of it (Q6_K drops lo * lo, 2^-22 more), and a row is summed in
-f32 in fewer than K / 8 steps, so |err| <= (2^-21 + K / 8 * 2^-24) * S with
-S = sum |x| (|d sc q| + |dmin m|) <= 3 max|w| sum |x|.
+The bound: an element of x loses at most 2^-23 of itself, or 2^-50 of its row's
+largest element, to its two halves; Q6_K drops lo * lo, 2^-22 of the product,
+and Q4_K's pair of a sub-block's coefficient holds 2^-22; a row is summed in f32
+in fewer than K / 8 steps.  So |err| <= (2^-21 + K / 8 * 2^-24) * S + 2^-49 *
+max|x| * W, with the sub-blocks' S = sum |x| (|d sc q| + |dmin m|) <= 3 max|w|
+sum |x| and W the same for |x| = 1: what an element's own weight is zero for
+never enters.
 """
 import numpy as np
 import pytest
@@ -55,8 +58,41 @@ def _want(dt, q, E, n, k, x, ids):
     for e in range(E):
         at = ids == e
         want[at] = xs[at] @ dense[e].T
-        tol[at] = 3 * np.abs(xs[at]).sum(1, keepdims=True) * np.abs(dense[e]).max(1)[None]
-    return want, tol * (2.0 ** -21 + k / 8 * 2.0 ** -24)
+        top = np.abs(dense[e]).reshape(n, k // 32, 32).max(2)
+        xa = np.abs(xs[at])
+        tol[at] = 3 * (2.0 ** -21 + k / 8 * 2.0 ** -24) * (xa.reshape(-1, k // 32, 32).sum(2) @ top.T) \
+            + 3 * 2.0 ** -49 * xa.max(1, keepdims=True) * (32 * top.sum(1))
+    return want, tol
+
+
+def _on_small_context(q, x, ids, call="one", q2=None, mib=1):
+    """The call captured on a context that holds `mib` MiB of workspace: the
+    kernels that need no copy of x serve it.  The result of one replay."""
+    import ctypes
+
+    from lloom_amd.lib import check, lib
+    from lloom_amd.quantized import _ptr, _stream
+
+    (E, n, k), (batch, in_dim1, _), topk = q.shape, x.shape, ids.shape[1]
+    y = torch.zeros(batch, topk, n, device="cuda")
+    ctx = ctypes.c_void_p()
+    check(lib().lloom_hip_ctx_create(0, ctypes.byref(ctx)))
+    check(lib().lloom_hip_ctx_reserve(ctx, mib << 20))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if call == "one":
+            check(lib().lloom_hip_moe_matmul(ctx, int(q.dtype), _ptr(q.storage), E, n, k, _ptr(x), batch, in_dim1,
+                                             _ptr(ids), topk, _ptr(y), 0, _stream(x)))
+        else:
+            check(lib().lloom_hip_moe_matmul_glu(ctx, int(q.dtype), _ptr(q.storage), _ptr(q2.storage), E, n, k,
+                                                 _ptr(x), batch, in_dim1, _ptr(ids), topk, _ptr(y), 0, _stream(x)))
+    for _ in range(2):  # the second replay counts
+        y.zero_()
+        graph.replay()
+    got = y.cpu().numpy()
+    del graph
+    lib().lloom_hip_ctx_destroy(ctx)
+    return got
 
 
 @pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
@@ -109,6 +145,43 @@ def test_moe_gemm_bad_id_and_nonfinite(L):
     assert not np.isfinite(y[5]).any()
     keep = np.arange(40) != 5
     assert (np.abs(y - want) <= tol)[keep].all()
+
+
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+@pytest.mark.parametrize("counts", [[40, 33, 64, 130], [12, 13, 9, 30]], ids=["64", "32"])
+@pytest.mark.parametrize("bits", [0, 20, 26])
+def test_moe_gemm_small_beside_outlier(L, dt, counts, bits):
+    """An element 2^bits larger than the rest meets weights that are zero: the
+    others keep their precision (f32 dots lose nothing to it either)."""
+    rng = np.random.default_rng(bits)
+    E, n, k = len(counts), 3100, 768
+    w = (rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)
+    w[..., 32:64] = w[..., 512:544] = 0
+    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), dt)
+    ids = np.repeat(np.arange(E), counts).astype(np.int32)[:, None]
+    x = rng.standard_normal((len(ids), 1, k)).astype(np.float32)
+    x[..., 37] *= 2.0 ** bits
+    x[::2, ..., 513] *= -(2.0 ** bits)
+    want, tol = _want(dt, q.data(), E, n, k, x, ids)
+    got = q.indexed_moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()).cpu().numpy()
+    assert (np.abs(got - want) <= tol).all(), (np.abs(got - want) / tol).max()
+
+
+@pytest.mark.parametrize("dt,E,n,k,per", [(O.Q4K, 64, 416, 2048, 5), (O.Q4K, 64, 512, 768, 7),
+                                          (O.Q6K, 64, 640, 2048, 5), (O.Q6K, 64, 512, 768, 14), (O.Q6K, 16, 320, 2048, 40)])
+def test_moe_gemm_no_further_off_than_the_other_kernels(L, dt, E, n, k, per):
+    """Against 64 bits (2-norm), the grouped GEMM is no further off than what
+    serves the same call without a copy of x (f32 dots below 8 planes an expert
+    and for Q6_K)."""
+    rng = np.random.default_rng(per)
+    q = L.QTensor.quantize(torch.from_numpy((rng.standard_normal((E, n, k)) * 0.02).astype(np.float32)).cuda(), dt)
+    ids = rng.integers(0, E, (E * per, 1)).astype(np.int32)
+    x = (rng.standard_normal((E * per, 1, k)) * rng.standard_normal((E * per, 1, k))).astype(np.float32)
+    xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    want, _ = _want(dt, q.data(), E, n, k, x, ids)
+    off = [np.linalg.norm(y - want) / np.linalg.norm(want)
+           for y in (q.indexed_moe_forward(xd, idd).cpu().numpy(), _on_small_context(q, xd, idd))]
+    assert off[0] <= off[1], off
 
 
 def test_moe_gemm_captured(L):
