@@ -170,7 +170,8 @@ int lloom_hip_qmatmul_workspace_bytes(lloom_hip_ctx* ctx, int ggml_type, int64_t
                                       int x_dtype, int y_dtype, size_t* bytes);
 /* Grow the context workspace to at least `bytes` now.  A call that would
  * grow it while its stream is being captured fails with LLOOM_HIP_ENOMEM
- * instead; outgrown workspaces stay allocated until lloom_hip_ctx_destroy
+ * instead (a routed call that could use more than it needs takes a slower
+ * kernel); outgrown workspaces stay allocated until lloom_hip_ctx_destroy
  * (graphs captured earlier keep using theirs). */
 int lloom_hip_ctx_reserve(lloom_hip_ctx* ctx, size_t bytes);
 /* Bytes the context workspace holds now. */
@@ -201,21 +202,32 @@ int lloom_hip_qmatmul_noalloc(lloom_hip_ctx* ctx, int ggml_type, const void* w_d
  * matmul_t_indexed (mod.rs:766-810): W [n_experts, n, k] packed, x f32
  * [batch, in_dim1, k] with in_dim1 in {1, topk}, ids u32 [batch, topk],
  * y f32 [batch, topk, n]; plane (b, t) = x[b, t or 0] . W[ids[b, t]]^T.
- * The dots take the f32 activations as they are (no activation
- * quantization, as on the CPU arm) against the exactly dequantized weights,
- * factored per 16-element run: scale * sum(q * x) - min * sum(x), the CPU
- * arm's dot of a dequantized row in another rounding order.  n_experts is at
- * most 4096 (LLOOM_HIP_ESHAPE beyond).  Calls with several planes an expert
- * keep a converted copy of x in the workspace; where it cannot grow (a capture)
- * another kernel serves the call, in another rounding order.  An id >=
- * n_experts yields a zero plane
- * and LLOOM_HIP_EEXPERT from this call (it synchronizes the stream to read
- * the device flag) unless strict is 0, in which case the next
- * lloom_hip_ctx_sync reports it. */
+ * The activations are not quantized (as on the CPU arm) and the weights are
+ * exactly dequantized; sums are f32, in another order than the CPU arm's dot of
+ * a dequantized row.  With few planes an expert the dots take x as it is,
+ * factored per 16-element run: scale * sum(q * x) - min * sum(x).  With more, x
+ * goes to the matrix cores as two fp16 halves a value, exact to 2^-23 of it (or
+ * 2^-50 of its row's largest element, where that is more), and the result is
+ * no further from the exact one than the f32 dots' (the decode form with 1.75
+ * to 2.5 planes an expert: to 2^-22).  n_experts is at most 4096
+ * (LLOOM_HIP_ESHAPE beyond).  Calls with several planes an expert keep the
+ * halves of x in the workspace.  Where it cannot grow (a capture, or no memory)
+ * a slower kernel that needs only the routing serves the call, in another
+ * rounding order (Q4_K with 8 planes an expert: halves exact to 2^-22 of an
+ * element or 2^-39 of its row's largest): a caller that captures reserves
+ * lloom_hip_moe_workspace_bytes first and gets the eager call's kernel and bits.
+ * An id >= n_experts yields a zero plane and LLOOM_HIP_EEXPERT from this call
+ * (it synchronizes the stream to read the flag) unless strict is 0, in which
+ * case the next lloom_hip_ctx_sync reports it. */
 int lloom_hip_moe_matmul(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, int64_t n_experts,
                          int64_t n, int64_t k, const float* x_dev, int64_t batch, int64_t in_dim1,
                          const uint32_t* ids_dev, int64_t topk, float* y_dev, int strict,
                          void* stream);
+
+/* Workspace a routed call (one weight, pair or SwiGLU) of this shape takes, so
+ * a caller can reserve it before capturing the call into a graph. */
+int lloom_hip_moe_workspace_bytes(int ggml_type, int64_t n_experts, int64_t n, int64_t k, int64_t batch,
+                                  int64_t in_dim1, int64_t topk, size_t* bytes);
 
 /* Gate and up of one routed layer in one launch: QTensor::
  * indexed_moe_forward_pair (mod.rs:1365-1455; one Metal launch,

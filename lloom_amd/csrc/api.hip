@@ -65,27 +65,38 @@ static const char* type_name(int t) {
 // refused while `s` is being captured into a graph: an allocation there
 // would not be part of the graph, so the caller reserves the workspace first
 // (lloom_hip_ctx_reserve).
-static int ensure_ws(lloom_hip_ctx* ctx, size_t bytes, hipStream_t s, void** out) {
+enum WsState { WS_OK, WS_CAPTURING, WS_NO_MEMORY };
+static WsState try_ws(lloom_hip_ctx* ctx, size_t bytes, hipStream_t s, void** out) {
     if (bytes > ctx->ws_bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
-            return fail(LLOOM_HIP_ENOMEM,
-                        "the call needs a workspace of %zu bytes and the context holds %zu: it cannot grow while "
-                        "the stream is being captured (reserve it first with lloom_hip_ctx_reserve)",
-                        bytes, ctx->ws_bytes);
+        if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) return WS_CAPTURING;
         size_t want = bytes > 2 * ctx->ws_bytes ? bytes : 2 * ctx->ws_bytes;
         want = (want + 0xFFFFF) & ~(size_t)0xFFFFF;
         void* fresh = nullptr;
         if (hipMalloc(&fresh, want) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(LLOOM_HIP_ENOMEM, "workspace allocation of %zu bytes failed", want);
+            return WS_NO_MEMORY;
         }
         if (ctx->ws) ctx->retired.push_back(ctx->ws);
         ctx->ws = fresh;
         ctx->ws_bytes = want;
     }
     *out = ctx->ws;
-    return LLOOM_HIP_OK;
+    return WS_OK;
+}
+
+// The same, for a call that cannot do with less.
+static int ensure_ws(lloom_hip_ctx* ctx, size_t bytes, hipStream_t s, void** out) {
+    switch (try_ws(ctx, bytes, s, out)) {
+        case WS_OK: return LLOOM_HIP_OK;
+        case WS_CAPTURING:
+            return fail(LLOOM_HIP_ENOMEM,
+                        "the call needs a workspace of %zu bytes and the context holds %zu: it cannot grow while "
+                        "the stream is being captured (reserve it first with lloom_hip_ctx_reserve)",
+                        bytes, ctx->ws_bytes);
+        case WS_NO_MEMORY: break;
+    }
+    return fail(LLOOM_HIP_ENOMEM, "workspace allocation for %zu bytes failed", bytes);
 }
 
 extern "C" {
@@ -439,13 +450,9 @@ static int strict_bad(lloom_hip_ctx* ctx, hipStream_t s, bool* bad) {
     return LLOOM_HIP_OK;
 }
 
-static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const void* w2_dev, int64_t n_experts,
-                    int64_t n, int64_t k, const float* x_dev, int64_t batch, int64_t in_dim1,
-                    const uint32_t* ids_dev, int64_t topk, float* y_dev, float* y2_dev, int mode, int strict,
-                    void* stream) {
-    if (!ctx || !w_dev || !x_dev || !ids_dev || !y_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null argument");
-    if (mode != MOE_ONE && !w2_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null up weight");
-    if (mode == MOE_PAIR && !y2_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null up output");
+// A routed call's type and shapes.
+static int moe_check(int ggml_type, int64_t n_experts, int64_t n, int64_t k, int64_t batch, int64_t in_dim1,
+                     int64_t topk) {
     if (!is_weight_type(ggml_type))
         return fail(LLOOM_HIP_EDTYPE, "moe_matmul: weight dtype %s (%d) is not supported on the HIP quantized path", type_name(ggml_type), ggml_type);
     int be = block_elems(ggml_type);
@@ -459,6 +466,17 @@ static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const 
     if (n_experts > MOE_MAX_EXPERTS)
         return fail(LLOOM_HIP_ESHAPE, "moe_matmul: %lld experts, at most %d are routed on the device",
                     (long long)n_experts, MOE_MAX_EXPERTS);
+    return LLOOM_HIP_OK;
+}
+
+static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const void* w2_dev, int64_t n_experts,
+                    int64_t n, int64_t k, const float* x_dev, int64_t batch, int64_t in_dim1,
+                    const uint32_t* ids_dev, int64_t topk, float* y_dev, float* y2_dev, int mode, int strict,
+                    void* stream) {
+    if (!ctx || !w_dev || !x_dev || !ids_dev || !y_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null argument");
+    if (mode != MOE_ONE && !w2_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null up weight");
+    if (mode == MOE_PAIR && !y2_dev) return fail(LLOOM_HIP_EINVAL, "moe_matmul: null up output");
+    if (int rc = moe_check(ggml_type, n_experts, n, k, batch, in_dim1, topk)) return rc;
     if ((uintptr_t)w_dev % (ggml_type == T_Q4K ? 16 : 4) || (uintptr_t)x_dev % 16 ||
         (w2_dev && (uintptr_t)w2_dev % (ggml_type == T_Q4K ? 16 : 4)))
         return fail(LLOOM_HIP_EINVAL, "moe_matmul: misaligned weight or x pointer");
@@ -470,11 +488,10 @@ static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const 
     // cannot grow to hold it (a capture, or no memory), the kernels that need
     // the routing ints alone serve the call
     const int64_t rows = in_dim1 == 1 ? batch : batch * topk;
-    int rc = LLOOM_HIP_ENOMEM;
-    if (moe_gemm_fits(ggml_type, n_experts, batch * topk, rows, n, k))
-        rc = ensure_ws(ctx, moe_gemm_workspace_bytes(n_experts, batch * topk, rows, k), s, &ws);
-    if (rc) rc = ensure_ws(ctx, moe_workspace_bytes(n_experts, batch * topk, n, k, mode), s, &ws);
-    if (rc) return rc;
+    if (!moe_gemm_fits(ggml_type, n_experts, batch * topk, rows, n, k) ||
+        try_ws(ctx, moe_gemm_workspace_bytes(n_experts, batch * topk, rows, k), s, &ws) != WS_OK) {
+        if (int rc = ensure_ws(ctx, moe_workspace_bytes(n_experts, batch * topk, n, k, mode), s, &ws)) return rc;
+    }
     HIP_OK(launch_moe(ggml_type, w_dev, n_experts, n, k, x_dev, batch, in_dim1, ids_dev, topk, y_dev, (int*)ws,
                       ctx->ws_bytes, id_flags(ctx, strict), mode, w2_dev, y2_dev, s));
     if (strict) {
@@ -486,6 +503,20 @@ static int moe_impl(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, const 
 }
 
 extern "C" {
+
+int lloom_hip_moe_workspace_bytes(int ggml_type, int64_t n_experts, int64_t n, int64_t k, int64_t batch,
+                                  int64_t in_dim1, int64_t topk, size_t* bytes) {
+    if (!bytes) return fail(LLOOM_HIP_EINVAL, "moe_workspace_bytes: null output");
+    if (int rc = moe_check(ggml_type, n_experts, n, k, batch, in_dim1, topk)) return rc;
+    const int64_t planes = batch * topk, rows = in_dim1 == 1 ? batch : planes;
+    size_t need = moe_workspace_bytes(n_experts, planes, n, k, MOE_GLU);  // the largest of the three calls'
+    if (moe_gemm_fits(ggml_type, n_experts, planes, rows, n, k)) {
+        const size_t gemm = moe_gemm_workspace_bytes(n_experts, planes, rows, k);
+        if (gemm > need) need = gemm;
+    }
+    *bytes = need;
+    return LLOOM_HIP_OK;
+}
 
 int lloom_hip_moe_matmul(lloom_hip_ctx* ctx, int ggml_type, const void* w_dev, int64_t n_experts, int64_t n,
                          int64_t k, const float* x_dev, int64_t batch, int64_t in_dim1, const uint32_t* ids_dev,

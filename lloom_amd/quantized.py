@@ -144,6 +144,15 @@ def qmatmul_workspace_bytes(dtype, n, k, m, x_dtype=torch.float32, y_dtype=torch
     return out.value
 
 
+def moe_workspace_bytes(dtype, n_experts, n, k, batch, in_dim1, topk):
+    """The workspace any routed call of these shapes takes (reserve_workspace
+    it before a capture)."""
+    out = ctypes.c_size_t()
+    check(lib().lloom_hip_moe_workspace_bytes(int(GgmlDType(dtype)), n_experts, n, k, batch, in_dim1, topk,
+                                              ctypes.byref(out)))
+    return out.value
+
+
 def set_mv_rows_max(rows, device=0):
     check(lib().lloom_hip_ctx_set_mv_rows_max(_ctx(device), rows))
 

@@ -205,6 +205,17 @@ extern "C" {
         strict: c_int,
         stream: *mut c_void,
     ) -> c_int;
+    // No counterpart in the reference: the workspace a routed call of these shapes takes.
+    pub fn lloom_hip_moe_workspace_bytes(
+        ggml_type: c_int,
+        n_experts: i64,
+        n: i64,
+        k: i64,
+        batch: i64,
+        in_dim1: i64,
+        topk: i64,
+        bytes: *mut usize,
+    ) -> c_int;
     pub fn lloom_hip_moe_matmul_pair(
         ctx: *mut lloom_hip_ctx,
         ggml_type: c_int,

@@ -47,6 +47,27 @@ def test_weight_bytes_and_refusals():
     assert isinstance(lloom_amd.LloomHipError(3, "x"), RuntimeError)
 
 
+def test_moe_workspace_bytes():
+    """What a routed call takes: its routing lists, from several planes an
+    expert on also a copy of x; the refusals are the call's."""
+    from lloom_amd.lib import lib
+    from lloom_amd.quantized import moe_workspace_bytes
+
+    few = moe_workspace_bytes(12, 128, 768, 2048, 4, 1, 8)
+    assert 0 < few < 1 << 16
+    for dt, in_dim1, rows in ((12, 1, 512), (12, 8, 4096), (14, 8, 4096)):
+        need = moe_workspace_bytes(dt, 128, 768, 2048, 512, in_dim1, 8)
+        assert rows * 2048 * 4 < need < rows * 2048 * 4 * 1.05 + (1 << 17)
+    assert moe_workspace_bytes(8, 128, 768, 2048, 512, 1, 8) < 1 << 16  # Q8_0 keeps no copy
+    # rows too long to stage: a SwiGLU holds its up half
+    assert moe_workspace_bytes(8, 4, 512, 32768, 2, 1, 2) > 4 * 512 * 4
+    out = ctypes.c_size_t()
+    for args, code in (((7, 8, 64, 256, 1, 1, 2), 2), ((12, 8, 64, 100, 1, 1, 2), 3), ((12, 8, 64, 256, 1, 3, 2), 3),
+                       ((12, 5000, 64, 256, 1, 1, 2), 3), ((12, 0, 64, 256, 1, 1, 2), 1)):
+        assert lib().lloom_hip_moe_workspace_bytes(*args, ctypes.byref(out)) == code
+    assert lib().lloom_hip_moe_workspace_bytes(12, 8, 64, 256, 1, 1, 2, None) == 1
+
+
 def test_synth_is_deterministic_and_normal():
     import lloom_amd as L
 

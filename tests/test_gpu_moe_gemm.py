@@ -167,7 +167,7 @@ def test_moe_gemm_small_beside_outlier(L, dt, counts, bits):
     assert (np.abs(got - want) <= tol).all(), (np.abs(got - want) / tol).max()
 
 
-@pytest.mark.parametrize("dt,E,n,k,per", [(O.Q4K, 64, 416, 2048, 5), (O.Q4K, 64, 512, 768, 7),
+@pytest.mark.parametrize("dt,E,n,k,per", [(O.Q4K, 64, 416, 2048, 5), (O.Q4K, 64, 512, 768, 7), (O.Q4K, 16, 320, 2048, 40),
                                           (O.Q6K, 64, 640, 2048, 5), (O.Q6K, 64, 512, 768, 14), (O.Q6K, 16, 320, 2048, 40)])
 def test_moe_gemm_no_further_off_than_the_other_kernels(L, dt, E, n, k, per):
     """Against 64 bits (2-norm), the grouped GEMM is no further off than what
@@ -184,18 +184,16 @@ def test_moe_gemm_no_further_off_than_the_other_kernels(L, dt, E, n, k, per):
     assert off[0] <= off[1], off
 
 
-def test_moe_gemm_captured(L):
-    """Replays equal the eager call, and a capture on a context whose
-    workspace cannot hold the activations is served all the same."""
-    import ctypes
-
-    from lloom_amd.lib import check, lib
-    from lloom_amd.quantized import _ptr
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+def test_moe_gemm_captured(L, dt):
+    """Replays equal the eager call, on a context that reserved what the size
+    query says too."""
+    from lloom_amd.quantized import moe_workspace_bytes
 
     rng = np.random.default_rng(4)
-    E, n, k, batch, topk = 4, 96, 2048, 128, 4
+    E, n, k, batch, topk = 4, 400, 2048, 128, 4
     w = (rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)
-    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), O.Q4K)
+    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), dt)
     ids = torch.from_numpy(rng.integers(0, E, (batch, topk)).astype(np.int32)).cuda()
     x = torch.from_numpy(rng.standard_normal((batch, topk, k)).astype(np.float32)).cuda()
     eager = q.indexed_moe_forward(x, ids)
@@ -207,17 +205,32 @@ def test_moe_gemm_captured(L):
         y.zero_()
         graph.replay()
         assert torch.equal(y, eager)
-    ctx = ctypes.c_void_p()
-    check(lib().lloom_hip_ctx_create(0, ctypes.byref(ctx)))
-    check(lib().lloom_hip_ctx_reserve(ctx, 1 << 20))
-    small = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(small):
-        check(lib().lloom_hip_moe_matmul(ctx, O.Q4K, _ptr(q.storage), E, n, k, _ptr(x), batch, topk, _ptr(ids), topk,
-                                         _ptr(y), 0, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
-    want, tol = _want(O.Q4K, q.data(), E, n, k, x.cpu().numpy(), ids.cpu().numpy())
-    for _ in range(2):
-        y.zero_()
-        small.replay()
-        assert (np.abs(y.cpu().numpy() - want) <= tol).all()
-    del small
-    lib().lloom_hip_ctx_destroy(ctx)
+    need = moe_workspace_bytes(dt, E, n, k, batch, topk, topk)
+    assert np.array_equal(_on_small_context(q, x, ids, mib=(need + (1 << 20) - 1) >> 20), eager.cpu().numpy())
+
+
+@pytest.mark.parametrize("dt,E,n,k,topk,planes", [
+    (O.Q4K, 4, 400, 2048, 4, 512), (O.Q4K, 8, 200, 768, 4, 1600),  # 8 planes an expert: in-kernel and sorted routing
+    (O.Q4K, 160, 132, 512, 7, 1120), (O.Q6K, 4, 400, 2048, 4, 512), (O.Q6K, 64, 200, 512, 4, 1280)])
+@pytest.mark.parametrize("call", ["one", "glu"])
+def test_moe_captured_without_room_for_x(L, dt, E, n, k, topk, planes, call):
+    """A capture on a context whose workspace cannot hold the copy of x is
+    served all the same, leaves no error message, and replays right, in-kernel
+    routing (up to 1024 planes) and sorted."""
+    from lloom_amd.lib import lib
+
+    rng = np.random.default_rng(planes)
+    w = (rng.standard_normal((2, E, n, k)) * 0.05).astype(np.float32)
+    qg, qu = (L.QTensor.quantize(torch.from_numpy(v).cuda(), dt) for v in w)
+    ids = rng.integers(0, E, (planes // topk, topk)).astype(np.int32)
+    x = rng.standard_normal((planes // topk, topk, k)).astype(np.float32)
+    assert lib().lloom_hip_ctx_create(-1, None) and b"out is null" in lib().lloom_hip_last_error()
+    y = _on_small_context(qg, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), call, qu)
+    assert b"out is null" in lib().lloom_hip_last_error()
+    g, gtol = _want(dt, qg.data(), E, n, k, x, ids)
+    if call == "one":
+        assert (np.abs(y - g) <= gtol).all()
+        return
+    u, utol = _want(dt, qu.data(), E, n, k, x, ids)
+    silu = g / (1 + np.exp(-g))
+    assert (np.abs(y - silu * u) <= 1.1 * gtol * np.abs(u) + np.abs(silu) * utol + 2 * gtol * utol + 1e-6 * np.abs(silu * u)).all()
