@@ -147,6 +147,56 @@ def test_moe_gemm_bad_id_and_nonfinite(L):
     assert (np.abs(y - want) <= tol)[keep].all()
 
 
+def _us(f):
+    """The median time of a call among others, in microseconds."""
+    f()
+    torch.cuda.synchronize()
+    times = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(10):
+            f()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 100)
+    return sorted(times)[2]
+
+
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+def test_moe_gemm_many_bad_ids(L, dt):
+    """Half of the ids out of range, in every 64 planes: their outputs are zero
+    in each of the three calls, the others as without them, and such planes cost
+    no more than good ones."""
+    from lloom_amd.lib import lib
+    from lloom_amd.quantized import _ctx
+
+    rng = np.random.default_rng(8)
+    E, n, k, batch, topk = 5, 129, 512, 731, 4
+    w = (rng.standard_normal((2, E, n, k)) * 0.05).astype(np.float32)
+    qg, qu = (L.QTensor.quantize(torch.from_numpy(v).cuda(), dt) for v in w)
+    ids = torch.from_numpy(rng.integers(0, E, (batch, topk)).astype(np.int32)).cuda()
+    x = torch.from_numpy(rng.standard_normal((batch, 1, k)).astype(np.float32)).cuda()
+    out = torch.from_numpy(rng.random((batch, topk)) < 0.5).cuda()
+    bad = ids.clone()
+    bad[out] = torch.from_numpy(rng.choice([E, -1, 1 << 30], int(out.sum())).astype(np.int32)).cuda()
+    calls = [lambda i: [qg.indexed_moe_forward(x, i, strict=False)],
+             lambda i: qg.indexed_moe_forward_pair(qu, x, i, strict=False),
+             lambda i: [qg.indexed_moe_forward_glu_as(qu, x, i, strict=False)]]
+    for call in calls:
+        torch.full((2 * batch * topk * n,), 7.0, device="cuda")  # the outputs' memory held something else
+        for got, good in zip(call(bad), call(ids)):
+            assert not got[out].any()
+            assert torch.equal(got[~out], good[~out])
+    assert lib().lloom_hip_ctx_sync(_ctx(0)) == 4
+    q = L.QTensor.quantize(torch.randn(8, 768, 2048, device="cuda"), dt)
+    x, ids = torch.randn(4096, 1, 2048, device="cuda"), torch.arange(4096, device="cuda", dtype=torch.int32)[:, None] % 8
+    y = torch.empty(4096, 1, 768, device="cuda")
+    good, none = (_us(lambda i=i: q.indexed_moe_forward_into(x, i, y)) for i in (ids, ids + 8))
+    assert none < 3 * good, (none, good)
+    assert lib().lloom_hip_ctx_sync(_ctx(0)) == 4
+
+
 @pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
 @pytest.mark.parametrize("counts", [[40, 33, 64, 130], [12, 13, 9, 30]], ids=["64", "32"])
 @pytest.mark.parametrize("bits", [0, 20, 26])
