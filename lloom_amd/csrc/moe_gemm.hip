@@ -121,19 +121,25 @@ bool moe_gemm_fits(int type, int64_t E, int64_t planes, int64_t rows, int64_t n,
 
 // ------------------------------------------------------------------- prep --
 
-// Workgroup e collects the planes of expert e.  It counts every expert's
-// planes, so it knows by itself where its planes and tiles go and the
+// Workgroups that route, at most: each reads all ids, so past a CU's worth of
+// them more would only repeat that ([4096, 64, 256], 128 K planes: 365 us with one
+// an expert, 130 with these, 291 with k_moe_route and k_moe_mfma).
+constexpr int MG_ROUTERS = 256, MG_PER_MAX = (MOE_MAX_EXPERTS + MG_ROUTERS - 1) / MG_ROUTERS;
+
+// Workgroup r of R collects the planes of `per` experts.  It counts every
+// expert's planes, so it knows by itself where its planes and tiles go and the
 // workgroups need nothing of each other (one workgroup for all experts took
 // 17 us at 4096 planes, this 4).  The order inside an expert follows the LDS
 // atomics; every plane's dot is computed on its own, so no result depends on
 // it.
-__device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, int E, int* hdr, int4* tiles,
+__device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int r, int per, int E, int* hdr, int4* tiles,
                          int* sorted, IdFlags flags, float* y, float* y2, int n, int tile_rows) {
-    __shared__ int s_cnt[MOE_MAX_EXPERTS];
-    __shared__ int s_first, s_tile, s_tiles, s_at;
-    const int tid = threadIdx.x;
+    __shared__ int s_cnt[MOE_MAX_EXPERTS], s_at[MG_PER_MAX];
+    __shared__ int s_first, s_tile, s_tiles;
+    const int tid = threadIdx.x, lane = tid & 63, R = (E + per - 1) / per;
+    const int e0 = r * per, e1 = min(e0 + per, E);
     for (int i = tid; i < E; i += 1024) s_cnt[i] = 0;
-    if (tid == 0) s_first = s_tile = s_tiles = s_at = 0;
+    if (tid == 0) s_first = s_tile = s_tiles = 0;
     __syncthreads();
     int bad = 0;
     for (int p0 = tid; p0 < planes; p0 += 8 * 1024) {
@@ -153,8 +159,7 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
         // dealt to the workgroups' waves, which store a plane together (one
         // lane a plane, in one workgroup, took 1.8 ms for 4096 planes of 768
         // outputs, the call this way 45 us)
-        const int lane = tid & 63;
-        for (int64_t p = 64 * (e + E * (tid >> 6)); p < planes; p += 64 * 16 * E) {
+        for (int64_t p = 64 * (r + R * (tid >> 6)); p < planes; p += 64 * 16 * R) {
             const bool out = p + lane < planes && ids[p + lane] >= (uint32_t)E;
             for (uint64_t m = __ballot(out); m; m &= m - 1) {
                 const int64_t at = (p + __builtin_ctzll(m)) * n;
@@ -168,8 +173,8 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
     int first = 0, tile = 0, all = 0;  // planes and tiles of smaller experts, tiles of all
     for (int i = tid; i < E; i += 1024) {
         const int c = s_cnt[i], t = (c + tile_rows - 1) / tile_rows;
-        first += i < e ? c : 0;
-        tile += i < e ? t : 0;
+        first += i < e0 ? c : 0;
+        tile += i < e0 ? t : 0;
         all += t;
     }
 #pragma unroll
@@ -178,31 +183,40 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int e, in
         tile += __shfl_xor(tile, o, 64);
         all += __shfl_xor(all, o, 64);
     }
-    if ((tid & 63) == 0 && all) {
+    if (lane == 0 && all) {
         atomicAdd(&s_first, first);
         atomicAdd(&s_tile, tile);
         atomicAdd(&s_tiles, all);
     }
     __syncthreads();
-    if (tid == 0 && e == 0) {
+    if (tid == 0 && r == 0) {
         flags.call[0] = bad;            // this call: read back by a strict call
         if (bad) flags.sticky[0] = 1;  // until the next lloom_hip_ctx_sync
         hdr[1] = s_tiles;
     }
-    const int c = s_cnt[e];
-    if (c == 0) return;  // uniform
     first = s_first;
     tile = s_tile;
-    // the planes over as few tiles as hold them, each a multiple of 32
-    const int k = (c + tile_rows - 1) / tile_rows, rows = ((c + k - 1) / k + 31) & ~31;
-    for (int i = tid; i < k; i += 1024) tiles[tile + i] = make_int4(e, first + i * rows, min(rows, c - i * rows), 0);
+    const int none = first;
+    for (int e = e0; e < e1; e++) {
+        // the planes over as few tiles as hold them, each a multiple of 32
+        const int c = s_cnt[e], k = (c + tile_rows - 1) / tile_rows;
+        if (c) {
+            const int rows = ((c + k - 1) / k + 31) & ~31;
+            for (int i = tid; i < k; i += 1024) tiles[tile + i] = make_int4(e, first + i * rows, min(rows, c - i * rows), 0);
+        }
+        if (tid == 0) s_at[e - e0] = first;
+        first += c;
+        tile += k;
+    }
+    if (first == none) return;  // uniform
+    __syncthreads();
     for (int p0 = tid; p0 < planes; p0 += 8 * 1024) {
         uint32_t id[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) id[i] = p0 + i * 1024 < planes ? ids[p0 + i * 1024] : ~0u;
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            if (id[i] == (uint32_t)e) sorted[first + atomicAdd(&s_at, 1)] = p0 + i * 1024;
+            if (id[i] - e0 < (uint32_t)(e1 - e0)) sorted[atomicAdd(&s_at[id[i] - e0], 1)] = p0 + i * 1024;
     }
 }
 
@@ -228,18 +242,20 @@ __device__ __forceinline__ int mg_xq_off(int t, int h) {
     return (t >> 3) * 512 + ((t >> 2) & 1) * 128 + ((t & 3) * 2 + h) * 16;
 }
 
-// The first E workgroups route; the others convert 16 rows each, one a wave.
+// The first ceil(E / per) workgroups route; the others convert 16 rows each, one
+// a wave.
 template <int TYPE>
 __global__ __launch_bounds__(1024) void k_moe_gemm_prep(const float* __restrict__ X, int rows, int K,
                                                         uint8_t* __restrict__ xq, _Float16* __restrict__ sums,
                                                         float* __restrict__ inv, const uint32_t* __restrict__ ids,
-                                                        int planes, int E, int* hdr, int4* tiles, int* sorted,
+                                                        int planes, int per, int E, int* hdr, int4* tiles, int* sorted,
                                                         IdFlags flags, float* y, float* y2, int n, int tile_rows) {
-    if ((int)blockIdx.x < E) {
-        mg_route(ids, planes, blockIdx.x, E, hdr, tiles, sorted, flags, y, y2, n, tile_rows);
+    const int routers = (E + per - 1) / per;
+    if ((int)blockIdx.x < routers) {
+        mg_route(ids, planes, blockIdx.x, per, E, hdr, tiles, sorted, flags, y, y2, n, tile_rows);
         return;
     }
-    const int lane = threadIdx.x & 63, row = (blockIdx.x - E) * 16 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, row = (blockIdx.x - routers) * 16 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int k8 = K >> 3;
     const float* x = X + (int64_t)row * K;
@@ -757,6 +773,7 @@ static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     const int64_t planes = c.batch * c.topk, rows = c.in_dim1 == 1 ? c.batch : planes;
     const MgLayout l = mg_layout(c.E, planes, rows, c.k);
     const int tile_rows = mg_tile_rows(TYPE, c.E, planes, c.k);
+    const int per = (int)((c.E + MG_ROUTERS - 1) / MG_ROUTERS);
     uint8_t* ws = (uint8_t*)c.ws;
     int* hdr = (int*)ws;
     int4* tiles = (int4*)(ws + l.tiles);
@@ -764,8 +781,8 @@ static hipError_t moe_gemm_type(const MoeGemmCall& c, hipStream_t s) {
     float* inv = (float*)(ws + l.inv);
     uint8_t* sums = ws + l.sums;
     uint8_t* xq = ws + l.xq;
-    hipLaunchKernelGGL(k_moe_gemm_prep<TYPE>, dim3((unsigned)(c.E + (rows + 15) / 16)), dim3(1024), 0, s,
-                       c.x, (int)rows, (int)c.k, xq, (_Float16*)sums, inv, c.ids, (int)planes, (int)c.E, hdr, tiles,
+    hipLaunchKernelGGL(k_moe_gemm_prep<TYPE>, dim3((unsigned)((c.E + per - 1) / per + (rows + 15) / 16)), dim3(1024), 0, s,
+                       c.x, (int)rows, (int)c.k, xq, (_Float16*)sums, inv, c.ids, (int)planes, per, (int)c.E, hdr, tiles,
                        sorted, c.flags, c.y, c.mode == MOE_PAIR ? c.y2 : nullptr, (int)c.n, tile_rows);
     if (hipError_t e = hipGetLastError()) return e;
     const bool glu = c.mode == MOE_GLU;

@@ -197,6 +197,31 @@ def test_moe_gemm_many_bad_ids(L, dt):
     assert lib().lloom_hip_ctx_sync(_ctx(0)) == 4
 
 
+@pytest.mark.parametrize("dt,E", [(O.Q4K, 255), (O.Q4K, 257), (O.Q4K, 600), (O.Q6K, 1025), (O.Q4K, 4096)])
+def test_moe_gemm_many_experts(L, dt, E):
+    """More experts than routing workgroups, some of them with no plane."""
+    rng = np.random.default_rng(E)
+    n, k, planes = 40, 256, 14 * E
+    q = L.QTensor.quantize(torch.from_numpy((rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)).cuda(), dt)
+    ids = np.minimum((rng.random((planes // 2, 2)) ** 2 * E).astype(np.int32), E - 1)
+    ids[ids % 7 == 3] = E - 1
+    x = rng.standard_normal((planes // 2, 1, k)).astype(np.float32)
+    got = q.indexed_moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()).cpu().numpy()
+    want, tol = _want(dt, q.data(), E, n, k, x, ids)
+    assert (np.abs(got - want) <= tol).all()
+
+
+def test_moe_gemm_routing_cost(L):
+    """128 K planes over 4096 experts cost about what they do over 256."""
+    us = []
+    for E in (256, 4096):
+        q = L.QTensor.quantize(torch.randn(E, 64, 256, device="cuda"), O.Q4K)
+        x, y = torch.randn(1 << 17, 1, 256, device="cuda"), torch.empty(1 << 17, 1, 64, device="cuda")
+        ids = torch.arange(1 << 17, device="cuda", dtype=torch.int32)[:, None] % E
+        us.append(_us(lambda: q.indexed_moe_forward_into(x, ids, y)))
+    assert us[1] < 2 * us[0], us
+
+
 @pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
 @pytest.mark.parametrize("counts", [[40, 33, 64, 130], [12, 13, 9, 30]], ids=["64", "32"])
 @pytest.mark.parametrize("bits", [0, 20, 26])
