@@ -433,7 +433,7 @@ int lloom_hip_cast(lloom_hip_ctx* ctx, const void* src_dev, int src_dtype, void*
 // The flags of a call that holds the context's lock.  A strict call's host
 // flag is cleared here: the one before it waited for its kernels.
 static IdFlags id_flags(lloom_hip_ctx* ctx, int strict) {
-    if (!strict) return {ctx->flags + 1, ctx->flags};
+    if (!strict) return {nullptr, ctx->flags};
     *(volatile int*)ctx->call_flag = 0;
     return {ctx->call_flag, ctx->flags};
 }

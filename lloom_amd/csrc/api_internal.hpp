@@ -20,7 +20,7 @@ struct lloom_hip_ctx {
     // earlier, keep reading them, so growth needs no device synchronization.
     // Growth at least doubles, so they hold less than the current one.
     std::vector<void*> retired;
-    int* flags = nullptr;  // [0] sticky id error, [1] the last non-strict call's
+    int* flags = nullptr;  // [0] sticky id error
     // What a strict call's kernel reports, in host memory: the call reads it
     // when its stream has drained, with no copy (a pageable 4-byte copy took 10
     // us of a 37 us routed call).

@@ -8,11 +8,15 @@
 namespace lloom {
 
 // Where a kernel reports an out-of-range id: `call` gets 0 or 1 (a strict
-// call's is host memory, read once its stream has drained), `sticky` 1, until
-// the next lloom_hip_ctx_sync.
+// call's host memory, read once its stream has drained; null otherwise),
+// `sticky` 1, until the next lloom_hip_ctx_sync.
 struct IdFlags {
     int *call, *sticky;
 };
+__device__ __forceinline__ void report_ids(IdFlags f, int bad) {
+    if (f.call) f.call[0] = bad;
+    if (bad) f.sticky[0] = 1;
+}
 
 // quant.hip
 hipError_t launch_quantize_act(int vec_dot_type, const float* x, void* out, int64_t elems, hipStream_t s);
@@ -22,7 +26,7 @@ hipError_t launch_dequantize(int type, const void* w, void* y, int out_dtype, in
 // src and dst 16-byte aligned.
 hipError_t launch_cast(int src_t, const void* src, int dst_t, void* dst, int64_t count, hipStream_t s);
 // Rows ids[0 .. n_ids) of an [rows, hidden] weight, dequantized; a bad id
-// gives a zero row and sets both flags (flags.call only ever to 1).
+// gives a zero row and sets the flags (flags.call only ever to 1).
 hipError_t launch_embedding(int type, const void* w, int64_t rows, int64_t hidden, const uint32_t* ids, int64_t n_ids,
                             void* y, int out_dtype, IdFlags flags, hipStream_t s);
 

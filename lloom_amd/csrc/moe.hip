@@ -109,8 +109,7 @@ __global__ __launch_bounds__(1024) void k_moe_route(const uint32_t* __restrict__
         if (e < (uint32_t)E) sorted[atomicAdd(&s_cur[e], 1)] = p;
     }
     if (tid == 0) {
-        flags.call[0] = s_bad;             // this call: read back by a strict call
-        if (s_bad) flags.sticky[0] = 1;  // until the next lloom_hip_ctx_sync
+        report_ids(flags, s_bad);
         ws[1] = s_active;
     }
 }
@@ -431,8 +430,7 @@ __global__ __launch_bounds__(256) void k_moe_lds(const uint8_t* __restrict__ W, 
             }
             bad = __syncthreads_or(bad);
             if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.z == 0) {
-                flags.call[0] = bad;  // this call: read back by a strict call
-                if (bad) flags.sticky[0] = 1;
+                report_ids(flags, bad);
             }
             return;
         }
@@ -694,8 +692,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MOEM_WAVES_
             }
             bad = __syncthreads_or(bad);
             if (tid == 0 && blockIdx.x == 0 && blockIdx.z == 0) {
-                flags.call[0] = bad;  // this call: read back by a strict call
-                if (bad) flags.sticky[0] = 1;
+                report_ids(flags, bad);
             }
             return;
         }
@@ -998,8 +995,7 @@ __global__ __launch_bounds__(64 * NSB) void k_moe_dma(const uint8_t* __restrict_
         }
         bad = __syncthreads_or(bad);
         if (tid == 0 && blockIdx.x == 0 && blockIdx.z == 0) {
-            flags.call[0] = bad;  // this call: read back by a strict call
-            if (bad) flags.sticky[0] = 1;
+            report_ids(flags, bad);
         }
         return;
     }

@@ -190,8 +190,7 @@ __device__ void mg_route(const uint32_t* __restrict__ ids, int planes, int r, in
     }
     __syncthreads();
     if (tid == 0 && r == 0) {
-        flags.call[0] = bad;            // this call: read back by a strict call
-        if (bad) flags.sticky[0] = 1;  // until the next lloom_hip_ctx_sync
+        report_ids(flags, bad);
         hdr[1] = s_tiles;
     }
     first = s_first;

@@ -483,7 +483,7 @@ __device__ __forceinline__ uint32_t load4_a2(const uint8_t* p) {
 // CPU arm's QuantizedType::embedding, :812-838): output block ob belongs to
 // output row ob / rb and reads block ob % rb of weight row ids[row].  With
 // ids null the map is the identity (dequantize).  An id >= rows stores a
-// zero row and raises both flags.
+// zero row and raises the flags.
 struct RowMap {
     const uint32_t* ids;
     int64_t rb, rows;
@@ -498,7 +498,7 @@ __device__ __forceinline__ int64_t src_block(int64_t ob, const RowMap& rm) {
     if ((int64_t)id >= rm.rows) {
         if (ob % rm.rb == 0) {
             *rm.flags.sticky = 1;
-            *rm.flags.call = 1;
+            if (rm.flags.call) *rm.flags.call = 1;
         }
         return -1;
     }
@@ -648,7 +648,7 @@ static hipError_t dequant_t(int type, const void* w, OutT* y, int64_t elems, con
 }
 
 hipError_t launch_dequantize(int type, const void* w, void* y, int out_dtype, int64_t elems, hipStream_t s) {
-    const RowMap rm{nullptr, 1, 0, nullptr};
+    const RowMap rm{nullptr, 1, 0, {nullptr, nullptr}};
     if (out_dtype == T_F16) return dequant_t<uint16_t>(type, w, (uint16_t*)y, elems, rm, s);
     return dequant_t<float>(type, w, (float*)y, elems, rm, s);
 }
