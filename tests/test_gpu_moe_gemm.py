@@ -2,11 +2,13 @@
 an expert on average) against a float64 product of the dequantized
 weights (O.dequantize, the CPU oracle's to_float), through the public calls.
 
-Where it can go wrong: planes of one expert around the 16-row tile and the
-64-row cut (1, 31, 32, 33, 63, 64, 65, 129 and none), weight rows off the
-workgroup's 128 (64 for the SwiGLU), one superblock a row, activations one
-row a token and one a slot, tiles of 32 planes and of 64, an out-of-range id,
-and a capture whose workspace holds only the routing.
+Where it can go wrong: planes of one expert around the 32-plane tile and the
+64-plane cut (1, 31, 32, 33, 63, 64, 65, 129 and none), weight rows off the
+workgroup's 128 (64 for the SwiGLU), one superblock a row and many, activations
+one row a token and one a slot, tiles of 32 planes and of 64, an outlier beside
+small elements, more experts than routing workgroups, out-of-range ids, and a
+capture whose workspace holds only the routing.  Each case asserts whether the
+grouped GEMM is what serves it.
 
 The bound: an element of x loses at most 2^-23 of itself, or 2^-50 of its row's
 largest element, to its two halves; Q6_K drops lo * lo, 2^-22 of the product,
@@ -95,14 +97,26 @@ def _on_small_context(q, x, ids, call="one", q2=None, mib=1):
     return got
 
 
+def _served(dt, E, n, k, x, ids):
+    """Whether the grouped GEMM serves the call: its workspace holds x."""
+    from lloom_amd.quantized import moe_workspace_bytes
+
+    return moe_workspace_bytes(dt, E, n, k, x.shape[0], x.shape[1], ids.shape[1]) > 4 * x.size
+
+
+SHAPES = [(200, 768, 4, False), (8, 256, 3, True), (1100, 512, 1, False), (177, 2048, 2, True), (2065, 256, 2, False),
+          (600, 2048, 3, True), (601, 768, 2, False)]
+
+
 @pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
 @pytest.mark.parametrize("counts", [COUNTS, FEW], ids=["many", "few"])
-@pytest.mark.parametrize("n,k,topk,per_slot", [(200, 768, 4, False), (8, 256, 3, True), (1100, 512, 1, False),
-                                               (177, 2048, 2, True), (2065, 256, 2, False)])
+@pytest.mark.parametrize("n,k,topk,per_slot", SHAPES)
 def test_moe_gemm_matches_f64(L, dt, n, k, topk, per_slot, counts):
     rng = np.random.default_rng(n + k)
     E = len(counts)
     w, x, ids = _case(rng, dt, E, n, k, topk, per_slot, counts)
+    # small Q6_K calls are another kernel's: the same result
+    assert _served(dt, E, n, k, x, ids) == (dt == O.Q4K or ids.size * n >= 65536)
     qg, qu = (L.QTensor.quantize(torch.from_numpy(v).cuda(), dt) for v in w)
     xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
     g, u = (q.indexed_moe_forward(xd, idd).cpu().numpy() for q in (qg, qu))
@@ -116,16 +130,18 @@ def test_moe_gemm_matches_f64(L, dt, n, k, topk, per_slot, counts):
     np.testing.assert_allclose(glu, g / (1 + np.exp(-g.astype(np.float64))) * u, rtol=2e-6, atol=1e-30)
 
 
-def test_moe_gemm_bad_id_and_nonfinite(L):
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+def test_moe_gemm_bad_id_and_nonfinite(L, dt):
     """A bad id zeroes its plane and is refused; a row with an infinity
     spoils its own planes and no other."""
     rng = np.random.default_rng(3)
-    E, n, k = 3, 70, 512
+    E, n, k = 3, 900, 512
     w = (rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)
-    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), O.Q4K)
+    q = L.QTensor.quantize(torch.from_numpy(w).cuda(), dt)
     ids = rng.integers(0, E, (40, 2)).astype(np.int32)
     x = rng.standard_normal((40, 1, k)).astype(np.float32)
-    want, tol = _want(O.Q4K, q.data(), E, n, k, x, ids)
+    assert _served(dt, E, n, k, x, ids)
+    want, tol = _want(dt, q.data(), E, n, k, x, ids)
     bad = ids.copy()
     bad[7, 1] = E
     xd = torch.from_numpy(x).cuda()
@@ -206,6 +222,7 @@ def test_moe_gemm_many_experts(L, dt, E):
     ids = np.minimum((rng.random((planes // 2, 2)) ** 2 * E).astype(np.int32), E - 1)
     ids[ids % 7 == 3] = E - 1
     x = rng.standard_normal((planes // 2, 1, k)).astype(np.float32)
+    assert _served(dt, E, n, k, x, ids)
     got = q.indexed_moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()).cpu().numpy()
     want, tol = _want(dt, q.data(), E, n, k, x, ids)
     assert (np.abs(got - want) <= tol).all()
@@ -235,6 +252,7 @@ def test_moe_gemm_small_beside_outlier(L, dt, counts, bits):
     q = L.QTensor.quantize(torch.from_numpy(w).cuda(), dt)
     ids = np.repeat(np.arange(E), counts).astype(np.int32)[:, None]
     x = rng.standard_normal((len(ids), 1, k)).astype(np.float32)
+    assert _served(dt, E, n, k, x, ids)
     x[..., 37] *= 2.0 ** bits
     x[::2, ..., 513] *= -(2.0 ** bits)
     want, tol = _want(dt, q.data(), E, n, k, x, ids)
@@ -253,6 +271,7 @@ def test_moe_gemm_no_further_off_than_the_other_kernels(L, dt, E, n, k, per):
     ids = rng.integers(0, E, (E * per, 1)).astype(np.int32)
     x = (rng.standard_normal((E * per, 1, k)) * rng.standard_normal((E * per, 1, k))).astype(np.float32)
     xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    assert _served(dt, E, n, k, x, ids)
     want, _ = _want(dt, q.data(), E, n, k, x, ids)
     off = [np.linalg.norm(y - want) / np.linalg.norm(want)
            for y in (q.indexed_moe_forward(xd, idd).cpu().numpy(), _on_small_context(q, xd, idd))]

@@ -538,9 +538,9 @@ def test_moe_run_to_run_identical(L):
 
 
 def test_moe_many_planes_and_magnitudes(L):
-    """Q4_K experts with dense routing (about 24 planes an expert: more than
-    one pass of staged planes) and planes of very different magnitude (the
-    fp16 operand path scales each plane by its own power of two): 1e4-scaled,
+    """Q4_K experts with dense routing (about 24 planes an expert) and planes
+    of very different magnitude (the fp16 operand path scales each row of x by
+    its own power of two): 1e4-scaled,
     1e-6-scaled, all-zero, and one element past the fp16 range."""
     rng = np.random.default_rng(21)
     E, n, k, batch, topk = 4, 80, 1024, 24, 4
@@ -566,9 +566,9 @@ def test_moe_many_planes_and_magnitudes(L):
 
 @pytest.mark.parametrize("dt", [O.Q4K, O.Q8_0])
 def test_moe_more_planes_than_one_list(L, dt):
-    """1200 planes: past the in-kernel routing list, so the routing kernel
-    sorts the planes first; a bad id among them is refused and its planes
-    zeroed."""
+    """1200 planes, past the in-kernel routing list: Q8_0 sorts them in the
+    routing kernel first, Q4_K takes the grouped GEMM, which routes in its prep;
+    a bad id among them is refused and its planes zeroed."""
     rng = np.random.default_rng(31)
     E, n, k, batch, topk = 8, 24, 256, 300, 4
     got, want, _ = _moe_case(L, dt, E, n, k, batch, topk, 1, seed=31)
@@ -736,8 +736,7 @@ def test_moe_pair_bad_id_zeroes_both(L):
                                                      (256, 512, True, 300)])
 def test_moe_dense_routing(L, n, k, in_dim1_is_topk, batch):
     """Q4_K experts with prefill-dense routing (at least 8 planes an active
-    expert: the fp16-MFMA kernel, 16 planes a pass; 1200 planes route
-    through the sorting launch): the down projection's shape (k = 768, a
+    expert: the grouped GEMM): the down projection's shape (k = 768, a
     plane per slot), ragged n, against the oracle and a float64 dense
     reference."""
     topk = 4
