@@ -539,9 +539,10 @@ __device__ __forceinline__ int mg_key(int r) { return (r >> 1) & 7; }
 // LDS holds two stages of half a superblock (eight MFMA steps): the rows' x'
 // in octets of 8 rows, an octet's 128-byte line (hi or lo, four steps) as one
 // 1 KB DMA: row r's 16-byte piece u at place u ^ mg_key(r) of its line.
-// While a stage is computed, the next one's DMAs and the next superblock's
-// weight loads are in flight; a stage starts with one counted wait and one
-// barrier.  Rows past np hold whatever LDS held: their sums are not stored.
+// While a stage is computed, the next one's DMAs and (Q4_K) the next
+// superblock's weight loads are in flight; a stage starts with one counted wait
+// and one barrier.  Q6_K's weights are 2-byte aligned and realigned where they
+// are loaded, which waits for them (and for the DMAs) there.  Rows past np hold whatever LDS held: their sums are not stored.
 template <int TYPE, int ROWS, int MT, bool GLU, bool MID>
 __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y,
                                         uint8_t* smem, const int* s_plane, const int* s_row, const float* s_inv) {
@@ -719,14 +720,17 @@ __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const
 
 // What bounds it: [128, 768, 2048] Q4_K, 2000 tokens top-8, the SwiGLU launch
 // (two weights, 201 GFLOP of hi and lo products) takes 267 us with its prep
-// (0.75 PFLOP/s; 261 with hi and lo in one sum; 301 on 16x16x32 MFMAs, whose twice as many issue slots left
-// less room for the unpacking).  On that earlier form, only the loads (no MFMA,
-// no unpacking) took 273, only the arithmetic 246: a superblock's two L2 round
-// trips and its arithmetic hide each other only in part at two workgroups a CU.
-// At 64 tokens it is the weight stream (113 MB a weight, 2.5 TB/s).  Eight
-// waves sharing one x' tile (half the L2 stream) took 313: one workgroup a CU
-// leaves nothing to run at its barriers and its ends.  With the rows of x'
-// interleaved by half superblock instead of whole it measured the same.
+// (0.75 PFLOP/s; 262 with hi and lo in one sum).  The matrix cores are busy 44 %
+// of the cycles, the VALU 39, both 14, neither 31: two waves a SIMD, whose
+// barriers (two a superblock) and L2 round trips the other one covers in part.
+// Q6_K, one weight of [128, 2048, 768]: 226 us with its prep, 35, 34, 15 and 46:
+// its loads are waited for in place.  At 64 tokens the Q4_K call is the weight
+// stream (113 MB in 46 us, 2.5 TB/s).  Tried on earlier forms of this kernel:
+// 16x16x32 MFMAs (SwiGLU launch 301 against 273 then: twice the issue slots
+// left less room for the unpacking); eight waves sharing one x' tile, half the
+// L2 stream (313 against 290: one workgroup a CU leaves nothing to run at its
+// barriers and its ends); the rows of x' interleaved by half superblock instead
+// of whole (the same).
 // A workgroup takes item (tile of planes, weight block): items are dealt to
 // the XCDs in contiguous runs (workgroup b runs on XCD b % 8), so the blocks
 // of one tile, which read the same activations, and the tiles of one expert,
