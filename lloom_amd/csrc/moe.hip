@@ -592,8 +592,8 @@ __global__ __launch_bounds__(256) void k_moe_lds(const uint8_t* __restrict__ W, 
 // ------------------------------------------- Q4_K experts on fp16 MFMA --
 // Q4_K from 8 planes an expert where the grouped GEMM cannot serve the call: no
 // workspace for its copy of x (a capture that reserved less, or no memory), or
-// rows * K past its offsets.  [128, 768, 2048] top-8: 512 tokens 228 us against
-// the GEMM's 65, and 549 for k_moe_lds.
+// rows * K past its offsets.  [128, 768, 2048] top-8: 512 tokens 229 us against
+// the GEMM's 66, and 378 for k_moe_lds.
 // The same contract (f32 activations, exactly dequantized weights, f32
 // accumulation) on v_mfma_f32_16x16x32_f16.  A workgroup (4 waves) owns
 // 64 NT weight rows of one expert; each wave NT 16-row tiles over all of K.

@@ -109,7 +109,7 @@ size_t moe_gemm_workspace_bytes(int64_t E, int64_t planes, int64_t rows, int64_t
 //     [8, 768, 2048] 8 planes an expert 34 (34) / 31 (41), 12 34 (34) / 41 (55)
 // Over E 8 .. 256, n 512 .. 2048, k 256 .. 4096 the rule is at most 1.11 (Q4_K)
 // and 1.19 (Q6_K, [8, 768, 4096] with 12 planes an expert) of the better one.
-// With 8 planes an expert Q4_K comes here at any size (11 / 14 us at [8, 256,
+// With 8 planes an expert Q4_K comes here at any size (11 / 13 us at [8, 256,
 // 256], 21 / 53 at [8, 768, 2048] against k_moe_mfma).
 bool moe_gemm_fits(int type, int64_t E, int64_t planes, int64_t rows, int64_t n, int64_t k) {
     if ((type != T_Q4K && type != T_Q6K) || k % 256) return false;
@@ -542,7 +542,8 @@ __device__ __forceinline__ int mg_key(int r) { return (r >> 1) & 7; }
 // While a stage is computed, the next one's DMAs and (Q4_K) the next
 // superblock's weight loads are in flight; a stage starts with one counted wait
 // and one barrier.  Q6_K's weights are 2-byte aligned and realigned where they
-// are loaded, which waits for them (and for the DMAs) there.  Rows past np hold whatever LDS held: their sums are not stored.
+// are loaded, which waits for them (and for the DMAs) there.  Rows past np hold
+// whatever LDS held: their sums are not stored.
 template <int TYPE, int ROWS, int MT, bool GLU, bool MID>
 __device__ __forceinline__ void mg_tile(const MgArgs& A, int np, int col0, const uint8_t* W0, const uint8_t* W1, float* Y,
                                         uint8_t* smem, const int* s_plane, const int* s_row, const float* s_inv) {
