@@ -260,6 +260,23 @@ def test_moe_gemm_small_beside_outlier(L, dt, counts, bits):
     assert (np.abs(got - want) <= tol).all(), (np.abs(got - want) / tol).max()
 
 
+@pytest.mark.parametrize("dt", [O.Q4K, O.Q6K])
+def test_moe_gemm_tiny_rows(L, dt):
+    """Rows whose power-of-two scale would leave the normal numbers, down to
+    subnormal x, on the grouped GEMM and without room for a copy of x (half of
+    the last place of a subnormal result comes on top of the bound)."""
+    rng = np.random.default_rng(9)
+    E, n, k = 4, 320, 2048
+    q = L.QTensor.quantize(torch.from_numpy((rng.standard_normal((E, n, k)) * 0.05).astype(np.float32)).cuda(), dt)
+    ids = rng.integers(0, E, (240, 1)).astype(np.int32)
+    x = np.ldexp(rng.standard_normal((240, 1, k)).astype(np.float32), np.repeat([-100, -114, -119, -133], 60)[:, None, None])
+    assert _served(dt, E, n, k, x, ids)
+    want, tol = _want(dt, q.data(), E, n, k, x, ids)
+    xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    for got in (q.indexed_moe_forward(xd, idd).cpu().numpy(), _on_small_context(q, xd, idd)):
+        assert (np.abs(got - want) <= tol + 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("dt,E,n,k,per", [(O.Q4K, 64, 416, 2048, 5), (O.Q4K, 64, 512, 768, 7), (O.Q4K, 16, 320, 2048, 40),
                                           (O.Q6K, 64, 640, 2048, 5), (O.Q6K, 64, 512, 768, 14), (O.Q6K, 16, 320, 2048, 40)])
 def test_moe_gemm_no_further_off_than_the_other_kernels(L, dt, E, n, k, per):
